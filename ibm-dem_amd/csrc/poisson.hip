@@ -43,7 +43,6 @@ using namespace bk;
 constexpr int RB = 256;           // threads per block for level kernels
 constexpr int RED_BLOCKS = 1024;
 constexpr int RED_T = 256;
-constexpr int COARSE_T = 1024;
 
 struct LaunchShape {
     dim3 grid, block;
@@ -913,12 +912,340 @@ ProlongShape prolong_shape(const LevelDev &d) {
     return {sh.grid, sh.block, x2, by % 2 == 0 && need <= (unsigned)(x2 ? PRO2_TILE : PRO_TILE)};
 }
 
-// coarsest level, one work-group. Small levels (<= COARSE_LDS cells, every
-// level the grids here coarsen to) live in LDS with a precomputed neighbour
-// table whose missing (wall) neighbours point at a zero slot, so the sweeps
-// evaluate exactly nbsum's expression without index arithmetic; larger
-// coarsest levels run the same sweeps in global memory.
+// ---------------------------------------------------------------------------
+// The coarsest level of a hierarchy: `sweeps` symmetric pairs of red-black
+// Gauss-Seidel sweeps from x = 0, colours 0, 1, 0, 1, ... and then 1, 0, 1,
+// 0, ... . Where the order turns, colour 1 would be swept twice in a row; a
+// cell's update reads only the other colour, so the second pass writes the
+// same values and is left out: 4 sweeps - 1 half sweeps of strictly
+// alternating colour, the same result bit for bit. A level whose colouring is
+// inconsistent (an odd periodic extent) runs 2 sweeps damped Jacobi sweeps.
+//
+// How far halving gets depends on the extents: multiples of 32 end at a few
+// hundred cells, other even extents at thousands or 10^5. Three forms, by
+// the level's size (each cell's arithmetic is the same in all of them):
+//   coarse_wg    up to CWG_PAIRS x-pairs: one work-group with x in LDS and
+//                each thread's pairs in registers. Bound by the chain of
+//                half sweeps (LDS round, six dependent FP64 operations,
+//                barrier): 24 us a solve at 455 cells, 73 us at 7,920, 137 us
+//                at 15,700.
+//   coarse_jac   Jacobi levels of up to CJ_CELLS cells, likewise.
+//   coarse_tile  larger levels of either kind: the level in tiles over the
+//                whole chip, CT_H half sweeps a launch on a tile with a
+//                CT_H-cell halo in LDS. One work-group over the whole level
+//                in global memory took 9.6 ms a solve at 50x38x65 (123,500
+//                cells).
+// ---------------------------------------------------------------------------
 constexpr int COARSE_LDS = 512;
+
+__device__ __forceinline__ int coarse_half_sweeps(int sweeps) { return 4 * sweeps - 1; }
+
+// One work-group of NT threads, CP x-pairs per thread (pair q = t + NT m).
+// x is kept in LDS in two colour halves of one slot per pair; slot hs of each
+// half is 0 and stands for missing neighbours.
+constexpr int CWG_PAIRS = 8192;
+template <typename T, int NT, int CP>
+__device__ __forceinline__ void coarse_wg_body(const Blk &kb, const LevelDev &L, T *__restrict__ xg,
+                                               const T *__restrict__ bg, int sweeps,
+                                               const double *__restrict__ stop) {
+    static_assert(NT * CP <= CWG_PAIRS, "pairs fit the LDS halves");
+    if (*stop != 0.0) return;
+    __shared__ T xs[2 * (NT * CP + 1)];
+    const int t = threadIdx.x;
+    const int rl = (L.nx + 1) >> 1, hs = rl * L.ny * L.nz;   // pairs (an odd row's last pair has one cell)
+    const int H = hs + 1;
+    const bool px = L.bt[0] == IBMDEM_BC_PERIODIC, py = L.bt[2] == IBMDEM_BC_PERIODIC,
+               pz = L.bt[4] == IBMDEM_BC_PERIODIC;
+    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
+    // per pair: its parity (the colour of its even cell; -1: no pair), the
+    // slots of its neighbours within the other colour's half (two per
+    // register) and, by cell, right-hand side and 1/diagonal
+    int ca[CP], nx2[CP], ny2[CP], nz2[CP];
+    T bv[CP][2], id[CP][2];
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        const int q = t + NT * m;
+        ca[m] = -1;
+        nx2[m] = ny2[m] = nz2[m] = 0;
+        bv[m][0] = bv[m][1] = id[m][0] = id[m][1] = T(0);
+        if (q >= hs) continue;
+        const int row = q / rl, p = q - row * rl, k = row / L.ny, j = row - k * L.ny;
+        const int i = 2 * p, last = L.nx - 1;
+        ca[m] = (j + k) & 1;
+        // the even cell's west neighbour is an odd cell, the odd cell's east
+        // neighbour an even one (periodic x: nx is even)
+        const int w = p > 0 ? q - 1 : (px ? q + rl - 1 : hs);
+        const int e = i + 2 <= last ? q + 1 : (px ? q + 1 - rl : hs);
+        const int s = j > 0 ? q - rl : (py ? q + (L.ny - 1) * rl : hs);
+        const int n = j < L.ny - 1 ? q + rl : (py ? q - (L.ny - 1) * rl : hs);
+        const int pl = rl * L.ny;
+        const int b = k > 0 ? q - pl : (pz ? q + (L.nz - 1) * pl : hs);
+        const int u = k < L.nz - 1 ? q + pl : (pz ? q - (L.nz - 1) * pl : hs);
+        nx2[m] = w | e << 16;
+        ny2[m] = s | n << 16;
+        nz2[m] = b | u << 16;
+        bv[m][0] = bg[lidx(L, i, j, k)];
+        id[m][0] = T(L.idiag[diag_index(L, i, j, k)]);
+        if (i < last) {   // else the odd cell does not exist: it stays 0
+            bv[m][1] = bg[lidx(L, i + 1, j, k)];
+            id[m][1] = T(L.idiag[diag_index(L, i + 1, j, k)]);
+        }
+    }
+    for (int q = t; q < 2 * H; q += NT) xs[q] = T(0);
+    __syncthreads();
+    const int ns = coarse_half_sweeps(sweeps);
+    for (int s = 0; s < ns; ++s) {
+        const int color = s & 1;
+        T *own = xs + color * H;
+        const T *oth = xs + (1 - color) * H;
+#pragma unroll
+        for (int m = 0; m < CP; ++m) {
+            if (ca[m] < 0) continue;
+            const int q = t + NT * m;
+            const bool even = ca[m] == color;
+            const T part = oth[q], xo = oth[even ? nx2[m] & 0xffff : nx2[m] >> 16];
+            const T sx = ((even ? xo : part) + (even ? part : xo)) * ihx2;
+            const T sy = (oth[ny2[m] & 0xffff] + oth[ny2[m] >> 16]) * ihy2;
+            const T sz = (oth[nz2[m] & 0xffff] + oth[nz2[m] >> 16]) * ihz2;
+            own[q] = ((even ? bv[m][0] : bv[m][1]) + (sx + sy + sz)) * (even ? id[m][0] : id[m][1]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        if (ca[m] < 0) continue;
+        const int q = t + NT * m, row = q / rl, p = q - row * rl, k = row / L.ny, j = row - k * L.ny;
+        xg[lidx(L, 2 * p, j, k)] = xs[ca[m] * H + q];
+        if (2 * p + 1 < L.nx) xg[lidx(L, 2 * p + 1, j, k)] = xs[(1 - ca[m]) * H + q];
+    }
+}
+template <typename T, int NT, int CP>
+__global__ __launch_bounds__(NT) void k_coarse_wg(LevelDev L, T *__restrict__ xg, const T *__restrict__ bg, int sweeps,
+                                                  const double *__restrict__ stop) {
+    coarse_wg_body<T, NT, CP>(hw_blk(), L, xg, bg, sweeps, stop);
+}
+
+// Jacobi levels in one work-group: CP cells per thread (cell q = t + NT m, x
+// fastest), the iterate in two LDS arrays read and written in turn, so a
+// sweep is one LDS round and one barrier; slot n of both is 0 and stands for
+// missing neighbours. One wavefront with the cells in table-driven rounds and
+// two barriers a sweep took 55 us at 8x6x7 and 65 us at 15x2x15; this takes
+// 10 us at both.
+constexpr int CJ_CELLS = 8192;
+template <typename T, int NT, int CP>
+__device__ __forceinline__ void coarse_jac_body(const Blk &kb, const LevelDev &L, T *__restrict__ xg,
+                                                const T *__restrict__ bg, int sweeps,
+                                                const double *__restrict__ stop) {
+    static_assert(NT * CP <= CJ_CELLS, "16-bit neighbour slots");
+    if (*stop != 0.0) return;
+    __shared__ T xs[2][NT * CP + 1];
+    const int t = threadIdx.x, n = L.nx * L.ny * L.nz, pl = L.nx * L.ny;
+    const bool px = L.bt[0] == IBMDEM_BC_PERIODIC, py = L.bt[2] == IBMDEM_BC_PERIODIC,
+               pz = L.bt[4] == IBMDEM_BC_PERIODIC;
+    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2), om = T(0.8);
+    int nbx[CP], nby[CP], nbz[CP];   // two neighbour slots each
+    T bv[CP], id[CP], xv[CP];
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        const int q = t + NT * m;
+        nbx[m] = nby[m] = nbz[m] = 0;
+        bv[m] = id[m] = xv[m] = T(0);
+        if (q >= n) continue;
+        const int row = q / L.nx, i = q - row * L.nx, k = row / L.ny, j = row - k * L.ny;
+        const int w = i > 0 ? q - 1 : (px ? q + L.nx - 1 : n), e = i < L.nx - 1 ? q + 1 : (px ? q - L.nx + 1 : n);
+        const int s = j > 0 ? q - L.nx : (py ? q + pl - L.nx : n),
+                  r = j < L.ny - 1 ? q + L.nx : (py ? q - pl + L.nx : n);
+        const int b = k > 0 ? q - pl : (pz ? q + n - pl : n), u = k < L.nz - 1 ? q + pl : (pz ? q - n + pl : n);
+        nbx[m] = w | e << 16;
+        nby[m] = s | r << 16;
+        nbz[m] = b | u << 16;
+        bv[m] = bg[lidx(L, i, j, k)];
+        id[m] = T(L.idiag[diag_index(L, i, j, k)]);
+        xs[0][q] = T(0);
+    }
+    if (t == 0) xs[0][n] = xs[1][n] = T(0);
+    __syncthreads();
+    for (int s = 0; s < 2 * sweeps; ++s) {
+        const T *x = xs[s & 1];
+        T *y = xs[1 - (s & 1)];
+#pragma unroll
+        for (int m = 0; m < CP; ++m) {
+            const int q = t + NT * m;
+            if (q >= n) continue;
+            const T sx = (x[nbx[m] & 0xffff] + x[nbx[m] >> 16]) * ihx2;
+            const T sy = (x[nby[m] & 0xffff] + x[nby[m] >> 16]) * ihy2;
+            const T sz = (x[nbz[m] & 0xffff] + x[nbz[m] >> 16]) * ihz2;
+            const T xn = (bv[m] + (sx + sy + sz)) * id[m];
+            xv[m] = xv[m] + om * (xn - xv[m]);
+            y[q] = xv[m];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int m = 0; m < CP; ++m) {
+        const int q = t + NT * m;
+        if (q >= n) continue;
+        const int row = q / L.nx, i = q - row * L.nx, k = row / L.ny, j = row - k * L.ny;
+        xg[lidx(L, i, j, k)] = xv[m];
+    }
+}
+template <typename T, int NT, int CP>
+__global__ __launch_bounds__(NT) void k_coarse_jac(LevelDev L, T *__restrict__ xg, const T *__restrict__ bg, int sweeps,
+                                                   const double *__restrict__ stop) {
+    coarse_jac_body<T, NT, CP>(hw_blk(), L, xg, bg, sweeps, stop);
+}
+
+// Tiles of CT_X x CT_Y x CT_Z cells, CT_H half sweeps (Jacobi: sweeps) s0 ..
+// s0 + ns - 1 from xin to xout (s0 = 0: from x = 0). The tile is loaded with a
+// halo of CT_H cells (wrapped across periodic sides, inactive zeros beyond
+// the others) and swept as a whole; the outermost layer is never updated, so
+// after s half sweeps the cells s layers in are exact, and the tile itself
+// is exact after CT_H. Halo cells are the neighbouring tiles' cells with
+// their own arithmetic, so the result does not depend on the tiling. At
+// 50x38x65 in FP64 a launch of four half sweeps takes 9.5 us on 180 blocks
+// (start, loads and stores ~7 us, ~0.6 us a half sweep), the solve 0.23 ms.
+constexpr int CT_X = 16, CT_Y = 8, CT_Z = 8, CT_H = 4, CT_T = 1024;
+constexpr int CT_RL = (CT_X + 2 * CT_H) / 2, CT_EY = CT_Y + 2 * CT_H, CT_EZ = CT_Z + 2 * CT_H;
+constexpr int CT_NP = CT_RL * CT_EY * CT_EZ, CT_PL = CT_RL * CT_EY;   // x-pairs of a tile, of a plane
+constexpr int CT_M = CT_NP / CT_T;
+static_assert(CT_NP % CT_T == 0 && CT_X % 2 == 0 && CT_H % 2 == 0, "whole x-pairs and threads");
+// the level's index of an unwrapped one, -1 beyond a side that is not periodic
+__device__ __forceinline__ int ct_map(int v, int n, int lo) {
+    if (v >= 0 && v < n) return v;
+    if (lo != IBMDEM_BC_PERIODIC) return -1;
+    v %= n;
+    return v < 0 ? v + n : v;
+}
+template <typename T, bool JAC>
+__device__ __forceinline__ void coarse_tile_body(const Blk &kb, const LevelDev &L, const T *__restrict__ xin,
+                                                 T *__restrict__ xout, const T *__restrict__ bg, int s0, int ns,
+                                                 const double *__restrict__ stop) {
+    const double stopped = *stop;
+    __shared__ T xs[2 * CT_NP];
+    const int t = threadIdx.x;
+    const int ox = kb.bx * CT_X - CT_H, oy = kb.by * CT_Y - CT_H, oz = kb.bz * CT_Z - CT_H;
+    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
+    int ca[CT_M];
+    bool upd[CT_M][2];
+    T bv[CT_M][2], id[CT_M][2], xv[CT_M][2];
+    const T id_int = T(L.idiag[DIAG_INTERIOR]);
+#pragma unroll
+    for (int m = 0; m < CT_M; ++m) {
+        const int q = t + CT_T * m, z = q / CT_PL, y = (q - z * CT_PL) / CT_RL, p = q - z * CT_PL - y * CT_RL;
+        const int j = ct_map(oy + y, L.ny, L.bt[2]), k = ct_map(oz + z, L.nz, L.bt[4]);
+        ca[m] = (oy + y + oz + z) & 1;   // ox is even
+        const bool inner = y > 0 && y < CT_EY - 1 && z > 0 && z < CT_EZ - 1;
+        upd[m][0] = inner && p > 0;
+        upd[m][1] = inner && p < CT_RL - 1;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int i = ct_map(ox + 2 * p + e, L.nx, L.bt[0]);
+            const bool act = i >= 0 && j >= 0 && k >= 0;
+            const int g = act ? lidx(L, i, j, k) : 0;   // inactive cells load cell 0 and drop it
+            const int di = act ? diag_index(L, i, j, k) : DIAG_INTERIOR;
+            const T bl = bg[g], xl = s0 > 0 ? xin[g] : T(0);
+            T il = id_int;
+            if (di != DIAG_INTERIOR) il = T(L.idiag[di]);
+            bv[m][e] = act ? bl : T(0);
+            id[m][e] = act ? il : T(0);
+            xv[m][e] = act ? xl : T(0);
+            upd[m][e] = upd[m][e] && act;
+        }
+    }
+    // every load is in flight before the first is used
+    if (stopped != 0.0) return;
+#pragma unroll
+    for (int m = 0; m < CT_M; ++m)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) xs[((ca[m] + e) & 1) * CT_NP + t + CT_T * m] = xv[m][e];
+    __syncthreads();
+    // nbsum of cell e of pair q from the other colour's half
+    auto nb = [&](const T *oth, int q, int e) {
+        const T xw = oth[e ? q : q - 1], xe = oth[e ? q + 1 : q];
+        const T sx = (xw + xe) * ihx2;
+        const T syy = (oth[q - CT_RL] + oth[q + CT_RL]) * ihy2;
+        const T szz = (oth[q - CT_PL] + oth[q + CT_PL]) * ihz2;
+        return sx + syy + szz;
+    };
+    for (int s = s0; s < s0 + ns; ++s) {
+        if (JAC) {
+            const T om = T(0.8);
+            T nv[CT_M][2];
+#pragma unroll
+            for (int m = 0; m < CT_M; ++m)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int q = t + CT_T * m, c = (ca[m] + e) & 1;
+                    const T x0 = xs[c * CT_NP + q];
+                    nv[m][e] = x0;
+                    if (upd[m][e]) {
+                        const T xn = (bv[m][e] + nb(xs + (1 - c) * CT_NP, q, e)) * id[m][e];
+                        nv[m][e] = x0 + om * (xn - x0);
+                    }
+                }
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < CT_M; ++m)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) xs[((ca[m] + e) & 1) * CT_NP + t + CT_T * m] = nv[m][e];
+        } else {
+            const int color = s & 1;
+#pragma unroll
+            for (int m = 0; m < CT_M; ++m) {
+                const int q = t + CT_T * m, e = ca[m] == color ? 0 : 1;
+                if (e ? upd[m][1] : upd[m][0])
+                    xs[color * CT_NP + q] = ((e ? bv[m][1] : bv[m][0]) + nb(xs + (1 - color) * CT_NP, q, e)) *
+                                            (e ? id[m][1] : id[m][0]);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int m = 0; m < CT_M; ++m) {
+        const int q = t + CT_T * m, z = q / CT_PL, y = (q - z * CT_PL) / CT_RL, p = q - z * CT_PL - y * CT_RL;
+        if (p < CT_H / 2 || p >= (CT_X + CT_H) / 2 || y < CT_H || y >= CT_Y + CT_H || z < CT_H || z >= CT_Z + CT_H)
+            continue;
+        const int j = oy + y, k = oz + z;
+        if (j >= L.ny || k >= L.nz) continue;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int i = ox + 2 * p + e;
+            if (i < L.nx) xout[lidx(L, i, j, k)] = xs[((ca[m] + e) & 1) * CT_NP + q];
+        }
+    }
+}
+template <typename T, bool JAC>
+__global__ __launch_bounds__(CT_T) void k_coarse_tile(LevelDev L, const T *__restrict__ xin, T *__restrict__ xout,
+                                                      const T *__restrict__ bg, int s0, int ns,
+                                                      const double *__restrict__ stop) {
+    coarse_tile_body<T, JAC>(hw_blk(), L, xin, xout, bg, s0, ns, stop);
+}
+
+// Which form a coarsest level takes: one work-group where the level fits its
+// LDS and registers, with as few wavefronts as hold the level in one or two
+// rounds (a barrier of four is faster than one of sixteen), tiles above. At
+// the line, CWG_PAIRS pairs in FP64, one work-group takes 137 us and the
+// tiles' 24 launches 190 us.
+enum CoarseForm { CF_WG256, CF_WG1, CF_WG2, CF_WG4, CF_WG8, CF_JAC512, CF_JAC2, CF_JAC8, CF_TILE, CF_TILE_JAC };
+CoarseForm coarse_form(const LevelDev &d) {
+    const long n = (long)d.nx * d.ny * d.nz, pairs = (long)((d.nx + 1) / 2) * d.ny * d.nz;
+    if (!d.rb_valid) return n <= 512 ? CF_JAC512 : n <= 2048 ? CF_JAC2 : n <= CJ_CELLS ? CF_JAC8 : CF_TILE_JAC;
+    if (pairs <= 512) return CF_WG256;
+    return pairs <= 1024 ? CF_WG1 : pairs <= 2048 ? CF_WG2 : pairs <= 4096 ? CF_WG4 : pairs <= CWG_PAIRS ? CF_WG8 : CF_TILE;
+}
+int coarse_threads(CoarseForm f) { return f == CF_WG256 ? 256 : f == CF_JAC512 ? 512 : 1024; }
+// the tile form's launches: launch q of n does half sweeps s0 .. s0 + ns - 1
+// and reads what launch q - 1 wrote; the last one writes x (not tmp)
+struct CoarseTileStep {
+    int s0, ns;
+    bool to_x;
+};
+int coarse_tile_launches(bool jac, int sweeps) { return div_up(jac ? 2 * sweeps : 4 * sweeps - 1, CT_H); }
+CoarseTileStep coarse_tile_step(bool jac, int sweeps, int q) {
+    const int total = jac ? 2 * sweeps : 4 * sweeps - 1, n = coarse_tile_launches(jac, sweeps);
+    return {q * CT_H, std::min(CT_H, total - q * CT_H), (n - 1 - q) % 2 == 0};
+}
+dim3 coarse_tile_grid(const LevelDev &d) { return dim3(div_up(d.nx, CT_X), div_up(d.ny, CT_Y), div_up(d.nz, CT_Z)); }
 
 // The symmetric red-black sweeps of a coarsest level of n <= 64 CQ cells on
 // one wavefront (lane l owns the cells q = l + 64 t): the lane's neighbour
@@ -959,8 +1286,8 @@ __device__ __forceinline__ void coarse_reg_sweeps(T *x, const T *b, const short 
             }
         wave_barrier_lds();
     };
-    for (int s = 0; s < sweeps; ++s) { half(0); half(1); }
-    for (int s = 0; s < sweeps; ++s) { half(1); half(0); }
+    for (int s = 1; s < 2 * sweeps; ++s) { half(0); half(1); }
+    half(0);
 }
 // the register-held sweeps for levels of up to 256 cells; false: larger
 template <typename T>
@@ -974,107 +1301,36 @@ __device__ __forceinline__ bool coarse_sweeps_small(T *x, const T *b, const shor
     return true;
 }
 
+// the coarsest level's solve on the context's stream
 template <typename T>
-__device__ __forceinline__ void coarse_lds_body(const Blk &kb, const LevelDev &L, T *__restrict__ xg, const T *__restrict__ bg,
-                                                   int sweeps, const double *__restrict__ stop) {
-    if (*stop != 0.0) return;
-    __shared__ T x[COARSE_LDS + 1], b[COARSE_LDS], id[COARSE_LDS], t[COARSE_LDS];
-    __shared__ short nb[6][COARSE_LDS];
-    __shared__ unsigned char col[COARSE_LDS];
-    const int n = L.nx * L.ny * L.nz;
-    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
-    for (int q = kb.tx; q < n; q += 64) {
-        const int i = q % L.nx, j = (q / L.nx) % L.ny, k = q / (L.nx * L.ny);
-        const int a[3] = {i, j, k}, m[3] = {L.nx, L.ny, L.nz};
-        for (int d = 0; d < 3; ++d)
-            for (int dir = 0; dir < 2; ++dir) {
-                int p[3] = {a[0], a[1], a[2]};
-                int v = p[d] + (dir ? 1 : -1);
-                int idx;
-                if (v < 0) idx = L.bt[2 * d] != IBMDEM_BC_PERIODIC ? -1 : v + m[d];
-                else if (v >= m[d]) idx = L.bt[2 * d + 1] != IBMDEM_BC_PERIODIC ? -1 : v - m[d];
-                else idx = v;
-                p[d] = idx;
-                nb[2 * d + dir][q] = (short)(idx < 0 ? n : (p[2] * L.ny + p[1]) * L.nx + p[0]);
-            }
-        id[q] = T(L.idiag[diag_index(L, i, j, k)]);
-        col[q] = (unsigned char)((i + j + k) & 1);
-        b[q] = bg[lidx(L, i, j, k)];
-        x[q] = T(0);
-    }
-    if (kb.tx == 0) x[n] = T(0);
-    __syncthreads();
-    auto upd = [&](int q) -> T {
-        const T sx = (x[nb[0][q]] + x[nb[1][q]]) * ihx2;
-        const T sy = (x[nb[2][q]] + x[nb[3][q]]) * ihy2;
-        const T sz = (x[nb[4][q]] + x[nb[5][q]]) * ihz2;
-        return (b[q] + (sx + sy + sz)) * id[q];
-    };
-    auto half = [&](int color) {
-        for (int q = kb.tx; q < n; q += 64)
-            if (col[q] == color) x[q] = upd(q);
-        __syncthreads();
-    };
-    if (L.rb_valid) {
-        if (!coarse_sweeps_small<T>(x, b, nb, id, col, n, sweeps, ihx2, ihy2, ihz2)) {
-            for (int s = 0; s < sweeps; ++s) { half(0); half(1); }
-            for (int s = 0; s < sweeps; ++s) { half(1); half(0); }
-        }
-    } else {
-        const T om = T(0.8);
-        for (int s = 0; s < 2 * sweeps; ++s) {
-            for (int q = kb.tx; q < n; q += 64) t[q] = x[q] + om * (upd(q) - x[q]);
-            __syncthreads();
-            for (int q = kb.tx; q < n; q += 64) x[q] = t[q];
-            __syncthreads();
+void launch_coarsest(hipStream_t s, const LevelDev &d, T *x, const T *b, T *tmp, int sweeps, const double *stop) {
+    const CoarseForm f = coarse_form(d);
+    const dim3 one(1);
+    switch (f) {
+    case CF_WG8: hipLaunchKernelGGL((k_coarse_wg<T, 1024, 8>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    case CF_JAC512: hipLaunchKernelGGL((k_coarse_jac<T, 512, 1>), one, dim3(512), 0, s, d, x, b, sweeps, stop); break;
+    case CF_JAC2: hipLaunchKernelGGL((k_coarse_jac<T, 1024, 2>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    case CF_JAC8: hipLaunchKernelGGL((k_coarse_jac<T, 1024, 8>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    case CF_WG256: hipLaunchKernelGGL((k_coarse_wg<T, 256, 2>), one, dim3(256), 0, s, d, x, b, sweeps, stop); break;
+    case CF_WG1: hipLaunchKernelGGL((k_coarse_wg<T, 1024, 1>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    case CF_WG2: hipLaunchKernelGGL((k_coarse_wg<T, 1024, 2>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    case CF_WG4: hipLaunchKernelGGL((k_coarse_wg<T, 1024, 4>), one, dim3(1024), 0, s, d, x, b, sweeps, stop); break;
+    default: {
+        const bool jac = f == CF_TILE_JAC;
+        const int n = coarse_tile_launches(jac, sweeps);
+        for (int q = 0; q < n; ++q) {
+            const CoarseTileStep st = coarse_tile_step(jac, sweeps, q);
+            const T *in = st.to_x ? tmp : x;
+            T *out = st.to_x ? x : tmp;
+            if (jac)
+                hipLaunchKernelGGL((k_coarse_tile<T, true>), coarse_tile_grid(d), dim3(CT_T), 0, s, d, in, out, b,
+                                   st.s0, st.ns, stop);
+            else
+                hipLaunchKernelGGL((k_coarse_tile<T, false>), coarse_tile_grid(d), dim3(CT_T), 0, s, d, in, out, b,
+                                   st.s0, st.ns, stop);
         }
     }
-    for (int q = kb.tx; q < n; q += 64) xg[lidx(L, q % L.nx, (q / L.nx) % L.ny, q / (L.nx * L.ny))] = x[q];
-}
-template <typename T>
-__global__ __launch_bounds__(64) void k_coarse_lds(LevelDev L, T *__restrict__ xg, const T *__restrict__ bg,
-                                                   int sweeps, const double *__restrict__ stop) {
-    coarse_lds_body<T>(hw_blk(), L, xg, bg, sweeps, stop);
-}
-
-template <typename T>
-__device__ __forceinline__ void coarse_body(const Blk &kb, const LevelDev &L, T *__restrict__ x, const T *__restrict__ b,
-                                                     T *__restrict__ tmp, int sweeps, const double *__restrict__ stop) {
-    if (*stop != 0.0) return;
-    const long n = (long)L.nx * L.ny * L.nz;
-    for (long q = kb.tx; q < n; q += COARSE_T) x[q] = T(0);
-    __syncthreads();
-    auto half = [&](int color) {
-        for (long q = kb.tx; q < n; q += COARSE_T) {
-            int i, j, k;
-            lcell(L, (int)q, i, j, k);
-            if (((i + j + k) & 1) != color) continue;
-            x[q] = (b[q] + nbsum(x, L, i, j, k)) * T(L.idiag[diag_index(L, i, j, k)]);
-        }
-        __syncthreads();
-    };
-    if (L.rb_valid) {
-        for (int s = 0; s < sweeps; ++s) { half(0); half(1); }
-        for (int s = 0; s < sweeps; ++s) { half(1); half(0); }
-    } else {
-        const T om = T(0.8);
-        for (int s = 0; s < 2 * sweeps; ++s) {
-            for (long q = kb.tx; q < n; q += COARSE_T) {
-                int i, j, k;
-                lcell(L, (int)q, i, j, k);
-                T xn = (b[q] + nbsum(x, L, i, j, k)) * T(L.idiag[diag_index(L, i, j, k)]);
-                tmp[q] = x[q] + om * (xn - x[q]);
-            }
-            __syncthreads();
-            for (long q = kb.tx; q < n; q += COARSE_T) x[q] = tmp[q];
-            __syncthreads();
-        }
     }
-}
-template <typename T>
-__global__ __launch_bounds__(COARSE_T) void k_coarse(LevelDev L, T *__restrict__ x, const T *__restrict__ b,
-                                                     T *__restrict__ tmp, int sweeps, const double *__restrict__ stop) {
-    coarse_body<T>(hw_blk(), L, x, b, tmp, sweeps, stop);
 }
 
 // ---------------------------------------------------------------------------
@@ -1082,8 +1338,7 @@ __global__ __launch_bounds__(COARSE_T) void k_coarse(LevelDev L, T *__restrict__
 // down to the coarsest, the whole V-cycle (smoothing, residual, restriction,
 // coarse sweeps, prolongation) runs in LDS with a barrier between phases, in
 // place of a few dozen launches that each cost more than their work. The
-// coarsest level sweeps on one wavefront from neighbour tables, as
-// k_coarse_lds does. Every cell's arithmetic is the multi-launch path's, so
+// coarsest level sweeps on one wavefront from neighbour tables. Every cell's arithmetic is the multi-launch path's, so
 // the result is the same bit for bit; b of level `first` comes from global
 // memory and its x goes back there for the prolongation to the level above.
 // ---------------------------------------------------------------------------
@@ -1234,7 +1489,8 @@ __device__ __forceinline__ void tail_prolong(const LevelDev &F, T *xf, const Lev
 
 // The coarsest level (n <= COARSE_LDS cells, consistent red-black colouring)
 // on wavefront 0: neighbour tables whose missing (wall) neighbours point at
-// the zero slot x[n], then the symmetric sweeps of k_coarse_lds.
+// the zero slot x[n], then the symmetric sweeps of coarse_wg (colour 1 once
+// where the order turns).
 template <typename T>
 __device__ __forceinline__ void tail_coarse(const LevelDev &L, T *x, const T *b, int sweeps,
                                             short (*nb)[COARSE_LDS], T *id, unsigned char *col) {
@@ -1272,8 +1528,8 @@ __device__ __forceinline__ void tail_coarse(const LevelDev &L, T *x, const T *b,
         wave_barrier_lds();
     };
     if (coarse_sweeps_small<T>(x, b, nb, id, col, n, sweeps, ihx2, ihy2, ihz2)) return;
-    for (int s = 0; s < sweeps; ++s) { half(0); half(1); }
-    for (int s = 0; s < sweeps; ++s) { half(1); half(0); }
+    for (int s = 1; s < 2 * sweeps; ++s) { half(0); half(1); }
+    half(0);
 }
 
 template <typename T>
@@ -1832,12 +2088,7 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
         return IBMDEM_OK;
     }
     if (l == c->nlev - 1) {
-        if (L.n <= COARSE_LDS)
-            hipLaunchKernelGGL((k_coarse_lds<T>), dim3(1), dim3(64), 0, s, d, L.x, L.b, c->cs.mg_coarse_sweeps,
-                               c->scal + SC_CONV);
-        else
-            hipLaunchKernelGGL((k_coarse<T>), dim3(1), dim3(COARSE_T), 0, s, d, L.x, L.b, L.r,
-                               c->cs.mg_coarse_sweeps, c->scal + SC_CONV);
+        launch_coarsest<T>(s, d, L.x, L.b, L.r, c->cs.mg_coarse_sweeps, c->scal + SC_CONV);
         CHECK_LAUNCH(c);
         return IBMDEM_OK;
     }
@@ -2047,7 +2298,7 @@ int poisson_setup(ibmdem_ctx *c) {
             if (need > (size_t)TAIL_BYTES || c->nlev - l > TAIL_MAXLEV) break;
             c->tail_first = l;
         }
-        if (c->tail_first == c->nlev - 1) c->tail_first = c->nlev;   // the coarsest alone: k_coarse_lds
+        if (c->tail_first == c->nlev - 1) c->tail_first = c->nlev;   // the coarsest alone: one launch as well
     }
     const char *nt = std::getenv("IBMDEM_NO_TAIL");
     if (nt && *nt && *nt != '0') c->tail_first = c->nlev;
@@ -2291,6 +2542,7 @@ struct BtArg {
     BGrid g;
     const LevelDev *lev;
     int first, last, pre, post, sweeps;
+    int s0, ns;   // the tile form's half sweeps
     T *x;
     const T *b;
     T *tmp;
@@ -2303,16 +2555,23 @@ __global__ __launch_bounds__(TAIL_T) void kb_tail(BTable<BtArg<T>> tab) {
                             glb(a.stop));
     });
 }
-template <typename T>
-__global__ __launch_bounds__(64) void kb_coarse_lds(BTable<BtArg<T>> tab) {
+template <typename T, int NT, int CP>
+__global__ __launch_bounds__(NT) void kb_coarse_jac(BTable<BtArg<T>> tab) {
     batch_for(tab, [&](const BtArg<T> &a, const Blk &kb) {
-        coarse_lds_body<T>(kb, *cst(a.lev + a.last), glb(a.x), glb(a.b), a.sweeps, glb(a.stop));
+        coarse_jac_body<T, NT, CP>(kb, *cst(a.lev + a.last), glb(a.x), glb(a.b), a.sweeps, glb(a.stop));
     });
 }
-template <typename T>
-__global__ __launch_bounds__(COARSE_T) void kb_coarse(BTable<BtArg<T>> tab) {
+template <typename T, int NT, int CP>
+__global__ __launch_bounds__(NT) void kb_coarse_wg(BTable<BtArg<T>> tab) {
     batch_for(tab, [&](const BtArg<T> &a, const Blk &kb) {
-        coarse_body<T>(kb, *cst(a.lev + a.last), glb(a.x), glb(a.b), glb(a.tmp), a.sweeps, glb(a.stop));
+        coarse_wg_body<T, NT, CP>(kb, *cst(a.lev + a.last), glb(a.x), glb(a.b), a.sweeps, glb(a.stop));
+    });
+}
+// one launch of the tile form: half sweeps s0 .. s0 + ns - 1 from tmp to x
+template <typename T, bool JAC>
+__global__ __launch_bounds__(CT_T) void kb_coarse_tile(BTable<BtArg<T>> tab) {
+    batch_for(tab, [&](const BtArg<T> &a, const Blk &kb) {
+        coarse_tile_body<T, JAC>(kb, *cst(a.lev + a.last), glb(a.tmp), glb(a.x), glb(a.b), a.s0, a.ns, glb(a.stop));
     });
 }
 
@@ -2396,13 +2655,17 @@ template <typename T>
 void launch_tail(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_tail<T>, dim3(o.blocks), dim3(TAIL_T), 0, s, table<BtArg<T>>(o));
 }
-template <typename T>
-void launch_coarse_lds(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_coarse_lds<T>, dim3(o.blocks), dim3(64), 0, s, table<BtArg<T>>(o));
+template <typename T, int NT, int CP>
+void launch_coarse_jac(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL((kb_coarse_jac<T, NT, CP>), dim3(o.blocks), dim3(NT), 0, s, table<BtArg<T>>(o));
 }
-template <typename T>
-void launch_coarse(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_coarse<T>, dim3(o.blocks), dim3(COARSE_T), 0, s, table<BtArg<T>>(o));
+template <typename T, int NT, int CP>
+void launch_coarse_wg(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL((kb_coarse_wg<T, NT, CP>), dim3(o.blocks), dim3(NT), 0, s, table<BtArg<T>>(o));
+}
+template <typename T, bool JAC>
+void launch_coarse_tile(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL((kb_coarse_tile<T, JAC>), dim3(o.blocks), dim3(CT_T), 0, s, table<BtArg<T>>(o));
 }
 void launch_matvec(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_matvec_dot, dim3(o.blocks), dim3(RB), 0, s, table<CgArg>(o));
@@ -2496,7 +2759,10 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
     };
     // the bottoms at level l
     auto bottoms = [&](int l) {
-        std::vector<BtArg<T>> tail, lds, glob;
+        // by form (coarse_form; the tails in the last list), and the tile
+        // form's launches, each over the cases that still have one to do
+        std::vector<BtArg<T>> by[CF_TILE + 1];
+        std::vector<std::vector<BtArg<T>>> tiles[2];
         for (ibmdem_ctx *c : cs) {
             if (bottom_level(c) != l) continue;
             MGLevel<T> &L = levels<T>(c)[l];
@@ -2513,21 +2779,45 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             a.stop = c->scal + SC_CONV;
             if (l >= c->tail_first) {
                 a.g = bgrid(dim3(1), dim3(TAIL_T));
-                tail.push_back(a);
-            } else if (L.n <= COARSE_LDS) {
-                a.g = bgrid(dim3(1), dim3(64));
-                lds.push_back(a);
-            } else {
-                a.g = bgrid(dim3(1), dim3(COARSE_T));
-                glob.push_back(a);
+                by[CF_TILE].push_back(a);
+                continue;
+            }
+            const CoarseForm f = coarse_form(L.d);
+            if (f < CF_TILE) {
+                a.g = bgrid(dim3(1), dim3(coarse_threads(f)));
+                by[f].push_back(a);
+                continue;
+            }
+            const bool jac = f == CF_TILE_JAC;
+            const int n = coarse_tile_launches(jac, a.sweeps);
+            if ((int)tiles[jac].size() < n) tiles[jac].resize(n);
+            a.g = bgrid(coarse_tile_grid(L.d), dim3(CT_T));
+            for (int q = 0; q < n; ++q) {
+                const CoarseTileStep st = coarse_tile_step(jac, a.sweeps, q);
+                a.s0 = st.s0;
+                a.ns = st.ns;
+                a.x = st.to_x ? L.x : L.r;
+                a.tmp = st.to_x ? L.r : L.x;
+                tiles[jac][q].push_back(a);
             }
         }
         int r;
         BOp o;
         o.kind = IBMDEM_BK_BOTTOM;
-        if ((r = add_op(ar, ops, launch_tail<T>, TAIL_T, tail, o, err))) return r;
-        if ((r = add_op(ar, ops, launch_coarse_lds<T>, 64, lds, o, err))) return r;
-        return add_op(ar, ops, launch_coarse<T>, COARSE_T, glob, o, err);
+        const BLaunch fn[CF_TILE + 1] = {launch_coarse_wg<T, 256, 2>,   launch_coarse_wg<T, 1024, 1>,
+                                         launch_coarse_wg<T, 1024, 2>,  launch_coarse_wg<T, 1024, 4>,
+                                         launch_coarse_wg<T, 1024, 8>,  launch_coarse_jac<T, 512, 1>,
+                                         launch_coarse_jac<T, 1024, 2>, launch_coarse_jac<T, 1024, 8>,
+                                         launch_tail<T>};
+        for (int f = 0; f <= CF_TILE; ++f)
+            if ((r = add_op(ar, ops, fn[f], f == CF_TILE ? TAIL_T : coarse_threads((CoarseForm)f), by[f], o, err)))
+                return r;
+        for (int jac = 0; jac < 2; ++jac)
+            for (const std::vector<BtArg<T>> &args : tiles[jac])
+                if ((r = add_op(ar, ops, jac ? launch_coarse_tile<T, true> : launch_coarse_tile<T, false>, CT_T, args,
+                                o, err)))
+                    return r;
+        return IBMDEM_OK;
     };
     for (int l = 0; l < depth; ++l) {
         // below level 0 every case that sweeps level l had its first sweep
