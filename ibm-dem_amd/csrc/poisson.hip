@@ -61,8 +61,6 @@ int pow2ceil(int v) {
     return p;
 }
 LaunchShape shape_for(int nx, int ny, int nz);
-// grid of a red-black half sweep (RB_ROWS rows per thread) on an nx*ny*nz level
-dim3 half_grid(int nx, int ny, int nz);
 // Blocks always hold RB threads (bx * by = RB, rows past the level masked),
 // so a launch over a batch of cases can run every case's blocks with one
 // block size and the same block decomposition as the case's own launch.
@@ -203,21 +201,6 @@ __device__ __forceinline__ T nbsum_pair_vals(const PairGeo &g, int h, T part, T 
     return sx + syy + szz;
 }
 
-// one red-black half sweep; each thread owns the cell of the colour in a
-// pair of x cells, in RB_ROWS = 2 adjacent rows (independent cells, so
-// their loads are in flight together, two of them shared). ZI: the level's
-// x is implicitly 0 (first sweep of a V-cycle visit); the other colour is
-// written 0. DOT (the last two level-0 sweeps of the preconditioner, whose
-// b is the CG residual r and whose x is z = M^-1 r): also one partial sum of
-// r.z over the block's updated cells into partial[pofs + block]; in the
-// mixed form (z64 set) r is read from the FP64 r64 and the sweep also
-// writes z64 = double(x), the FP64 z of its cells.
-// RES = 1 (the last pre-smoothing sweep): also the residual of the updated
-// cells, r = b - (diag x - nbsum) with the sweep's own nbsum (the other
-// colour does not change in between); RES = 2: only that residual, for the
-// cells of `color`, x unchanged. Together they give r = b - A x.
-constexpr int RB_ROWS = 2;
-static_assert(RB_ROWS == 2, "the half sweep shares loads between its two adjacent rows");
 // Two-value accesses of a colour half (8 bytes in FP32, 16 in FP64).
 template <typename T>
 struct Vec2;
@@ -239,342 +222,9 @@ __device__ __forceinline__ void st2(T *p, T v0, T v1) {
     *reinterpret_cast<typename Vec2<T>::type *>(p) = v;
 }
 
-// A half sweep with each thread on two adjacent x-pairs (pc, pc + 1, pc
-// even) of its RB_ROWS rows, on split levels whose rows hold an even number
-// of pairs: the two pairs' cells are adjacent in every colour half (and
-// every row starts at an even position), so each load and store of the
-// thread moves both values at once, half the memory instructions per cell
-// of rb_half_body. Each cell's neighbours, their association and the
-// update are rb_half_body's (nbsum_pair_vals), so x, r and z are the same
-// bit for bit; the r.z partial sums (DOT) follow this kernel's blocks.
-template <typename T, bool DOT, int RES, bool ZI>
-__device__ __forceinline__ void rb_half2_body(const Blk &kb, const LevelDev &L, T *__restrict__ x,
-                                              const T *__restrict__ b, int color, double *__restrict__ partial,
-                                              long pofs, T *__restrict__ r, const double *__restrict__ r64,
-                                              double *__restrict__ z64) {
-    const T id_int = T(L.idiag[DIAG_INTERIOR]), dg_int = T(L.diag[DIAG_INTERIOR]);
-    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
-    const int rl = L.nx >> 1, pl = rl * L.ny;
-    const int p0 = 2 * (kb.bx * kb.dx + kb.tx), k = kb.bz;
-    const int j0 = (kb.by * kb.dy + kb.ty) * RB_ROWS;
-    const bool px = L.bt[0] == IBMDEM_BC_PERIODIC, py = L.bt[2] == IBMDEM_BC_PERIODIC,
-               pz = L.bt[4] == IBMDEM_BC_PERIODIC;
-    // pairs past the row's end load from the last two (valid addresses)
-    // and are dropped at the stores
-    const int pc = min(p0, rl - 2);
-    T *own = x + (long)color * L.half;
-    T *oth = x + (long)(1 - color) * L.half;
-    // x neighbours outside the two pairs: the odd cell of pair pc - 1 (west
-    // of an even cell of pair pc) and the even cell of pair pc + 2 (east of
-    // an odd cell of pair pc + 1), as offsets from pair pc
-    const bool hw = pc > 0 || px, he = pc + 2 < rl || px;
-    const int dw = pc > 0 ? -1 : rl - 1, de = pc + 2 < rl ? 2 : 2 - rl;
-    const bool hb = k > 0 || pz, ht = k < L.nz - 1 || pz;
-    const int db = k > 0 ? -pl : (L.nz - 1) * pl, dt = k < L.nz - 1 ? pl : -(L.nz - 1) * pl;
-    const int cz = diag_count(k, L.nz, L.bt[4], L.bt[5]);
-    bool ok[RB_ROWS], hs[RB_ROWS], hn[RB_ROWS];
-    int pos[RB_ROWS], h[RB_ROWS], cyz[RB_ROWS];
-    T bo[RB_ROWS][2], av[RB_ROWS][2], xo[RB_ROWS], ys[RB_ROWS][2], yn[RB_ROWS][2], zb[RB_ROWS][2],
-        zt[RB_ROWS][2], ov[RB_ROWS][2];
-    const bool adj = j0 + 1 < L.ny;   // both rows exist: they share their y loads
-#pragma unroll
-    for (int rr = 0; rr < RB_ROWS; ++rr) {
-        const int j = min(j0 + rr, L.ny - 1);
-        ok[rr] = j0 + rr < L.ny && p0 < rl;
-        pos[rr] = (k * L.ny + j) * rl + pc;
-        h[rr] = ((j + k) & 1) == color ? 0 : 1;
-        hs[rr] = j > 0 || py;
-        hn[rr] = j < L.ny - 1 || py;
-        cyz[rr] = diag_count(j, L.ny, L.bt[2], L.bt[3]) * 4 + cz;
-        const T *q = oth + pos[rr];
-        ld2(b + (long)color * L.half + pos[rr], bo[rr][0], bo[rr][1]);
-        if (RES == 2) ld2(own + pos[rr], ov[rr][0], ov[rr][1]);
-        if (!ZI || RES == 2) {
-            ld2(q, av[rr][0], av[rr][1]);
-            xo[rr] = h[rr] == 0 ? q[hw ? dw : 0] : q[he ? de : 0];
-            ld2(q + (hb ? db : 0), zb[rr][0], zb[rr][1]);
-            ld2(q + (ht ? dt : 0), zt[rr][0], zt[rr][1]);
-        }
-    }
-    T sn[RB_ROWS][2];
-    if (ZI && RES != 2) {
-#pragma unroll
-        for (int rr = 0; rr < RB_ROWS; ++rr) sn[rr][0] = sn[rr][1] = T(0);
-    } else {
-        // row 0's north neighbours are row 1's pair values and row 1's
-        // south neighbours row 0's (when both rows exist)
-        const T *q0 = oth + pos[0], *q1 = oth + pos[1];
-        const int jr0 = min(j0, L.ny - 1), jr1 = min(j0 + 1, L.ny - 1);   // the rows' (clamped) indices
-        const int ds0 = jr0 > 0 ? -rl : (L.ny - 1) * rl;
-        const int dn1 = jr1 < L.ny - 1 ? rl : -(L.ny - 1) * rl;
-        ld2(q0 + (hs[0] ? ds0 : 0), ys[0][0], ys[0][1]);
-        ld2(q1 + (hn[1] ? dn1 : 0), yn[1][0], yn[1][1]);
-        if (adj) {
-            yn[0][0] = av[1][0]; yn[0][1] = av[1][1];
-            ys[1][0] = av[0][0]; ys[1][1] = av[0][1];
-        } else {
-            const int dn0 = jr0 < L.ny - 1 ? rl : -(L.ny - 1) * rl;
-            ld2(q0 + (hn[0] ? dn0 : 0), yn[0][0], yn[0][1]);
-            ys[1][0] = ys[0][0]; ys[1][1] = ys[0][1];   // row 1 does not exist
-        }
-#pragma unroll
-        for (int rr = 0; rr < RB_ROWS; ++rr)
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                // nbsum_pair_vals of the cell of pair pc + c: its pair value
-                // and its other x neighbour (inside the two pairs but for
-                // the outer ones)
-                const bool even = h[rr] == 0;
-                const T part = av[rr][c];
-                const T oxv = even ? (c == 0 ? xo[rr] : av[rr][0]) : (c == 0 ? av[rr][1] : xo[rr]);
-                const bool pw = even ? (c == 0 ? hw : true) : true;
-                const bool pe = even ? true : (c == 0 ? true : he);
-                const T vw = even ? oxv : part, ve = even ? part : oxv;
-                const T xw = pw ? vw : T(0), xe = pe ? ve : T(0);
-                const T xs = hs[rr] ? ys[rr][c] : T(0), xn = hn[rr] ? yn[rr][c] : T(0);
-                const T xb = hb ? zb[rr][c] : T(0), xt = ht ? zt[rr][c] : T(0);
-                const T sx = (xw + xe) * ihx2;
-                const T syy = (xs + xn) * ihy2;
-                const T szz = (xb + xt) * ihz2;
-                sn[rr][c] = sx + syy + szz;
-            }
-    }
-    double dsum = 0.0;
-#pragma unroll
-    for (int rr = 0; rr < RB_ROWS; ++rr) {
-        if (!ok[rr]) continue;
-        const int o = pos[rr];
-        const long go = (long)color * L.half + o;
-        T out[2], res[2];
-        double z[2];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const int di = diag_count(2 * (pc + c) + h[rr], L.nx, L.bt[0], L.bt[1]) * 16 + cyz[rr];
-            if (RES == 2) {
-                T dg;
-                if (di == DIAG_INTERIOR) dg = dg_int;
-                else dg = T(L.diag[di]);
-                res[c] = bo[rr][c] - (dg * ov[rr][c] - sn[rr][c]);
-                continue;
-            }
-            T id;
-            if (di == DIAG_INTERIOR) id = id_int;
-            else id = T(L.idiag[di]);
-            if (ZI) {
-                out[c] = (bo[rr][c] + T(0)) * id;
-            } else {
-                const T xn = (bo[rr][c] + sn[rr][c]) * id;
-                out[c] = xn;
-                if (RES == 1) {
-                    T dg;
-                    if (di == DIAG_INTERIOR) dg = dg_int;
-                    else dg = T(L.diag[di]);
-                    res[c] = bo[rr][c] - (dg * xn - sn[rr][c]);
-                }
-                z[c] = double(xn);
-            }
-        }
-        if (RES == 2) {
-            st2(r + go, res[0], res[1]);
-            continue;
-        }
-        if (ZI) st2(oth + o, T(0), T(0));
-        st2(own + o, out[0], out[1]);
-        if (RES == 1) st2(r + go, res[0], res[1]);
-        if (DOT) {
-            if (z64) {
-                double r0, r1;
-                ld2(r64 + go, r0, r1);
-                st2(z64 + go, z[0], z[1]);
-                dsum += r0 * z[0];
-                dsum += r1 * z[1];
-            } else {
-                dsum += double(bo[rr][0]) * z[0];
-                dsum += double(bo[rr][1]) * z[1];
-            }
-        }
-    }
-    if (DOT) {
-        __shared__ double red[RB];
-        const int nt = kb.dx * kb.dy, t = kb.ty * kb.dx + kb.tx;
-        red[t] = dsum;
-        __syncthreads();
-        for (int st = nt / 2; st > 0; st >>= 1) {
-            if (t < st) red[t] += red[t + st];
-            __syncthreads();
-        }
-        if (t == 0) partial[pofs + ((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = red[0];
-    }
-}
-
-template <typename T, typename TB, bool DOT = false, int RES = 0, bool ZI = false, bool X2 = false>
-__device__ __forceinline__ void rb_half_body(const Blk &kb, const LevelDev &L, T *__restrict__ x, const TB *__restrict__ b,
-                                                int color, const double *__restrict__ stop,
-                                                double *__restrict__ partial, long pofs, T *__restrict__ r,
-                                                const double *__restrict__ r64,
-                                                double *__restrict__ z64) {
-    if (*stop != 0.0) return;
-    if constexpr (X2) {
-        static_assert(std::is_same<T, TB>::value, "the two-pair sweep reads b in the level's type");
-        rb_half2_body<T, DOT, RES, ZI>(kb, L, x, b, color, partial, pofs, r, r64, z64);
-        return;
-    }
-    const T id_int = T(L.idiag[DIAG_INTERIOR]), dg_int = T(L.diag[DIAG_INTERIOR]);
-    const int ip = kb.bx * kb.dx + kb.tx;
-    const int k = kb.bz;
-    double dsum = 0.0;
-    if (L.split) {
-        // Two phases over the thread's rows: every load (b, the other
-        // colour's neighbours, the own value of the residual pass) is issued
-        // before the first store, so the rows' loads are in flight together.
-        // Stores go to this colour's half and x is read from the other half
-        // (the residual pass reads its own cells but does not write x), so
-        // the order changes no value.
-        T *own = x + (long)color * L.half;
-        T *oth = x + (long)(1 - color) * L.half;
-        bool ok[RB_ROWS];
-        int pos[RB_ROWS], dix[RB_ROWS];
-        TB bo[RB_ROWS];
-        T sn[RB_ROWS], ov[RB_ROWS];
-        // the thread's two rows are adjacent (j0, j0 + 1); rows and pairs
-        // past the level's end load from the last one (valid addresses, no
-        // branch) and are dropped in phase two
-        const int j0 = (kb.by * kb.dy + kb.ty) * RB_ROWS;
-        const int ipc = min(ip, (L.nx >> 1) - 1);
-        PairGeo g[RB_ROWS];
-        int h[RB_ROWS];
-#pragma unroll
-        for (int rr = 0; rr < RB_ROWS; ++rr) {
-            const int j = j0 + rr;
-            ok[rr] = j < L.ny && ip < (L.nx >> 1);
-            g[rr] = pair_geo(L, ipc, min(j, L.ny - 1), k);
-            h[rr] = g[rr].ca == color ? 0 : 1;   // which cell of the pair has this colour
-            pos[rr] = g[rr].pos;
-            dix[rr] = (h[rr] ? g[rr].cx1 : g[rr].cx0) * 16 + g[rr].cyz;
-            bo[rr] = b[(long)color * L.half + g[rr].pos];
-            if (RES == 2) ov[rr] = own[g[rr].pos];
-        }
-        if (ZI && RES != 2) {
-            sn[0] = sn[1] = T(0);
-        } else {
-            // nbsum_pair of both rows with two loads shared: when both rows
-            // exist, row 0's north neighbour is row 1's pair value and row
-            // 1's south neighbour is row 0's
-            const T *q0 = oth + g[0].pos, *q1 = oth + g[1].pos;
-            const T a = q0[0], c = q1[0];
-            const T ys0 = q0[g[0].hs ? g[0].ds : 0], yn1 = q1[g[1].hn ? g[1].dn : 0];
-            const T xo0 = q0[h[0] == 0 ? (g[0].hw ? g[0].dw : 0) : (g[0].he ? g[0].de : 0)];
-            const T xo1 = q1[h[1] == 0 ? (g[1].hw ? g[1].dw : 0) : (g[1].he ? g[1].de : 0)];
-            const T zb0 = q0[g[0].hb ? g[0].db : 0], zt0 = q0[g[0].ht ? g[0].dt : 0];
-            const T zb1 = q1[g[1].hb ? g[1].db : 0], zt1 = q1[g[1].ht ? g[1].dt : 0];
-            T yn0 = c, ys1 = a;
-            if (j0 + 1 >= L.ny) yn0 = q0[g[0].hn ? g[0].dn : 0];   // row 1 does not exist
-            sn[0] = nbsum_pair_vals(g[0], h[0], a, xo0, ys0, yn0, zb0, zt0, L);
-            sn[1] = nbsum_pair_vals(g[1], h[1], c, xo1, ys1, yn1, zb1, zt1, L);
-        }
-#pragma unroll
-        for (int rr = 0; rr < RB_ROWS; ++rr) {
-            if (!ok[rr]) continue;
-            const int o = pos[rr], di = dix[rr];
-            if (RES == 2) {
-                T dg;
-                if (di == DIAG_INTERIOR) dg = dg_int;
-                else dg = T(L.diag[di]);
-                r[(long)color * L.half + o] = T(bo[rr]) - (dg * ov[rr] - sn[rr]);
-                continue;
-            }
-            // cells with both neighbours in every dimension (all but the
-            // boundary layers) share table entry DIAG_INTERIOR, read once
-            T id;
-            if (di == DIAG_INTERIOR) id = id_int;
-            else id = T(L.idiag[di]);
-            if (ZI) {
-                oth[o] = T(0);
-                own[o] = (T(bo[rr]) + T(0)) * id;
-            } else {
-                const T xn = (T(bo[rr]) + sn[rr]) * id;
-                own[o] = xn;
-                if (RES == 1) {
-                    T dg;
-                    if (di == DIAG_INTERIOR) dg = dg_int;
-                    else dg = T(L.diag[di]);
-                    r[(long)color * L.half + o] = T(bo[rr]) - (dg * xn - sn[rr]);
-                }
-                if (DOT) {
-                    const long go = (long)color * L.half + o;
-                    if (z64) {
-                        z64[go] = double(xn);
-                        dsum += r64[go] * double(xn);
-                    } else {
-                        dsum += double(bo[rr]) * double(xn);
-                    }
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int rr = 0; rr < RB_ROWS; ++rr) {
-            const int j = (kb.by * kb.dy + kb.ty) * RB_ROWS + rr;
-            if (j >= L.ny) continue;
-            const int i = 2 * ip + ((j + k + color) & 1);
-            const int o = lidx(L, i, j, k);
-            if (ZI) {
-                const int io = 2 * ip + ((j + k + color + 1) & 1);
-                if (io < L.nx) x[lidx(L, io, j, k)] = T(0);
-                if (i >= L.nx) continue;
-                const T id = T(L.idiag[diag_index(L, i, j, k)]);
-                x[o] = (T(b[o]) + T(0)) * id;
-                continue;
-            }
-            if (i >= L.nx) continue;
-            const int di = diag_index(L, i, j, k);
-            const T sn = nbsum(x, L, i, j, k);
-            if (RES == 2) {
-                r[o] = T(b[o]) - (T(L.diag[di]) * x[o] - sn);
-                continue;
-            }
-            const T xn = (T(b[o]) + sn) * T(L.idiag[di]);
-            x[o] = xn;
-            if (RES == 1) r[o] = T(b[o]) - (T(L.diag[di]) * xn - sn);
-            if (DOT) {
-                if (z64) {
-                    z64[o] = double(xn);
-                    dsum += r64[o] * double(xn);
-                } else {
-                    dsum += double(b[o]) * double(xn);
-                }
-            }
-        }
-    }
-    if (DOT) {
-        __shared__ double red[RB];
-        const int nt = kb.dx * kb.dy, t = kb.ty * kb.dx + kb.tx;
-        red[t] = dsum;
-        __syncthreads();
-        for (int st = nt / 2; st > 0; st >>= 1) {
-            if (t < st) red[t] += red[t + st];
-            __syncthreads();
-        }
-        if (t == 0) partial[pofs + ((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = red[0];
-    }
-}
-template <typename T, typename TB, bool DOT = false, int RES = 0, bool ZI = false, bool X2 = false>
-__global__ __launch_bounds__(RB) void k_rb_half(LevelDev L, T *__restrict__ x, const TB *__restrict__ b,
-                                                int color, const double *__restrict__ stop,
-                                                double *__restrict__ partial, long pofs, T *__restrict__ r,
-                                                const double *__restrict__ r64 = nullptr,
-                                                double *__restrict__ z64 = nullptr) {
-    rb_half_body<T, TB, DOT, RES, ZI, X2>(hw_blk(), L, x, b, color, stop, partial, pofs, r, r64, z64);
-}
-
-dim3 half_grid(int nx, int ny, int nz) {
-    const LaunchShape rb = shape_for(div_up(nx, 2), ny, nz);
-    return dim3(rb.grid.x, div_up(ny, RB_ROWS * (int)rb.block.y), rb.grid.z);
-}
-
-// The half sweep's launch on a level: two-pair threads (rb_half2_body) where
-// the level is split and its rows hold an even number of pairs, else one
-// pair per thread.
+// The matrix-vector product's launch on a level: two rows per thread, two-pair
+// threads where the level is split and its rows hold an even number of
+// pairs, else one pair per thread.
 struct SweepShape {
     dim3 grid, block;
     bool x2;
@@ -582,7 +232,7 @@ struct SweepShape {
 SweepShape sweep_shape(const LevelDev &d) {
     const bool x2 = d.split && (d.nx >> 1) % 2 == 0;
     const LaunchShape sh = shape_for(x2 ? d.nx / 4 : div_up(d.nx, 2), d.ny, d.nz);
-    return {dim3(sh.grid.x, div_up(d.ny, RB_ROWS * (int)sh.block.y), sh.grid.z), sh.block, x2};
+    return {dim3(sh.grid.x, div_up(d.ny, 2 * (int)sh.block.y), sh.grid.z), sh.block, x2};
 }
 
 // cell index of a virtual coordinate one step beyond the level: a wall side
@@ -596,81 +246,6 @@ __device__ __forceinline__ int tile_coord(int v, int n, int lo, int hi) {
     return min(max(v, 0), n - 1);
 }
 
-// b_c = (1/8) sum w r_f over the 4x4x4 fine cells, w = wz*wy*wx from
-// (1/4,3/4,3/4,1/4). A block owns RS_CX x RS_CY coarse cells of one coarse
-// plane; the fine residual they weigh (2 RS_CX + 2 by 2 RS_CY + 2 by 4 fine
-// cells at virtual coordinates, mapped by tile_coord) is staged in LDS with
-// coalesced loads, and each thread sums its 64 terms from there in the
-// (z, y, x) order. With xc, the coarse level's first smoothing sweep (x = 0
-// before it: colour 0 takes (b + 0)/diag, colour 1 stays 0) is done here
-// too, each cell's value as that sweep computes it from the b just written,
-// and the coarse level's V-cycle starts with its second half sweep.
-constexpr int RS_CX = 32, RS_CY = 8;
-constexpr int RS_RX = 2 * RS_CX + 2, RS_RY = 2 * RS_CY + 2, RS_TILE = RS_RX * RS_RY * 4;
-static_assert(RS_CX * RS_CY == RB, "one coarse cell per thread");
-template <typename T>
-__device__ __forceinline__ void restrict_body(const Blk &kb, const LevelDev &F, const T *__restrict__ rf, const LevelDev &Cl,
-                                                 T *__restrict__ bc, T *__restrict__ xc, const double *__restrict__ stop) {
-    if (*stop != 0.0) return;
-    __shared__ T tile[RS_TILE];
-    const int t = kb.tx;
-    const int I0 = kb.bx * RS_CX, J0 = kb.by * RS_CY, K = kb.bz;
-    // The tile's rows r = z RS_RY + y: wavefront w loads columns 0..63 of
-    // the rows of fine plane z = w; a row's (j, k) and its part of the
-    // storage index are the same on every lane (scalars, k once per
-    // wavefront), the lane's part (its column's i) is computed once. Columns
-    // 64.. of every row are one more load for the first threads. All loads
-    // are issued before the first LDS store waits.
-    constexpr int NW = RB / 64, NROW = RS_RY * 4, RPW = NROW / NW, NEXTRA = (RS_RX - 64) * NROW;
-    static_assert(NW == 4 && RPW == RS_RY && RS_RX >= 64 && NEXTRA <= RB, "row split of the restriction tile");
-    const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int half = F.split ? F.half : 0, rl = F.split ? F.nx >> 1 : F.nx;
-    const int il = tile_coord(2 * I0 - 1 + lane, F.nx, F.bt[0], F.bt[1]);
-    // the lane's offset within a row for row parity 0 and 1
-    const int lo0 = F.split ? (il & 1) * half + (il >> 1) : il;
-    const int lo1 = F.split ? ((il & 1) ^ 1) * half + (il >> 1) : il;
-    T v[RPW], ve = T(0);
-    const int k = tile_coord(2 * K - 1 + w, F.nz, F.bt[4], F.bt[5]);
-#pragma unroll
-    for (int u = 0; u < RPW; ++u) {
-        const int j = tile_coord(2 * J0 - 1 + u, F.ny, F.bt[2], F.bt[3]);
-        const int rowoff = (k * F.ny + j) * rl;
-        v[u] = rf[rowoff + (((j + k) & 1) ? lo1 : lo0)];
-    }
-    if (t < NEXTRA) {
-        const int r = t / (RS_RX - 64), x = 64 + t % (RS_RX - 64), y = r % RS_RY, z = r / RS_RY;
-        const int i = tile_coord(2 * I0 - 1 + x, F.nx, F.bt[0], F.bt[1]);
-        const int j = tile_coord(2 * J0 - 1 + y, F.ny, F.bt[2], F.bt[3]);
-        const int k = tile_coord(2 * K - 1 + z, F.nz, F.bt[4], F.bt[5]);
-        ve = rf[lidx(F, i, j, k)];
-    }
-#pragma unroll
-    for (int u = 0; u < RPW; ++u) tile[(w * RS_RY + u) * RS_RX + lane] = v[u];
-    if (t < NEXTRA) tile[(t / (RS_RX - 64)) * RS_RX + 64 + t % (RS_RX - 64)] = ve;
-    __syncthreads();
-    const int I = I0 + t % RS_CX, J = J0 + t / RS_CX;
-    if (I >= Cl.nx || J >= Cl.ny) return;
-    const T wt[4] = {T(0.25), T(0.75), T(0.75), T(0.25)};
-    const T *base = tile + 2 * (t / RS_CX) * RS_RX + 2 * (t % RS_CX);
-    T s = T(0);
-    for (int c3 = 0; c3 < 4; ++c3)
-        for (int c2 = 0; c2 < 4; ++c2)
-            for (int c1 = 0; c1 < 4; ++c1) {
-                T w = wt[c3] * wt[c2] * wt[c1];
-                s = s + w * base[(c3 * RS_RY + c2) * RS_RX + c1];
-            }
-    const T bv = T(0.125) * s;
-    const int o = lidx(Cl, I, J, K);
-    bc[o] = bv;
-    if (xc) xc[o] = ((I + J + K) & 1) ? T(0) : (bv + T(0)) * T(Cl.idiag[diag_index(Cl, I, J, K)]);
-}
-template <typename T>
-__global__ __launch_bounds__(RB) void k_restrict(LevelDev F, const T *__restrict__ rf, LevelDev Cl,
-                                                 T *__restrict__ bc, T *__restrict__ xc,
-                                                 const double *__restrict__ stop) {
-    restrict_body<T>(hw_blk(), F, rf, Cl, bc, xc, stop);
-}
-
 __device__ __forceinline__ void parents(int f, int nc, int lo, int hi, int &p0, int &p1) {
     int cc = f / 2;
     int nb = (f & 1) ? cc + 1 : cc - 1;
@@ -679,238 +254,8 @@ __device__ __forceinline__ void parents(int f, int nc, int lo, int hi, int &p0, 
     p0 = cc; p1 = nb;
 }
 
-// x_f += sum (wz*wy*wx) x_c over the 8 parents, weights (3/4 own, 1/4
-// neighbour). The block's coarse parents (its x-pairs' coarse columns +-1,
-// its rows' coarse rows +-1, the plane's two parent planes) are staged in LDS
-// once, so each coarse value is read from memory once per block instead of
-// by every fine cell it weighs into; the sum is the same 8 products in the
-// same order.
-constexpr int PRO_TILE = 1024;   // (bx + 2) * (by / 2 + 2) * 2 <= 528 for the shapes of shape_for
-template <typename T>
-__device__ __forceinline__ void prolong_body(const Blk &kb, const LevelDev &F, T *__restrict__ xf, const LevelDev &Cl,
-                                                const T *__restrict__ xc, const double *__restrict__ stop) {
-    if (*stop != 0.0) return;
-    __shared__ T tile[PRO_TILE];
-    const int bx = kb.dx, by = kb.dy;
-    const int TX = bx + 2, TY = by / 2 + 2;
-    const int I0 = kb.bx * bx - 1, J0 = (kb.by * by) / 2 - 1;
-    const int k = kb.bz;
-    int pk[2];
-    parents(k, Cl.nz, Cl.bt[4], Cl.bt[5], pk[0], pk[1]);
-    const int t = kb.ty * bx + kb.tx;
-    // the thread's two fine values are loaded first, so their latency
-    // overlaps the staging of the coarse tile
-    const int ip = kb.bx * bx + kb.tx;
-    const int j = kb.by * by + kb.ty;
-    T xo[2] = {T(0), T(0)};
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-        if (j < F.ny && 2 * ip + h < F.nx) xo[h] = xf[lidx(F, 2 * ip + h, j, k)];
-    if (bx == 64) {
-        // one wavefront per kb.ty: wavefront w stages columns 0..63 of
-        // tile rows w, w + by, ... (row r = c TY + y); a row's (J, plane) and
-        // its part of the storage index are scalars, the lane's column index
-        // is computed once; columns 64 and 65 are one more load for the first
-        // threads. All loads are issued before the LDS stores wait.
-        const int lane = kb.tx, w = kb.ty, NROW = 2 * TY;
-        const int half = Cl.split ? Cl.half : 0, rl = Cl.split ? Cl.nx >> 1 : Cl.nx;
-        const int Il = tile_coord(I0 + lane, Cl.nx, Cl.bt[0], Cl.bt[1]);
-        const int lo0 = Cl.split ? (Il & 1) * half + (Il >> 1) : Il;
-        const int lo1 = Cl.split ? ((Il & 1) ^ 1) * half + (Il >> 1) : Il;
-        T v[4], ve = T(0);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int r = w + u * by;
-            v[u] = T(0);
-            if (r < NROW) {
-                const int y = r % TY, c = r / TY;
-                const int J = tile_coord(J0 + y, Cl.ny, Cl.bt[2], Cl.bt[3]), K = pk[c];
-                v[u] = xc[(K * Cl.ny + J) * rl + (((J + K) & 1) ? lo1 : lo0)];
-            }
-        }
-        if (t < 2 * NROW) {
-            const int r = t >> 1, x = 64 + (t & 1), y = r % TY, c = r / TY;
-            const int I = tile_coord(I0 + x, Cl.nx, Cl.bt[0], Cl.bt[1]);
-            const int J = tile_coord(J0 + y, Cl.ny, Cl.bt[2], Cl.bt[3]);
-            ve = xc[lidx(Cl, I, J, pk[c])];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int r = w + u * by;
-            if (r < NROW) tile[r * TX + lane] = v[u];
-        }
-        if (t < 2 * NROW) tile[(t >> 1) * TX + 64 + (t & 1)] = ve;
-    } else
-    // up to four loads of a thread in flight before the LDS stores wait
-    for (int q0 = t; q0 < 2 * TY * TX; q0 += 4 * bx * by) {
-        T v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u * bx * by;
-            if (q < 2 * TY * TX) {
-                const int x = q % TX, y = (q / TX) % TY, c = q / (TX * TY);
-                const int I = tile_coord(I0 + x, Cl.nx, Cl.bt[0], Cl.bt[1]);
-                const int J = tile_coord(J0 + y, Cl.ny, Cl.bt[2], Cl.bt[3]);
-                v[u] = xc[lidx(Cl, I, J, pk[c])];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int q = q0 + u * bx * by;
-            if (q < 2 * TY * TX) tile[q] = v[u];
-        }
-    }
-    __syncthreads();
-    if (j >= F.ny) return;
-    const T wt[2] = {T(0.75), T(0.25)};
-    // tile rows of the own and the neighbour coarse row
-    const int ty[2] = {j / 2 - J0, j / 2 + ((j & 1) ? 1 : -1) - J0};
-    // the thread's x-pair (2p, 2p+1), one cell of each colour
-    for (int h = 0; h < 2; ++h) {
-        const int i = 2 * ip + h;
-        if (i >= F.nx) return;
-        const int tx[2] = {i / 2 - I0, i / 2 + ((i & 1) ? 1 : -1) - I0};
-        T s = T(0);
-        for (int c3 = 0; c3 < 2; ++c3)
-            for (int c2 = 0; c2 < 2; ++c2)
-                for (int c1 = 0; c1 < 2; ++c1) {
-                    T w = wt[c3] * wt[c2] * wt[c1];
-                    s = s + w * tile[(c3 * TY + ty[c2]) * TX + tx[c1]];
-                }
-        xf[lidx(F, i, j, k)] = xo[h] + s;
-    }
-}
-template <typename T>
-__global__ __launch_bounds__(RB) void k_prolong(LevelDev F, T *__restrict__ xf, LevelDev Cl,
-                                                const T *__restrict__ xc, const double *__restrict__ stop) {
-    prolong_body<T>(hw_blk(), F, xf, Cl, xc, stop);
-}
-
-// The same prolongation with each thread on two adjacent x-pairs (pc, pc +
-// 1) of its row, on split fine levels whose rows hold an even number of
-// pairs: the thread's four fine values are two two-value loads (and
-// stores) of the colour halves. The block's coarse parents (its pairs'
-// coarse columns +-1, rows +-1, the plane's two parent planes) are staged in
-// LDS as prolong_body stages them; each fine value gets the same 8 products
-// in the same order.
-constexpr int PRO2_TILE = 1040;   // 2 (by / 2 + 2) (2 bx + 2) for the shapes of shape_for
-template <typename T>
-__device__ __forceinline__ void prolong2_body(const Blk &kb, const LevelDev &F, T *__restrict__ xf,
-                                              const LevelDev &Cl, const T *__restrict__ xc,
-                                              const double *__restrict__ stop) {
-    if (*stop != 0.0) return;
-    __shared__ T tile[PRO2_TILE];
-    const int bx = kb.dx, by = kb.dy;
-    const int TX = 2 * bx + 2, TY = by / 2 + 2;
-    const int I0 = 2 * kb.bx * bx - 1, J0 = (kb.by * by) / 2 - 1;
-    const int k = kb.bz;
-    int pk[2];
-    parents(k, Cl.nz, Cl.bt[4], Cl.bt[5], pk[0], pk[1]);
-    const int t = kb.ty * bx + kb.tx;
-    const int rl = F.nx >> 1;
-    const int p0 = 2 * (kb.bx * bx + kb.tx), pc = min(p0, rl - 2);
-    const int j = kb.by * by + kb.ty, jc = min(j, F.ny - 1);
-    const int ca = (jc + k) & 1;
-    const long pos = (long)(k * F.ny + jc) * rl + pc;
-    // fine values first (even cells of the two pairs in half ca, odd cells in
-    // half 1 - ca), so their latency overlaps the staging
-    T xo[2][2];
-    ld2(xf + (long)ca * F.half + pos, xo[0][0], xo[0][1]);
-    ld2(xf + (long)(1 - ca) * F.half + pos, xo[1][0], xo[1][1]);
-    // The tile's rows r = c TY + y (coarse row J0 + y of parent plane c).
-    // Rows of 64 or more columns: wavefront w stages rows w, w + NW, ...; a
-    // row's (J, K) are the same on every lane (scalars), and lane l takes
-    // columns l, l + 64, l + 128 (< TX), whose coarse indices it maps once.
-    // Column x is stored at (x & 1) * TXH + x / 2 of its row: the summing
-    // loop's lanes read columns two apart, which land in consecutive words.
-    const int TXH = bx + 1, NROW = 2 * TY, NW = bx * by / 64;
-    if (TX >= 64) {
-        const int lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-        int Ic[3];
-#pragma unroll
-        for (int u = 0; u < 3; ++u) Ic[u] = tile_coord(I0 + lane + 64 * u, Cl.nx, Cl.bt[0], Cl.bt[1]);
-        for (int r = w; r < NROW; r += NW) {
-            const int y = r % TY, c = r / TY;
-            const int J = tile_coord(J0 + y, Cl.ny, Cl.bt[2], Cl.bt[3]), K = pk[c];
-            T v[3];
-#pragma unroll
-            for (int u = 0; u < 3; ++u)
-                if (lane + 64 * u < TX) v[u] = xc[lidx(Cl, Ic[u], J, K)];
-#pragma unroll
-            for (int u = 0; u < 3; ++u) {
-                const int x = lane + 64 * u;
-                if (x < TX) tile[r * TX + (x & 1) * TXH + (x >> 1)] = v[u];
-            }
-        }
-    } else {
-        // short rows (blocks narrower than 32 pair-pairs): the tile's
-        // elements dealt to the threads in order, up to four loads of a
-        // thread in flight before the LDS stores wait
-        const int NT = NROW * TX;
-        for (int q0 = t; q0 < NT; q0 += 4 * bx * by) {
-            T v[4];
-            int dst[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int q = q0 + u * bx * by;
-                dst[u] = -1;
-                if (q < NT) {
-                    const int r = q / TX, x = q - r * TX, y = r % TY, c = r / TY;
-                    const int I = tile_coord(I0 + x, Cl.nx, Cl.bt[0], Cl.bt[1]);
-                    const int J = tile_coord(J0 + y, Cl.ny, Cl.bt[2], Cl.bt[3]);
-                    v[u] = xc[lidx(Cl, I, J, pk[c])];
-                    dst[u] = r * TX + (x & 1) * TXH + (x >> 1);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (dst[u] >= 0) tile[dst[u]] = v[u];
-        }
-    }
-    __syncthreads();
-    if (j >= F.ny || p0 >= rl) return;
-    const T wt[2] = {T(0.75), T(0.25)};
-    const int ty[2] = {j / 2 - J0, j / 2 + ((j & 1) ? 1 : -1) - J0};
-    T out[2][2];
-#pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int i = 2 * (pc + c) + h;
-            const int tx[2] = {i / 2 - I0, i / 2 + ((i & 1) ? 1 : -1) - I0};
-            const int sx[2] = {(tx[0] & 1) * TXH + (tx[0] >> 1), (tx[1] & 1) * TXH + (tx[1] >> 1)};
-            T s = T(0);
-            for (int c3 = 0; c3 < 2; ++c3)
-                for (int c2 = 0; c2 < 2; ++c2)
-                    for (int c1 = 0; c1 < 2; ++c1) {
-                        T wgt = wt[c3] * wt[c2] * wt[c1];
-                        s = s + wgt * tile[(c3 * TY + ty[c2]) * TX + sx[c1]];
-                    }
-            out[h][c] = xo[h][c] + s;
-        }
-    st2(xf + (long)ca * F.half + pos, out[0][0], out[0][1]);
-    st2(xf + (long)(1 - ca) * F.half + pos, out[1][0], out[1][1]);
-}
-template <typename T>
-__global__ __launch_bounds__(RB) void k_prolong2(LevelDev F, T *__restrict__ xf, LevelDev Cl,
-                                                 const T *__restrict__ xc, const double *__restrict__ stop) {
-    prolong2_body<T>(hw_blk(), F, xf, Cl, xc, stop);
-}
-
-// The prolongation's launch onto fine level d (one row per thread): two
-// pairs per thread where sweep_shape takes two, else one; ok = false when
-// the block's coarse tile would not fit the kernel's LDS tile.
-struct ProlongShape {
-    dim3 grid, block;
-    bool x2, ok;
-};
-ProlongShape prolong_shape(const LevelDev &d) {
-    const bool x2 = d.split && (d.nx >> 1) % 2 == 0;
-    const LaunchShape sh = shape_for(x2 ? d.nx / 4 : div_up(d.nx, 2), d.ny, d.nz);
-    const unsigned bx = sh.block.x, by = sh.block.y;
-    const unsigned need = x2 ? (2 * bx + 2) * (by / 2 + 2) * 2 : (bx + 2) * (by / 2 + 2) * 2;
-    return {sh.grid, sh.block, x2, by % 2 == 0 && need <= (unsigned)(x2 ? PRO2_TILE : PRO_TILE)};
-}
+#include "mgmarch.hpp"
+#include "mgtile.hpp"
 
 // ---------------------------------------------------------------------------
 // The coarsest level of a hierarchy: `sweeps` symmetric pairs of red-black
@@ -1350,120 +695,87 @@ static_assert(sizeof(LevelDev) % 4 == 0, "level descriptors copied by words");
 // divisions go through udiv_small)
 static_assert(TAIL_BYTES / 12 < (1 << 14), "tail levels small enough for udiv_small");
 
+// One half sweep of a level above the coarsest (split), by x-pairs. zero: x
+// is 0 before it, so the other colour takes part with 0 (a black sweep
+// follows, which reads red cells alone).
 template <typename T>
 __device__ __forceinline__ void tail_half(const LevelDev &L, T *x, const T *b, int color, bool zero) {
-    const int n = L.nx * L.ny * L.nz;
-    if (L.split) {   // by x-pairs, as k_rb_half
-        const int rl = L.nx >> 1;
-        T *own = x + color * L.half, *oth = x + (1 - color) * L.half;
-        for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
-            const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
-            const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
-            const int h = g.ca == color ? 0 : 1;
-            const T id = T(L.idiag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
-            const T bo = T(b[color * L.half + p]);
-            if (zero) {
-                oth[p] = T(0);
-                own[p] = (bo + T(0)) * id;
-            } else {
-                own[p] = (bo + nbsum_pair(oth, g, h, L)) * id;
-            }
-        }
-        __syncthreads();
-        return;
-    }
-    for (int q = threadIdx.x; q < n; q += TAIL_T) {
-        int i, j, k;
-        lcell_small(L, q, i, j, k);
-        if (((i + j + k) & 1) != color) {
-            if (zero) x[q] = T(0);
-            continue;
-        }
-        const T id = T(L.idiag[diag_index(L, i, j, k)]);
-        x[q] = zero ? (T(b[q]) + T(0)) * id : (T(b[q]) + nbsum(x, L, i, j, k)) * id;
+    const int rl = L.nx >> 1;
+    T *own = x + color * L.half, *oth = x + (1 - color) * L.half;
+    for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
+        const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
+        const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
+        const int h = g.ca == color ? 0 : 1;
+        const T id = T(L.idiag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
+        const T bo = T(b[color * L.half + p]);
+        own[p] = zero ? (bo + T(0)) * id : (bo + nbsum_pair(oth, g, h, L)) * id;
     }
     __syncthreads();
 }
 
+// the residual after the last black sweep (in FP64 of the red cells alone, as
+// the passes of mgmarch.hpp); every level above the coarsest is split
 template <typename T>
 __device__ __forceinline__ void tail_residual(const LevelDev &L, const T *x, const T *b, T *r) {
-    const int n = L.nx * L.ny * L.nz;
-    if (L.split) {   // by x-pairs, as the residual of k_rb_half
-        const int rl = L.nx >> 1;
-        for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
-            const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
-            const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
-            for (int h = 0; h < 2; ++h) {
-                const int own = (h ? 1 - g.ca : g.ca) * L.half, oth = (h ? g.ca : 1 - g.ca) * L.half;
-                const T dg = T(L.diag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
-                r[own + p] = T(b[own + p]) - (dg * x[own + p] - nbsum_pair(x + oth, g, h, L));
-            }
+    const int rl = L.nx >> 1;
+    for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
+        const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
+        const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
+        for (int c = 0; c < (RES_BLACK<T> ? 2 : 1); ++c) {
+            const int h = g.ca ^ c, own = c * L.half;   // the pair's cell of colour c
+            const T dg = T(L.diag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
+            r[own + p] = T(b[own + p]) - (dg * x[own + p] - nbsum_pair(x + (1 - c) * L.half, g, h, L));
         }
-        __syncthreads();
-        return;
-    }
-    for (int q = threadIdx.x; q < n; q += TAIL_T) {
-        int i, j, k;
-        lcell_small(L, q, i, j, k);
-        const T dg = T(L.diag[diag_index(L, i, j, k)]);
-        r[q] = T(b[q]) - (dg * x[q] - nbsum(x, L, i, j, k));
     }
     __syncthreads();
 }
 
+// restrict_body's sum from the level's residual in LDS
 template <typename T>
-__device__ __forceinline__ void tail_restrict(const LevelDev &F, const T *rf, const LevelDev &Cl, T *bc, T *xc) {
+__device__ __forceinline__ void tail_restrict(const LevelDev &F, const T *rf, const LevelDev &Cl, T *bc) {
     const T wt[4] = {T(0.25), T(0.75), T(0.75), T(0.25)};
-    const int n = Cl.nx * Cl.ny * Cl.nz;
-    const int rl = F.split ? F.nx >> 1 : F.nx, hs = F.split ? F.half : 0;
+    const int n = Cl.nx * Cl.ny * Cl.nz, rl = F.nx >> 1;
+    const bool px = F.bt[0] == IBMDEM_BC_PERIODIC;
     for (int q = threadIdx.x; q < n; q += TAIL_T) {
         int I, J, K;
         lcell_small(Cl, q, I, J, K);
-        // lidx(F, i, j, k) = ((i & 1) ^ ((j + k) & 1)) * half + row(j, k) + (i >> 1)
-        // when split, row(j, k) + i otherwise: its parts per tap coordinate
-        int xo[4], xp[4], ro[16], rp[16];
-        for (int a = 0; a < 4; ++a) {
-            const int fi = tile_coord(2 * I - 1 + a, F.nx, F.bt[0], F.bt[1]);
-            xo[a] = F.split ? fi >> 1 : fi;
-            xp[a] = fi & 1;
-        }
+        const bool lo = I == 0 && !px, hi = I == Cl.nx - 1 && !px;
+        // the row's pairs I - 1, I, I + 1 (wrapped; unused beyond other sides)
+        const int pm = I > 0 ? I - 1 : (px ? rl - 1 : 0), pp = I < rl - 1 ? I + 1 : (px ? 0 : I);
+        int fj[4];
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2) fj[c2] = tile_coord(2 * J - 1 + c2, F.ny, F.bt[2], F.bt[3]);
+        T s = T(0);
+#pragma unroll
         for (int c3 = 0; c3 < 4; ++c3) {
             const int fk = tile_coord(2 * K - 1 + c3, F.nz, F.bt[4], F.bt[5]);
+#pragma unroll
             for (int c2 = 0; c2 < 4; ++c2) {
-                const int fj = tile_coord(2 * J - 1 + c2, F.ny, F.bt[2], F.bt[3]);
-                ro[4 * c3 + c2] = (fk * F.ny + fj) * rl;
-                rp[4 * c3 + c2] = (fj + fk) & 1;
+                const T *row = rf + (fk * F.ny + fj[c2]) * rl;
+                s = restrict_row(s, wt[c3] * wt[c2], ((fj[c2] + fk) & 1) == 0, lo, hi,
+                                 [&](int d) { return row[d < 0 ? pm : (d > 0 ? pp : I)]; },
+                                 [&](int d) { return row[F.half + (d < 0 ? pm : (d > 0 ? pp : I))]; });
             }
         }
-        T s = T(0);
-        for (int c3 = 0; c3 < 4; ++c3)
-            for (int c2 = 0; c2 < 4; ++c2)
-                for (int c1 = 0; c1 < 4; ++c1) {
-                    T w = wt[c3] * wt[c2] * wt[c1];
-                    const int r = 4 * c3 + c2;
-                    s = s + w * rf[(xp[c1] ^ rp[r]) * hs + ro[r] + xo[c1]];
-                }
-        const T v = T(0.125) * s;
-        bc[q] = v;
-        // the coarse level's first sweep, as k_restrict does it with xc
-        if (xc) xc[q] = ((I + J + K) & 1) ? T(0) : (v + T(0)) * T(Cl.idiag[diag_index(Cl, I, J, K)]);
+        bc[q] = T(0.125) * s;
     }
     __syncthreads();
 }
 
+// the correction of the red cells (the black ones are swept next)
 template <typename T>
 __device__ __forceinline__ void tail_prolong(const LevelDev &F, T *xf, const LevelDev &Cl, const T *xc) {
     const T wt[2] = {T(0.75), T(0.25)};
-    const int n = F.nx * F.ny * F.nz;
-    const int rl = Cl.split ? Cl.nx >> 1 : Cl.nx, hs = Cl.split ? Cl.half : 0;
-    for (int q = threadIdx.x; q < n; q += TAIL_T) {
-        int i, j, k;
-        lcell_small(F, q, i, j, k);
+    const int rl = Cl.split ? Cl.nx >> 1 : Cl.nx, hs = Cl.split ? Cl.half : 0, fr = F.nx >> 1;
+    for (int q = threadIdx.x; q < F.half; q += TAIL_T) {
+        const int row = udiv_small(q, fr, F.m_row), k = udiv_small(row, F.ny, F.m_ny), j = row - k * F.ny;
+        const int i = 2 * (q - row * fr) + ((j + k) & 1);
         int pi[2], pj[2], pk[2];
         parents(i, Cl.nx, Cl.bt[0], Cl.bt[1], pi[0], pi[1]);
         parents(j, Cl.ny, Cl.bt[2], Cl.bt[3], pj[0], pj[1]);
         parents(k, Cl.nz, Cl.bt[4], Cl.bt[5], pk[0], pk[1]);
-        // lidx(Cl, .) by parts, as in tail_restrict
+        // lidx(Cl, i, j, k) = ((i & 1) ^ ((j + k) & 1)) * half + row(j, k) + (i >> 1)
+        // when split, row(j, k) + i otherwise: its parts per parent coordinate
         int xo[2], xp[2], ro[4], rp[4];
         for (int a = 0; a < 2; ++a) {
             xo[a] = Cl.split ? pi[a] >> 1 : pi[a];
@@ -1568,15 +880,13 @@ __device__ __forceinline__ void vcycle_tail_body(const Blk &kb, const LevelDev *
     auto R = [&](int l) { return B(l) + cells(l); };
     for (int q = kb.tx; q < cells(first); q += TAIL_T) B(first)[q] = bg[q];
     __syncthreads();
-    // below the first level, the restriction into a level also does its
-    // first sweep (the coarsest level sets its own x)
     for (int l = first; l < last; ++l) {
         for (int q = 0; q < pre; ++q) {
-            if (q > 0 || l == first) tail_half(LV(l), X(l), B(l), 0, q == 0);
+            tail_half(LV(l), X(l), B(l), 0, q == 0);
             tail_half(LV(l), X(l), B(l), 1, false);
         }
         tail_residual(LV(l), X(l), B(l), R(l));
-        tail_restrict(LV(l), R(l), LV(l + 1), B(l + 1), l + 1 < last ? X(l + 1) : (T *)nullptr);
+        tail_restrict(LV(l), R(l), LV(l + 1), B(l + 1));
     }
     if (kb.tx < 64) tail_coarse(LV(last), X(last), B(last), coarse_sweeps, s_nb, s_id, s_col);
     __syncthreads();
@@ -2063,17 +1373,54 @@ LevelDev make_level(int nx, int ny, int nz, const int bt[6], const double h[3]) 
     return L;
 }
 
-// one half sweep of a level, two-pair or one-pair threads as sweep_shape says
-template <typename T, bool DOT, int RES, bool ZI>
-void launch_half(const SweepShape &sw, hipStream_t s, const LevelDev &d, T *x, const T *b, int color,
-                 const double *stop, double *partial, long pofs, T *r, const double *r64 = nullptr,
-                 double *z64 = nullptr) {
-    if (sw.x2)
-        hipLaunchKernelGGL((k_rb_half<T, T, DOT, RES, ZI, true>), sw.grid, sw.block, 0, s, d, x, b, color, stop,
-                           partial, pofs, r, r64, z64);
+// pairs per thread of a level's passes: two where its rows hold an even number
+int march_pw(const LevelDev &d) { return (d.nx >> 1) % 2 == 0 ? 2 : 1; }
+
+// Levels of up to TILE_CELLS cells smooth in tiles (mgtile.hpp: two launches a
+// visit), larger ones in marching passes (mgmarch.hpp: six). In FP64 a visit's
+// launches take 18 us in tiles and 61 us in passes at 64^3, 66 and 63 us at
+// 64x64x256, 94 and 72 us at 128^3; the line lies where they meet, less the
+// gaps between four more launches. The mixed form's level 0 always marches
+// (its r.z sums, rz_half_body).
+constexpr long TILE_CELLS = 900000;
+template <typename T>
+bool tile_level(const LevelDev &d, int l, int pre, int post) {
+    return pre == 2 && post == 2 && (l > 0 || std::is_same<T, double>::value) &&
+           (long)d.nx * d.ny * d.nz <= TILE_CELLS;
+}
+template <typename T>
+bool tile_level(const ibmdem_ctx *c, int l) {
+    return tile_level<T>(c->lev64[l].d, l, c->cs.mg_pre, c->cs.mg_post);
+}
+
+template <typename T, int MODE, bool FROMB>
+void launch_march(hipStream_t s, const LevelDev &d, const T *xin, const T *b, T *out, T *out2, double *partial,
+                  const double *stop) {
+    const int pw = march_pw(d);
+    const MarchShape sh = march_shape<T>(d, pw);
+    const dim3 grid(8 * div_up(sh.ntx * sh.nty * sh.nzc, 8)), block(MT);
+    if (pw == 2)
+        hipLaunchKernelGGL((k_march<T, 2, MODE, FROMB>), grid, block, 0, s, d, xin, b, out, out2, partial, stop);
     else
-        hipLaunchKernelGGL((k_rb_half<T, T, DOT, RES, ZI>), sw.grid, sw.block, 0, s, d, x, b, color, stop, partial,
-                           pofs, r, r64, z64);
+        hipLaunchKernelGGL((k_march<T, 1, MODE, FROMB>), grid, block, 0, s, d, xin, b, out, out2, partial, stop);
+}
+
+// the mixed form's last two sweeps at level 0: x of the red cells in, the
+// black ones' x kept in x1
+void launch_rz(hipStream_t s, const LevelDev &d, const float *xr, float *x1, const double *r64, double *z64,
+               double *partial, const double *stop) {
+    const SweepShape sw = sweep_shape(d);
+    const long nb = (long)sw.grid.x * sw.grid.y * sw.grid.z;
+    for (int q = 0; q < 2; ++q) {   // black, red
+        const float *oth = q ? x1 : xr;
+        float *own = q ? nullptr : x1;
+        if (sw.x2)
+            hipLaunchKernelGGL(k_rz_half<2>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, z64, partial, q * nb,
+                               stop);
+        else
+            hipLaunchKernelGGL(k_rz_half<1>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, z64, partial, q * nb,
+                               stop);
+    }
 }
 
 template <typename T>
@@ -2092,90 +1439,108 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
         CHECK_LAUNCH(c);
         return IBMDEM_OK;
     }
-    // level-0 half-sweeps are the profiled (dominant) kernel: each reads the
-    // right-hand side and the other colour of half the cells and writes them;
-    // the residual variant also writes r of its half, the mixed form's r.z
-    // variant also reads the FP64 r and writes the FP64 z of its half
-    const double hb = l == 0 ? 1.5 * sizeof(T) * (double)L.n : 0.0;
-    const double hb_res = hb + (l == 0 ? 0.5 * sizeof(T) * (double)L.n : 0.0);
-    const double hb_dot = hb + (l == 0 && !std::is_same<T, double>::value ? 8.0 * (double)L.n : 0.0);
-    const SweepShape sw = sweep_shape(d);
-    const long nbh = (long)sw.grid.x * sw.grid.y * sw.grid.z;
-    // The pre- and the post-smoothing sweeps at level 0 are each timed as one
-    // group of back-to-back launches (one event pair per group).
-    double grp_bytes = 0.0;
-    int grp_n = 0;
-    auto group_begin = [&]() {
+    // Passes of two half sweeps (mgmarch.hpp) on the red half, out of place
+    // between the halves of x and r: the pre-smoothing passes in x, the
+    // residual in r's red half; the correction into r, the post-smoothing
+    // passes in r, the last one into x. At level 0 the pre- and the
+    // post-smoothing passes are each timed as one group of launches; a
+    // pass's bytes are its red input, b (of both colours) and what it writes
+    // (the mixed form's last pass: the FP64 r and z).
+    const double *stop = c->scal + SC_CONV;
+    T *x0 = L.x, *x1 = L.x + d.half, *r0 = L.r, *r1 = L.r + d.half, *cur = nullptr;
+    const double cell = sizeof(T) * (double)L.n;
+    double bytes = 0.0;
+    MGLevel<T> &C = lev[l + 1];
+    if (tile_level<T>(c, l)) {
+        // profiled at level 0: b read, the red cells' x written; b, x read,
+        // x written
         if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
-        grp_bytes = 0.0;
-        grp_n = 0;
-    };
-    auto group_end = [&]() {
-        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, grp_bytes, grp_n);
-    };
-    // res: 1 = the sweep also leaves the residual of its cells
-    auto half = [&](int color, int zero, int dot_slot = -1, int res = 0) {
-        ++grp_n;
-        if (dot_slot >= 0) {
-            // the mixed form reads the FP64 r and writes the FP64 z as well
-            const bool mixed = !std::is_same<T, double>::value;
-            launch_half<T, true, 0, false>(sw, s, d, L.x, L.b, color, c->scal + SC_CONV, c->partial,
-                                           dot_slot * nbh, (T *)nullptr, mixed ? c->cg_r : nullptr,
-                                           mixed ? c->cg_z : nullptr);
-            grp_bytes += hb_dot;
-            return;
-        }
-        if (res)
-            launch_half<T, false, 1, false>(sw, s, d, L.x, L.b, color, c->scal + SC_CONV, nullptr, 0L, L.r);
-        else if (zero)
-            launch_half<T, false, 0, true>(sw, s, d, L.x, L.b, color, c->scal + SC_CONV, nullptr, 0L, nullptr);
-        else
-            launch_half<T, false, 0, false>(sw, s, d, L.x, L.b, color, c->scal + SC_CONV, nullptr, 0L, nullptr);
-        grp_bytes += res ? hb_res : hb;
-    };
-    // pre-smoothing (red, black); the last black sweep also leaves r of the
-    // black cells, then r of the red cells
-    // below level 0 the restriction that wrote b also did the first sweep
-    group_begin();
+        hipLaunchKernelGGL((k_tile_down<T>), tile_grid(d), dim3(TileDown::NT), 0, s, d, L.b, r0, C.d, C.b, stop);
+        CHECK_LAUNCH(c);
+        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, 1.5 * cell, 1);
+        const int rc = vcycle<T>(c, lev, l + 1);
+        if (rc) return rc;
+        if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
+        hipLaunchKernelGGL((k_tile_up<T>), tile_grid(d), dim3(TileUp::NT), 0, s, d, L.b, r0, x0, C.d, C.x,
+                           dot && l == 0 ? c->partial : (double *)nullptr, stop);
+        CHECK_LAUNCH(c);
+        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, 2.5 * cell, 1);
+        return IBMDEM_OK;
+    }
+    if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
     for (int q = 0; q < c->cs.mg_pre; ++q) {
-        if (q > 0 || l == 0) half(0, q == 0 ? 1 : 0);
-        half(1, 0, -1, q == c->cs.mg_pre - 1 ? 1 : 0);
+        if (q == c->cs.mg_pre - 1) {
+            if (q == 0) {
+                launch_march<T, 1, true>(s, d, nullptr, L.b, r0, x0, nullptr, stop);
+                cur = x0;
+            } else {
+                launch_march<T, 1, false>(s, d, cur, L.b, r0, nullptr, nullptr, stop);
+            }
+            bytes += (RES_BLACK<T> ? 2.5 : 2.0) * cell;
+        } else {
+            T *to = cur == x0 ? x1 : x0;
+            if (q == 0) launch_march<T, 0, true>(s, d, nullptr, L.b, to, nullptr, nullptr, stop);
+            else launch_march<T, 0, false>(s, d, cur, L.b, to, nullptr, nullptr, stop);
+            bytes += (q == 0 ? 1.5 : 2.0) * cell;
+            cur = to;
+        }
         CHECK_LAUNCH(c);
     }
-    group_end();
-    launch_half<T, false, 2, false>(sw, s, d, L.x, L.b, 0, c->scal + SC_CONV, nullptr, 0L, L.r);
-    CHECK_LAUNCH(c);
-    MGLevel<T> &C = lev[l + 1];
+    if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, bytes, c->cs.mg_pre);
     const dim3 cs(div_up(C.d.nx, RS_CX), div_up(C.d.ny, RS_CY), C.d.nz);
-    // the coarse level's first sweep in the restriction when that level is
-    // swept by launches (not the work-group tail, not the coarsest)
-    const bool czero = l + 1 < c->tail_first && l + 1 != c->nlev - 1;
-    hipLaunchKernelGGL((k_restrict<T>), cs, dim3(RB), 0, s, d, L.r, C.d, C.b, czero ? C.x : (T *)nullptr,
-                       c->scal + SC_CONV);
+    hipLaunchKernelGGL((k_restrict<T>), cs, dim3(RB), 0, s, d, r0, C.d, C.b, stop);
     CHECK_LAUNCH(c);
     int rc = vcycle<T>(c, lev, l + 1);
     if (rc) return rc;
-    const ProlongShape ps = prolong_shape(d);
-    if (!ps.ok) {
-        return set_error(c, IBMDEM_ERR_ARG, "prolongation tile of " + std::to_string(ps.block.x) + "x" +
-                                                std::to_string(ps.block.y) + " threads does not fit");
-    }
-    if (ps.x2)
-        hipLaunchKernelGGL((k_prolong2<T>), ps.grid, ps.block, 0, s, d, L.x, C.d, C.x, c->scal + SC_CONV);
+    const LaunchShape ps = shape_for(d.nx / 2 / march_pw(d), d.ny, d.nz);
+    if (march_pw(d) == 2)
+        hipLaunchKernelGGL((k_prolong_red<T, 2>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
     else
-        hipLaunchKernelGGL((k_prolong<T>), ps.grid, ps.block, 0, s, d, L.x, C.d, C.x, c->scal + SC_CONV);
+        hipLaunchKernelGGL((k_prolong_red<T, 1>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
     CHECK_LAUNCH(c);
-    group_begin();
+    cur = r0;
+    bytes = 0.0;
+    if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
     for (int q = 0; q < c->cs.mg_post; ++q) {
-        // the last post sweep at level 0 finalizes z: with dot, it also
-        // leaves the partial sums of r.z (colour 1, then colour 0)
-        const bool last = dot && l == 0 && q == c->cs.mg_post - 1;
-        half(1, 0, last ? 0 : -1);
-        half(0, 0, last ? 1 : -1);
+        if (q < c->cs.mg_post - 1) {
+            T *to = cur == r0 ? r1 : r0;
+            launch_march<T, 0, false>(s, d, cur, L.b, to, nullptr, nullptr, stop);
+            bytes += 2.0 * cell;
+            cur = to;
+        } else if (dot && l == 0) {
+            // the last pass at level 0 finalizes z and leaves the partial
+            // sums of r.z (the mixed form reads the FP64 r and writes the
+            // FP64 z)
+            if constexpr (std::is_same<T, double>::value) {
+                launch_march<T, 2, false>(s, d, cur, L.b, x0, x1, c->partial, stop);
+                bytes += 2.5 * cell;
+            } else {
+                launch_rz(s, d, cur, x1, c->cg_r, c->cg_z, c->partial, stop);
+                bytes += 1.5 * cell + 16.0 * (double)L.n;
+            }
+        } else {
+            launch_march<T, 3, false>(s, d, cur, L.b, x0, x1, nullptr, stop);
+            bytes += 2.5 * cell;
+        }
         CHECK_LAUNCH(c);
     }
-    group_end();
+    if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, bytes, c->cs.mg_post);
     return IBMDEM_OK;
+}
+
+// partial sums of r.z the last level-0 launches leave
+int rz_blocks(const ibmdem_ctx *c) {
+    const LevelDev &d = c->lev64[0].d;
+    if (c->cs.precision == IBMDEM_MIXED) {
+        const dim3 g = sweep_shape(d).grid;
+        return 2 * (int)(g.x * g.y * g.z);
+    }
+    if (tile_level<double>(c, 0)) {
+        const dim3 g = tile_grid(d);
+        return (int)(g.x * g.y * g.z);
+    }
+    const MarchShape sh = march_shape<double>(d, march_pw(d));
+    return sh.ntx * sh.nty * sh.nzc;
 }
 
 int dot_into(ibmdem_ctx *c, const double *a, const double *b, int slot, int op);
@@ -2219,8 +1584,7 @@ int precondition_dot(ibmdem_ctx *c, int slot, int op) {
         rc = vcycle<double>(c, c->lev64, 0, true);
     }
     if (rc) return rc;
-    const dim3 g = sweep_shape(c->lev64[0].d).grid;   // the r.z sweeps' blocks
-    const int np = 2 * (int)(g.x * g.y * g.z);
+    const int np = rz_blocks(c);
     hipLaunchKernelGGL(k_final, dim3(1), dim3(FIN_T), 0, c->stream, c->partial, np, c->scal, slot, op, 0,
                        c->cs.poisson_rtol);
     CHECK_LAUNCH(c);
@@ -2244,12 +1608,24 @@ int read_scalars(ibmdem_ctx *c) {
 
 }  // namespace
 
-// partial sums the level-0 matrix-vector product (one per block) and the
-// last level-0 sweeps with r.z (one per block and colour) write
+// room for the partial sums of the level-0 matrix-vector product and of the
+// last level-0 launches with r.z, in any form
 long poisson_partials(int nx, int ny, int nz) {
     const LaunchShape mv = shape_for(div_up(nx, 2), ny, nz);
-    const dim3 h = half_grid(nx, ny, nz);
-    return std::max<long>((long)mv.grid.x * mv.grid.y * mv.grid.z, 2L * h.x * h.y * h.z);
+    long most = (long)mv.grid.x * mv.grid.y * mv.grid.z;
+    if (nx % 2 == 0) {
+        LevelDev d{};
+        d.nx = nx;
+        d.ny = ny;
+        d.nz = nz;
+        d.split = 1;
+        const dim3 sw = sweep_shape(d).grid, tl = tile_grid(d);
+        const MarchShape ma = march_shape<double>(d, march_pw(d));
+        most = std::max(most, 2L * sw.x * sw.y * sw.z);
+        most = std::max(most, (long)tl.x * tl.y * tl.z);
+        most = std::max(most, (long)ma.ntx * ma.nty * ma.nzc);
+    }
+    return most;
 }
 
 int poisson_setup(ibmdem_ctx *c) {
@@ -2478,23 +1854,65 @@ int poisson_solve(ibmdem_ctx *c, ibmdem_solve_info *info) {
 namespace {
 
 template <typename T>
-struct RbArg {
+struct MaArg {
     BGrid g;
     const LevelDev *L;
-    T *x;
-    const T *b;
-    const double *stop;
+    const T *xin, *b;
+    T *out, *out2;
     double *partial;
-    long pofs;
-    T *r;
-    const double *r64;
-    double *z64;
+    int nzp;   // planes of a chunk
+    const double *stop;
 };
-template <typename T, bool DOT, int RES, bool ZI, bool X2>
-__global__ __launch_bounds__(RB) void kb_rb_half(BTable<RbArg<T>> tab, int color) {
-    batch_for(tab, [&](const RbArg<T> &a, const Blk &kb) {
-        rb_half_body<T, T, DOT, RES, ZI, X2>(kb, *cst(a.L), glb(a.x), glb(a.b), color, glb(a.stop), glb(a.partial),
-                                             a.pofs, glb(a.r), glb(a.r64), glb(a.z64));
+template <typename T, int PW, int MODE, bool FROMB>
+__global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void kb_march(BTable<MaArg<T>> tab) {
+    batch_for(tab, [&](const MaArg<T> &a, const Blk &kb) {
+        march_body<T, PW, MODE, FROMB>(kb, *cst(a.L), glb(a.xin), glb(a.b), glb(a.out), glb(a.out2),
+                                       glb(a.partial), a.nzp, glb(a.stop));
+    });
+}
+
+struct RzArg {
+    BGrid g;
+    const LevelDev *L;
+    const float *oth;
+    float *own;
+    const double *r64;
+    double *z64, *partial;
+    long pofs;
+    const double *stop;
+};
+template <int PW>
+__global__ __launch_bounds__(RB) void kb_rz_half(BTable<RzArg> tab, int color) {
+    batch_for(tab, [&](const RzArg &a, const Blk &kb) {
+        rz_half_body<PW>(kb, *cst(a.L), glb(a.oth), color ? glb(a.own) : (float *)nullptr, color, glb(a.r64),
+                         glb(a.z64), glb(a.partial), a.pofs, glb(a.stop));
+    });
+}
+
+// a tile half of a level (down: b to the red cells' x and the coarse b; up:
+// from the coarse x to x)
+template <typename T>
+struct TlArg {
+    BGrid g;
+    const LevelDev *L, *C;
+    const T *b;
+    T *xr, *x;
+    T *bc;
+    const T *xc;
+    double *partial;
+    const double *stop;
+};
+template <typename T>
+__global__ __launch_bounds__(TileDown::NT) void kb_tile_down(BTable<TlArg<T>> tab) {
+    batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
+        tile_down_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xr), *cst(a.C), glb(a.bc), glb(a.stop));
+    });
+}
+template <typename T>
+__global__ __launch_bounds__(TileUp::NT) void kb_tile_up(BTable<TlArg<T>> tab) {
+    batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
+        tile_up_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xr), glb(a.x), *cst(a.C), glb(a.xc),
+                        a.partial ? glb(a.partial) : (double *)nullptr, glb(a.stop));
     });
 }
 
@@ -2503,14 +1921,13 @@ struct RsArg {
     BGrid g;
     const LevelDev *F, *C;
     const T *rf;
-    T *bc, *xc;   // xc: the coarse level's first sweep too (null: not)
+    T *bc;
     const double *stop;
 };
 template <typename T>
 __global__ __launch_bounds__(RB) void kb_restrict(BTable<RsArg<T>> tab) {
     batch_for(tab, [&](const RsArg<T> &a, const Blk &kb) {
-        restrict_body<T>(kb, *cst(a.F), glb(a.rf), *cst(a.C), glb(a.bc), a.xc ? glb(a.xc) : (T *)nullptr,
-                         glb(a.stop));
+        restrict_body<T>(kb, *cst(a.F), glb(a.rf), *cst(a.C), glb(a.bc), glb(a.stop));
     });
 }
 
@@ -2518,20 +1935,15 @@ template <typename T>
 struct PrArg {
     BGrid g;
     const LevelDev *F, *C;
-    T *xf;
+    const T *xin;
+    T *xout;
     const T *xc;
     const double *stop;
 };
-template <typename T>
+template <typename T, int PW>
 __global__ __launch_bounds__(RB) void kb_prolong(BTable<PrArg<T>> tab) {
     batch_for(tab, [&](const PrArg<T> &a, const Blk &kb) {
-        prolong_body<T>(kb, *cst(a.F), glb(a.xf), *cst(a.C), glb(a.xc), glb(a.stop));
-    });
-}
-template <typename T>
-__global__ __launch_bounds__(RB) void kb_prolong2(BTable<PrArg<T>> tab) {
-    batch_for(tab, [&](const PrArg<T> &a, const Blk &kb) {
-        prolong2_body<T>(kb, *cst(a.F), glb(a.xf), *cst(a.C), glb(a.xc), glb(a.stop));
+        prolong_red_body<T, PW>(kb, *cst(a.F), glb(a.xin), glb(a.xout), *cst(a.C), glb(a.xc), glb(a.stop));
     });
 }
 
@@ -2634,22 +2046,29 @@ struct BProf {
     std::vector<double> bytes;
     int n = 0;                          // launches recorded
 };
-template <typename T, bool DOT, int RES, bool ZI, bool X2>
-void launch_rb(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL((kb_rb_half<T, DOT, RES, ZI, X2>), dim3(o.blocks), dim3(RB), 0, s, table<RbArg<T>>(o),
-                       o.color);
+template <typename T, int PW, int MODE, bool FROMB>
+void launch_ma(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL((kb_march<T, PW, MODE, FROMB>), dim3(o.blocks), dim3(MT), 0, s, table<MaArg<T>>(o));
+}
+template <int PW>
+void launch_rzb(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL(kb_rz_half<PW>, dim3(o.blocks), dim3(RB), 0, s, table<RzArg>(o), o.color);
+}
+template <typename T>
+void launch_down(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL(kb_tile_down<T>, dim3(o.blocks), dim3(TileDown::NT), 0, s, table<TlArg<T>>(o));
+}
+template <typename T>
+void launch_up(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL(kb_tile_up<T>, dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
 }
 template <typename T>
 void launch_restrict(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_restrict<T>, dim3(o.blocks), dim3(RB), 0, s, table<RsArg<T>>(o));
 }
-template <typename T>
+template <typename T, int PW>
 void launch_prolong(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_prolong<T>, dim3(o.blocks), dim3(RB), 0, s, table<PrArg<T>>(o));
-}
-template <typename T>
-void launch_prolong2(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_prolong2<T>, dim3(o.blocks), dim3(RB), 0, s, table<PrArg<T>>(o));
+    hipLaunchKernelGGL((kb_prolong<T, PW>), dim3(o.blocks), dim3(RB), 0, s, table<PrArg<T>>(o));
 }
 template <typename T>
 void launch_tail(const BOp &o, hipStream_t s, int) {
@@ -2707,55 +2126,115 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
     int depth = 0;
     for (ibmdem_ctx *c : cs) depth = std::max(depth, bottom_level(c));
     int rc;
-    // a half sweep of level l of every case whose V-cycle goes below l: one
-    // launch for the cases that sweep it with two-pair threads, one for the
-    // others (sweep_shape)
-    auto half = [&](int l, int color, int zero, int dot_slot, int res) {
-        std::vector<RbArg<T>> args[2];
+    // The cells that smooth on level l, over the cases. Below level 0 tiles or
+    // passes (the same values) are chosen by them, as for one level of that
+    // size: a batch fills the chip, and the tiles' halo then costs time.
+    // Level 0 takes each case's own form, whose r.z sums are the form's.
+    auto cells_at = [&](int l) {
+        double n = 0.0;
+        for (ibmdem_ctx *c : cs)
+            if (l < bottom_level(c)) n += (double)levels<T>(c)[l].n;
+        return n;
+    };
+    auto tiled = [&](const ibmdem_ctx *c, int l) {
+        return tile_level<T>(c, l) && (l == 0 || cells_at(l) <= (double)TILE_CELLS);
+    };
+    // The pass of level l (vcycle's, MODE and FROMB by mode and fromb) of every
+    // case whose V-cycle goes below l: one launch for the cases with two-pair
+    // threads, one for the others. in and out: 0, 1 the halves of x, 2, 3 of r
+    auto pass = [&](int l, int mode, bool fromb, int in, int to, int to2) {
+        std::vector<MaArg<T>> args[2];
         BOp o[2];
-        // per cell of level 0: the half's b and the other colour read, the
-        // half's x written (the first sweep reads no x); the residual
-        // variants also read the half's own x or write its r; the mixed
-        // form's r.z variant also reads the FP64 r and writes the FP64 z
-        const double per = dot_slot >= 0 ? 1.5 * sizeof(T) + (mixed ? 8.0 : 0.0)
-                           : res          ? 2.0 * sizeof(T)
-                           : zero         ? 1.0 * sizeof(T)
-                                          : 1.5 * sizeof(T);
+        const double total = cells_at(l);
+        const double per = mode >= 2        ? 2.5 * sizeof(T)
+                           : mode == 0 && fromb ? 1.5 * sizeof(T)
+                           : mode == 1 && RES_BLACK<T> ? 2.5 * sizeof(T)
+                                                       : 2.0 * sizeof(T);
         for (ibmdem_ctx *c : cs) {
-            if (l >= bottom_level(c)) continue;
+            if (l >= bottom_level(c) || tiled(c, l)) continue;
             MGLevel<T> &L = levels<T>(c)[l];
-            const SweepShape sw = sweep_shape(L.d);
-            RbArg<T> a{};
-            a.g = bgrid(sw.grid, sw.block);
+            T *buf[4] = {L.x, L.x + L.d.half, L.r, L.r + L.d.half};
+            const int pw = march_pw(L.d);
+            const MarchShape sh = march_shape<T>(L.d, pw, mode == 2 ? 1.0 : (double)L.n / total);
+            MaArg<T> a{};
+            a.g = bgrid(dim3(sh.ntx, sh.nty, sh.nzc), dim3(MT));
             a.L = c->dlev + l;
-            a.x = L.x;
+            a.xin = in >= 0 ? buf[in] : nullptr;
             a.b = L.b;
+            a.out = buf[to];
+            a.out2 = to2 >= 0 ? buf[to2] : nullptr;
+            a.partial = mode == 2 ? c->partial : nullptr;
+            a.nzp = sh.nzp;
             a.stop = c->scal + SC_CONV;
-            a.partial = c->partial;
-            a.pofs = dot_slot >= 0 ? dot_slot * (long)sw.grid.x * sw.grid.y * sw.grid.z : 0;
-            a.r = res ? L.r : nullptr;
-            a.r64 = dot_slot >= 0 && mixed ? c->cg_r : nullptr;
-            a.z64 = dot_slot >= 0 && mixed ? c->cg_z : nullptr;
-            args[sw.x2].push_back(a);
-            if (l == 0) o[sw.x2].bytes += per * (double)c->n;
+            args[pw - 1].push_back(a);
+            if (l == 0) o[pw - 1].bytes += per * (double)c->n;
         }
-        for (int v = 0; v < 2; ++v) {
-            o[v].color = color;
+        const BLaunch fn[2][5] = {
+            {launch_ma<T, 1, 0, false>, launch_ma<T, 1, 0, true>, launch_ma<T, 1, 1, false>, launch_ma<T, 1, 1, true>,
+             mode == 2 ? launch_ma<double, 1, 2, false> : launch_ma<T, 1, 3, false>},
+            {launch_ma<T, 2, 0, false>, launch_ma<T, 2, 0, true>, launch_ma<T, 2, 1, false>, launch_ma<T, 2, 1, true>,
+             mode == 2 ? launch_ma<double, 2, 2, false> : launch_ma<T, 2, 3, false>}};
+        for (int v = 1; v >= 0; --v) {
             o[v].kind = l == 0 ? IBMDEM_BK_SMOOTH0 : IBMDEM_BK_SMOOTH;
+            const int r2 = add_op(ar, ops, fn[v][mode >= 2 ? 4 : 2 * mode + fromb], MT, args[v], o[v], err);
+            if (r2) return r2;
         }
-        const BLaunch fn[2] = {
-            dot_slot >= 0 ? launch_rb<T, true, 0, false, false>
-            : res == 2    ? launch_rb<T, false, 2, false, false>
-            : res == 1    ? launch_rb<T, false, 1, false, false>
-            : zero        ? launch_rb<T, false, 0, true, false>
-                          : launch_rb<T, false, 0, false, false>,
-            dot_slot >= 0 ? launch_rb<T, true, 0, false, true>
-            : res == 2    ? launch_rb<T, false, 2, false, true>
-            : res == 1    ? launch_rb<T, false, 1, false, true>
-            : zero        ? launch_rb<T, false, 0, true, true>
-                          : launch_rb<T, false, 0, false, true>};
-        int r2 = add_op(ar, ops, fn[1], RB, args[1], o[1], err);
-        return r2 ? r2 : add_op(ar, ops, fn[0], RB, args[0], o[0], err);
+        return (int)IBMDEM_OK;
+    };
+    // launch_rz of every case (the mixed form's last sweeps at level 0), the
+    // red cells' x in half `in` of r
+    auto rz = [&](int in) {
+        for (int q = 0; q < 2; ++q) {
+            std::vector<RzArg> args[2];
+            BOp o[2];
+            for (ibmdem_ctx *c : cs) {
+                MGLevel<float> &L = c->lev32[0];
+                const SweepShape sw = sweep_shape(L.d);
+                RzArg a{};
+                a.g = bgrid(sw.grid, sw.block);
+                a.L = c->dlev;
+                a.oth = q ? L.x + L.d.half : L.r + (in - 2) * (long)L.d.half;
+                a.own = L.x + L.d.half;
+                a.r64 = c->cg_r;
+                a.z64 = c->cg_z;
+                a.partial = c->partial;
+                a.pofs = q * (long)sw.grid.x * sw.grid.y * sw.grid.z;
+                a.stop = c->scal + SC_CONV;
+                args[sw.x2].push_back(a);
+                o[sw.x2].bytes += (q ? 10.0 : 12.0) * (double)c->n;
+            }
+            for (int v = 1; v >= 0; --v) {
+                o[v].color = 1 - q;
+                o[v].kind = IBMDEM_BK_SMOOTH0;
+                const int r2 = add_op(ar, ops, v ? launch_rzb<2> : launch_rzb<1>, RB, args[v], o[v], err);
+                if (r2) return r2;
+            }
+        }
+        return (int)IBMDEM_OK;
+    };
+    // the tile half of level l of every case that takes it
+    auto tile = [&](int l, bool up) {
+        std::vector<TlArg<T>> args;
+        BOp o;
+        o.kind = l == 0 ? IBMDEM_BK_SMOOTH0 : IBMDEM_BK_SMOOTH;
+        for (ibmdem_ctx *c : cs) {
+            if (l >= bottom_level(c) || !tiled(c, l)) continue;
+            MGLevel<T> &L = levels<T>(c)[l], &C = levels<T>(c)[l + 1];
+            TlArg<T> a{};
+            a.g = bgrid(tile_grid(L.d), dim3(256, (up ? TileUp::NT : TileDown::NT) / 256));
+            a.L = c->dlev + l;
+            a.C = c->dlev + l + 1;
+            a.b = L.b;
+            a.xr = L.r;
+            a.x = L.x;
+            a.bc = C.b;
+            a.xc = C.x;
+            a.partial = up && l == 0 ? c->partial : nullptr;
+            a.stop = c->scal + SC_CONV;
+            args.push_back(a);
+            if (l == 0) o.bytes += (up ? 2.5 : 1.5) * sizeof(T) * (double)c->n;
+        }
+        return add_op(ar, ops, up ? launch_up<T> : launch_down<T>, up ? TileUp::NT : TileDown::NT, args, o, err);
     };
     // the bottoms at level l
     auto bottoms = [&](int l) {
@@ -2819,17 +2298,26 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
                     return r;
         return IBMDEM_OK;
     };
+    int last_in = 0;   // the half of x the pre-smoothing leaves the red cells in
     for (int l = 0; l < depth; ++l) {
-        // below level 0 every case that sweeps level l had its first sweep
-        // done by the restriction into l
+        int cur = -1;
         for (int q = 0; q < pre; ++q) {
-            if ((q > 0 || l == 0) && (rc = half(l, 0, q == 0, -1, 0))) return rc;
-            if ((rc = half(l, 1, 0, -1, q == pre - 1 ? 1 : 0))) return rc;
+            const int to = cur == 0 ? 1 : 0;
+            if (q == pre - 1) {
+                if ((rc = pass(l, 1, q == 0, cur, 2, q == 0 ? 0 : -1))) return rc;
+                if (q == 0) cur = 0;
+            } else {
+                if ((rc = pass(l, 0, q == 0, cur, to, -1))) return rc;
+                cur = to;
+            }
         }
-        if ((rc = half(l, 0, 0, -1, 2))) return rc;
+        last_in = cur;
+        if ((rc = tile(l, false))) return rc;
         std::vector<RsArg<T>> rs;
+        BOp ors;
+        ors.kind = IBMDEM_BK_RESTRICT;
         for (ibmdem_ctx *c : cs) {
-            if (l >= bottom_level(c)) continue;
+            if (l >= bottom_level(c) || tiled(c, l)) continue;
             MGLevel<T> &F = levels<T>(c)[l], &C = levels<T>(c)[l + 1];
             RsArg<T> a{};
             a.g = bgrid(dim3(div_up(C.d.nx, RS_CX), div_up(C.d.ny, RS_CY), C.d.nz), dim3(RB));
@@ -2837,18 +2325,12 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             a.C = c->dlev + l + 1;
             a.rf = F.r;
             a.bc = C.b;
-            a.xc = l + 1 < bottom_level(c) ? C.x : nullptr;
             a.stop = c->scal + SC_CONV;
             rs.push_back(a);
+            // the residual read (in FP64 its red half), the coarse right-hand
+            // side written
+            ors.bytes += sizeof(T) * ((RES_BLACK<T> ? 1.0 : 0.5) * (double)F.n + (double)C.n);
         }
-        BOp ors;
-        ors.kind = IBMDEM_BK_RESTRICT;
-        // the fine residual read, the coarse right-hand side (and where the
-        // first coarse sweep is fused, the coarse x) written
-        for (ibmdem_ctx *c : cs)
-            if (l < bottom_level(c))
-                ors.bytes += sizeof(T) * (double)(levels<T>(c)[l].n + levels<T>(c)[l + 1].n *
-                                                  (l + 1 < bottom_level(c) ? 2 : 1));
         if ((rc = add_op(ar, ops, launch_restrict<T>, RB, rs, ors, err))) return rc;
         if ((rc = bottoms(l + 1))) return rc;
     }
@@ -2856,41 +2338,45 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         std::vector<PrArg<T>> pr[2];
         BOp opr[2];
         for (ibmdem_ctx *c : cs) {
-            if (l >= bottom_level(c)) continue;
+            if (l >= bottom_level(c) || tiled(c, l)) continue;
             MGLevel<T> &F = levels<T>(c)[l], &C = levels<T>(c)[l + 1];
-            const ProlongShape sh = prolong_shape(F.d);
-            if (!sh.ok) {
-                err = "prolongation tile does not fit";
-                return IBMDEM_ERR_ARG;
-            }
+            const int pw = march_pw(F.d);
+            const LaunchShape sh = shape_for(F.d.nx / 2 / pw, F.d.ny, F.d.nz);
             PrArg<T> a{};
             a.g = bgrid(sh.grid, sh.block);
             a.F = c->dlev + l;
             a.C = c->dlev + l + 1;
-            a.xf = F.x;
+            a.xin = F.x + last_in * (long)F.d.half;
+            a.xout = F.r;
             a.xc = C.x;
             a.stop = c->scal + SC_CONV;
-            pr[sh.x2].push_back(a);
-            // the coarse solution read, the fine one read and written
-            opr[sh.x2].bytes += sizeof(T) * (double)(2 * F.n + C.n);
+            pr[pw - 1].push_back(a);
+            // the coarse solution and the red cells read, the latter written
+            opr[pw - 1].bytes += sizeof(T) * (double)(F.n + C.n);
         }
         opr[0].kind = opr[1].kind = IBMDEM_BK_PROLONG;
-        if ((rc = add_op(ar, ops, launch_prolong2<T>, RB, pr[1], opr[1], err))) return rc;
-        if ((rc = add_op(ar, ops, launch_prolong<T>, RB, pr[0], opr[0], err))) return rc;
+        if ((rc = add_op(ar, ops, launch_prolong<T, 2>, RB, pr[1], opr[1], err))) return rc;
+        if ((rc = add_op(ar, ops, launch_prolong<T, 1>, RB, pr[0], opr[0], err))) return rc;
+        if ((rc = tile(l, true))) return rc;
+        int cur = 2;
         for (int q = 0; q < post; ++q) {
-            const bool last = l == 0 && q == post - 1;
-            if ((rc = half(l, 1, 0, last ? 0 : -1, 0))) return rc;
-            if ((rc = half(l, 0, 0, last ? 1 : -1, 0))) return rc;
+            const bool last = q == post - 1;
+            const int to = cur == 2 ? 3 : 2;
+            if (last && l == 0 && mixed) {
+                if ((rc = rz(cur))) return rc;
+                break;
+            }
+            if ((rc = pass(l, last ? (l == 0 ? 2 : 3) : 0, false, cur, last ? 0 : to, last ? 1 : -1))) return rc;
+            cur = to;
         }
     }
     std::vector<CgArg> fin;
     for (ibmdem_ctx *c : cs) {
-        const dim3 g = sweep_shape(c->lev64[0].d).grid;   // the r.z sweeps' blocks
         CgArg a{};
         a.g = bgrid(dim3(1), dim3(FIN_T));
         a.partial = c->partial;
         a.scal = c->scal;
-        a.np = 2 * (int)(g.x * g.y * g.z);
+        a.np = rz_blocks(c);
         a.rtol = c->cs.poisson_rtol;
         fin.push_back(a);
     }

@@ -52,3 +52,41 @@ def _close(a, b, tol):
 ])
 def test_coarsest_level_forms(gpu_lib, oracle_lib, n, bt):
     _close(_iterate(gpu_lib, n, bt), _iterate(oracle_lib, n, bt), 1e-12)
+
+
+# the fused passes and transfers of the levels above the coarsest: one and two
+# pairs per thread, whole and tiled rows, partial tiles and chunks in every
+# dimension, levels smaller than a tile's halo, every side type
+@pytest.mark.parametrize("n,bt", [
+    ((4, 4, 4), [W] * 6),
+    ((6, 4, 10), [P, P, P, P, W, W]),
+    ((12, 20, 4), [W, W, P, P, P, P]),
+    ((26, 14, 22), [P] * 6),
+    ((62, 4, 8), [W] * 6),
+    ((34, 58, 18), [W, W, W, W, I, O]),
+    ((8, 130, 40), [P, P, W, W, P, P]),
+    ((260, 28, 16), [P] * 6),
+    ((264, 12, 20), [W] * 6),
+    ((130, 44, 12), [I, O, P, P, W, W]),
+    ((386, 8, 6), [P, P, W, W, W, W]),
+    ((520, 30, 8), [I, O, W, W, P, P]),
+    ((24, 40, 152), [W, W, I, O, P, P]),
+])
+def test_fused_passes(gpu_lib, oracle_lib, n, bt):
+    _close(_iterate(gpu_lib, n, bt), _iterate(oracle_lib, n, bt), 1e-12)
+
+
+@pytest.mark.parametrize("pre,post", [(1, 1), (1, 3), (3, 1), (4, 2)])
+def test_smoothing_counts(gpu_lib, oracle_lib, pre, post):
+    """Passes that are both first and last, and the buffers of odd counts."""
+    n, bt = (40, 26, 36), [P, P, W, W, W, W]
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        case = cases.build_case(*n, bt, rtol=1e-30, max_iter=1, mg_pre=pre, mg_post=post)
+        rhs = np.random.default_rng(9).normal(size=n[::-1])
+        with Simulation(lib, case) as s:
+            s.upload_poisson_rhs(rhs)
+            with pytest.raises(IbmdemError):
+                s.poisson()
+            out.append(s.download_poisson()[0])
+    _close(out[0], out[1], 1e-12)
