@@ -25,7 +25,8 @@
 // Spreading is deterministic: no two wavefronts ever add to one value. One
 // wavefront owns a tile and keeps the tile's force (3 x 512 doubles) in LDS.
 // It stages its entry list in chunks (delta factors, fdrag*vol and the cell
-// of the marker or of its image) and takes the entries in list order: lane l
+// of the marker or of its image, the lanes whose cells lie in the tile) and
+// takes the entries in list order: lane l
 // adds the entry's contribution -(fdrag*vol)*w to cell l of the entry's
 // 4x4x4 support (when that cell is in the tile) with an LDS add. The 64
 // lanes of one entry add to 64 different cells, and the LDS applies a
@@ -667,14 +668,18 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// one lane's input for one staged entry. The packed entry id is kept raw
-// until its records are loaded (one pipeline stage later), so issuing the
-// load never waits for it.
+// One lane's input for one staged chunk: lane l < CAP the record of entry l,
+// and every lane its share of the chunk's factor rows: 16-byte pair lane + 64 r
+// of the CAP rows of 12, so that consecutive lanes read consecutive pairs. The
+// packed entry id is kept raw until its records are loaded (one pipeline
+// stage later), so issuing the load never waits for it.
+constexpr int FPL = CAP * 12 / 64;   // factor pairs per lane
+static_assert(CAP * 12 % 64 == 0, "factor rows shared evenly");
 struct EntryIn {
     double x0, x1, x2, f0, f1, f2;
-    double2 fw[12]; // the marker's delta factors (k_records)
+    double2 fw[FPL];
     int cell;       // the marker's cell (linear)
-    uint32_t en;    // marker << SBITS | image code
+    uint32_t en;    // marker << SBITS | image code (0 beyond the list)
     bool valid;     // the lane stages an entry
 };
 
@@ -686,8 +691,16 @@ __device__ __forceinline__ void load_entry_id(const SpreadArgs &a, int e, bool v
 // wavefront is valid: the register then cannot look pending at the summing
 // loop, which would otherwise wait for every load in flight before reusing
 // it. (The empty asm only reads the register; it emits no instruction.)
+// Rows of entries beyond the list are marker 0's and are not used.
 __device__ __forceinline__ void load_entry_rec(const SpreadArgs &a, EntryIn &in) {
+    const int lane = threadIdx.x;
     asm volatile("" ::"v"(in.en));
+#pragma unroll
+    for (int r = 0; r < FPL; ++r) {
+        const int q = lane + 64 * r, e = q / 12;
+        const uint32_t m = (uint32_t)__shfl((int)in.en, e, 64) >> SBITS;
+        in.fw[r] = reinterpret_cast<const double2 *>(a.fac)[12L * m + (q - 12 * e)];
+    }
     if (in.valid) {
         const long m = (long)(in.en >> SBITS);
         // each load has exactly the width of what is used: no dead
@@ -699,79 +712,107 @@ __device__ __forceinline__ void load_entry_rec(const SpreadArgs &a, EntryIn &in)
         in.x0 = r01.x; in.x1 = r01.y; in.x2 = r[2];
         in.cell = reinterpret_cast<const int *>(r + 3)[0];   // low word of the cell slot
         in.f0 = r45.x; in.f1 = r45.y; in.f2 = r[6];
-        const double2 *mf = reinterpret_cast<const double2 *>(a.fac + 24 * m);
-#pragma unroll
-        for (int q = 0; q < 12; ++q) in.fw[q] = mf[q];
     }
 }
 
-// What the summing loop needs of a staged entry that is the same for every
-// lane: the support's corner relative to the tile (packed, 5 bits per
-// dimension, biased by 8) and fdrag*vol. The staging lane keeps it in
-// registers and the loop reads it with readlane, so it costs no LDS
-// bandwidth.
-struct EntryUni {
-    int corner;
-    double f0, f1, f2;
-};
-
-// delta factors of the lane's entry into LDS row `lane`; its cell and
-// fdrag*vol into u
-template <bool P2>
-__device__ __forceinline__ void stage_entry(const SpreadArgs &a, const EntryIn &in, double2 (*s_w)[WST2],
-                                            int i0, int j0, int k0, EntryUni &u) {
-    const GridDev &g = a.g;
-    const int lane = threadIdx.x;
-    if (!in.valid) return;
-    const uint32_t code = in.en & ((1u << SBITS) - 1);
-    const double L3[3] = {g.L[0], g.L[1], g.L[2]};
-    const double dd[3] = {g.dx, g.dy, g.dz};
-    const double id3[3] = {1.0 / g.dx, 1.0 / g.dy, 1.0 / g.dz};
-    const double xm[3] = {in.x0, in.x1, in.x2};
-    const int cc[3] = {in.cell % g.nx + 1, (in.cell / g.nx) % g.ny + 1, in.cell / (g.nx * g.ny) + 1};
-    // with a power-of-two cell volume the 1/dV of every weight is an exact
-    // scaling, folded into fdrag*vol here once per entry (bitwise the same
-    // products as fv * (w * (1/dV)))
-    if (P2) {
-        u.f0 = in.f0 * a.idV; u.f1 = in.f1 * a.idV; u.f2 = in.f2 * a.idV;
-    } else {
-        u.f0 = in.f0; u.f1 = in.f1; u.f2 = in.f2;
-    }
-    int cim[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        const uint32_t c = (code >> (3 * d)) & 7u;
-        if (c == 0u) {
-            // the marker itself: its factors from k_records
-            cim[d] = cc[d];
-#pragma unroll
-            for (int o = 0; o < 4; ++o) s_w[lane][d * 4 + o] = in.fw[d * 4 + o];
-            continue;
-        }
-        double xp = xm[d];
-        if (c == 1u || c == 2u) xp = xp + (c == 1u ? -L3[d] : L3[d]);
-        else xp = 2.0 * (c == 3u ? 0.0 : L3[d]) - xp;
-        const int cimg = cell_of(xp, dd[d]);
-        cim[d] = cimg;
-        // the centre factor at offset +2 is always 0 (see k_records)
-        for (int o = 0; o < 4; ++o)
-            s_w[lane][d * 4 + o] = make_double2(wt_face<P2>(xp, cimg + o - 1, dd[d], id3[d]),
-                                                o < 3 ? wt_cent<P2>(xp, cimg + o - 1, dd[d], id3[d]) : 0.0);
-    }
-    // support cells cim - 1 .. cim + 2 reach the tile, so each corner offset
-    // lies in [-3, 7]; clamping to [-4, 8] changes nothing (such a support
-    // misses the tile either way) and keeps the packed fields in range
-    const int o3[3] = {i0, j0, k0};
-    u.corner = 0;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) u.corner |= (min(max(cim[d] - 1 - o3[d], -4), 8) + 8) << (5 * d);
-}
-
-// One wavefront per active tile (block b takes tile slot tile_slot(b)).
 // LDS position of tile cell (x, y, z): z planes 68 doubles apart, so the 32
 // lanes of a half-wavefront (support offsets 4 x 4 x 2) hit 32 different
 // 8-byte bank pairs
 constexpr int ACC_Z = TL * TL + 4, ACC_N = ACC_Z * TL;
+
+// What the summing loop needs of a staged entry that is the same for every
+// lane: fdrag*vol, the accumulator index of the support's corner (and its
+// tile cell, first iteration) and the lanes whose support cell lies in the
+// tile (none beyond the list). The staging lane keeps it in registers and the
+// loop reads it with readlane, so it costs no LDS bandwidth, and the lanes'
+// mask no arithmetic on every lane for every entry.
+struct EntryUni {
+    double f0, f1, f2;
+    int base, cell;
+    unsigned mlo, mhi;
+};
+
+// where the weights' 1/dV goes (stage_entry)
+enum { DV_POW2, DV_FOLD, DV_EACH };
+
+// the factor rows of the chunk into LDS; what is uniform of the lane's entry
+// into u. Image entries overwrite their rows' image dimensions.
+template <int DV>
+__device__ __forceinline__ void stage_entry(const SpreadArgs &a, const EntryIn &in, double2 (*s_w)[WST2],
+                                            int i0, int j0, int k0, EntryUni &u) {
+    const GridDev &g = a.g;
+    const int lane = threadIdx.x;
+#pragma unroll
+    for (int r = 0; r < FPL; ++r) {
+        const int q = lane + 64 * r, e = q / 12;
+        s_w[e][q - 12 * e] = in.fw[r];
+    }
+    u.mlo = u.mhi = 0u;
+    if (!in.valid) return;
+    const uint32_t code = in.en & ((1u << SBITS) - 1);
+    const double L3[3] = {g.L[0], g.L[1], g.L[2]};
+    const double dd[3] = {g.dx, g.dy, g.dz};
+    const double xm[3] = {in.x0, in.x1, in.x2};
+    int cim[3] = {in.cell % g.nx + 1, (in.cell / g.nx) % g.ny + 1, in.cell / (g.nx * g.ny) + 1};
+    // The 1/dV of every weight is folded into fdrag*vol here, once per entry:
+    // with a power-of-two cell volume an exact scaling (bitwise the same
+    // products as fv * (w * (1/dV))), else the same two roundings in another
+    // order, taken in FP64 contexts (the mixed form amplifies a last-bit
+    // change through its FP32 predictor and keeps the division of each weight)
+    if (DV == DV_POW2) {
+        u.f0 = in.f0 * a.idV; u.f1 = in.f1 * a.idV; u.f2 = in.f2 * a.idV;
+    } else if (DV == DV_FOLD) {
+        u.f0 = in.f0 / a.dV; u.f1 = in.f1 / a.dV; u.f2 = in.f2 / a.dV;
+    } else {
+        u.f0 = in.f0; u.f1 = in.f1; u.f2 = in.f2;
+    }
+    if (code != 0u) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint32_t c = (code >> (3 * d)) & 7u;
+            if (c == 0u) continue;   // the marker itself: its factors from k_records
+            double xp = xm[d];
+            if (c == 1u || c == 2u) xp = xp + (c == 1u ? -L3[d] : L3[d]);
+            else xp = 2.0 * (c == 3u ? 0.0 : L3[d]) - xp;
+            const int cimg = cell_of(xp, dd[d]);
+            const double id = 1.0 / dd[d];
+            constexpr bool P2 = DV == DV_POW2;
+            cim[d] = cimg;
+            // the centre factor at offset +2 is always 0 (see k_records)
+            for (int o = 0; o < 4; ++o)
+                s_w[lane][d * 4 + o] = make_double2(wt_face<P2>(xp, cimg + o - 1, dd[d], id),
+                                                    o < 3 ? wt_cent<P2>(xp, cimg + o - 1, dd[d], id) : 0.0);
+        }
+    }
+    // support cells cim - 1 .. cim + 2 reach the tile, so each corner offset
+    // lies in [-3, 7]; clamping to [-4, 8] changes nothing (such a support
+    // misses the tile either way)
+    const int o3[3] = {i0, j0, k0};
+    int b[3];
+    unsigned in4[3];   // which of the four offsets lie in the tile
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        b[d] = min(max(cim[d] - 1 - o3[d], -4), 8);
+        in4[d] = (0xfu << max(-b[d], 0)) & (0xfu >> max(b[d] - (TL - 4), 0)) & 0xfu;
+    }
+    u.base = b[0] + TL * b[1] + ACC_Z * b[2];
+    u.cell = b[0] + TL * (b[1] + TL * b[2]);
+    // lane (oa, ob, oc) = bit oa + 4 ob + 16 oc
+    unsigned xy = 0u;
+#pragma unroll
+    for (int o = 0; o < 4; ++o) xy |= (in4[1] >> o & 1u) ? in4[0] << (4 * o) : 0u;
+    u.mlo = ((in4[2] & 1u) ? xy : 0u) | ((in4[2] & 2u) ? xy << 16 : 0u);
+    u.mhi = ((in4[2] & 4u) ? xy : 0u) | ((in4[2] & 8u) ? xy << 16 : 0u);
+}
+
+// One wavefront per active tile (block b takes tile slot tile_slot(b)). At
+// 256^3 with 904,000 markers: 399 us a launch (434 us with each lane loading
+// an entry's whole factor row and testing every entry's support itself), of
+// which the staging takes ~40, the epilogue 70 and the summing loop 290; the
+// loop's LDS traffic alone, 48 bytes read and three adds per lane and entry,
+// is 52 of its 75 cycles an entry. Measured and slower: a wavefront per
+// component (530 us: the entries' scalar work three times), rows read one
+// group ahead (408 us).
 // s += v as one LDS add without return (ds_add_f64: round to nearest even,
 // the same result as s - p for v = -p). The LDS executes a wavefront's
 // operations in issue order, so successive adds to one cell land in program
@@ -840,7 +881,7 @@ __device__ __forceinline__ void tile_epilogue(const SpreadArgs &a, int slot, dou
     }
 }
 
-template <bool P2>
+template <int DV>
 __device__ __forceinline__ void spread_tiles_body(const Blk &kb, const SpreadArgs &a) {
     __shared__ double s_acc[3][ACC_N];         // the tile's force
     __shared__ unsigned s_touch[TC / 32];      // cells some entry reached
@@ -879,56 +920,56 @@ __device__ __forceinline__ void spread_tiles_body(const Blk &kb, const SpreadArg
     load_entry_id(a, elo + CAP + lane, lane < min(CAP, ehi - elo - CAP), nx);
     for (int e0 = elo; e0 < ehi; e0 += CAP) {
         const int ne = min(CAP, ehi - e0);
-        stage_entry<P2>(a, in, s_w, i0, j0, k0, uni);
+        stage_entry<DV>(a, in, s_w, i0, j0, k0, uni);
         wave_sync();
         in = nx;
         load_entry_rec(a, in);
         load_entry_id(a, e0 + 2 * CAP + lane, lane < min(CAP, ehi - e0 - 2 * CAP), nx);
         // SU entries at a time: their factor rows are read and their terms
         // formed first, then their adds are issued back to back in entry
-        // order (rows at or past ne hold stale data and are not added)
+        // order (entries at or past ne have an empty mask)
         for (int g0 = 0; g0 < ne; g0 += SU) {
             double t0[SU], t1[SU], t2[SU];
-            int qa[SU], qt[SU];
-            bool hit[SU];
+            int qa[SU];
+            unsigned long long hit[SU];
 #pragma unroll
             for (int u = 0; u < SU; ++u) {
                 const int e = g0 + u;
                 // the entry's uniform values from its staging lane (e is the
                 // same on every lane, so these are scalars)
-                const int cp = __builtin_amdgcn_readlane(uni.corner, e);
-                const int bx = (cp & 31) - 8, by = ((cp >> 5) & 31) - 8, bz = ((cp >> 10) & 31) - 8;
-                const int lx = bx + oa, ly = by + ob, lz = bz + oc;
-                hit[u] = e < ne && (unsigned)lx < (unsigned)TL && (unsigned)ly < (unsigned)TL &&
-                         (unsigned)lz < (unsigned)TL;
-                qa[u] = (bx + TL * by + ACC_Z * bz) + loff;
-                qt[u] = lx + TL * (ly + TL * lz);
+                hit[u] = ((unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)uni.mhi, e) << 32) |
+                         (unsigned)__builtin_amdgcn_readlane((int)uni.mlo, e);
+                qa[u] = __builtin_amdgcn_readlane(uni.base, e) + loff;
                 const double f0 = readlane_f64(uni.f0, e), f1 = readlane_f64(uni.f1, e),
                              f2 = readlane_f64(uni.f2, e);
                 const double2 wx = s_w[e][oa], wy = s_w[e][4 + ob], wz = s_w[e][8 + oc];
                 // (face, centre): u takes the x face, v the y face, w the z face
                 const double pu = wx.x * wy.y * wz.y, pv = wx.y * wy.x * wz.y, pw = wx.y * wy.y * wz.x;
-                const double wu = P2 ? pu : pu / a.dV, wv = P2 ? pv : pv / a.dV, ww = P2 ? pw : pw / a.dV;
+                const bool each = DV == DV_EACH;
+                const double wu = each ? pu / a.dV : pu, wv = each ? pv / a.dV : pv, ww = each ? pw / a.dV : pw;
                 t0[u] = f0 * wu;
                 t1[u] = f1 * wv;
                 t2[u] = f2 * ww;
             }
 #pragma unroll
             for (int u = 0; u < SU; ++u) {
-                if (!hit[u]) continue;
+                if (!__builtin_amdgcn_inverse_ballot_w64(hit[u])) continue;
                 lds_add(&s_acc[0][qa[u]], -t0[u]);
                 lds_add(&s_acc[1][qa[u]], -t1[u]);
                 lds_add(&s_acc[2][qa[u]], -t2[u]);
-                if (a.first) atomicOr(&s_touch[qt[u] >> 5], 1u << (qt[u] & 31));
+                if (a.first) {
+                    const int qt = __builtin_amdgcn_readlane(uni.cell, g0 + u) + oa + TL * (ob + TL * oc);
+                    atomicOr(&s_touch[qt >> 5], 1u << (qt & 31));
+                }
             }
         }
         wave_sync();   // the rows are rewritten by the next chunk
     }
     tile_epilogue(a, slot, s_acc, s_touch, i0, j0, k0);
 }
-template <bool P2>
+template <int DV>
 __global__ __launch_bounds__(64) void k_spread_tiles(SpreadArgs a) {
-    spread_tiles_body<P2>(hw_blk(), a);
+    spread_tiles_body<DV>(hw_blk(), a);
 }
 
 __global__ __launch_bounds__(64) void k_scatter_force(const int *__restrict__ meta, const int *__restrict__ tiles,
@@ -1000,6 +1041,10 @@ TileGeom tile_geom(const GridDev &g) { return TileGeom{div_up(g.nx, TL), div_up(
 // is an exact multiplication by the reciprocal
 bool pow2_grid(const ibmdem_ctx *c) {
     return is_pow2(c->g.dx) && is_pow2(c->g.dy) && is_pow2(c->g.dz) && is_pow2(c->dV);
+}
+
+int spread_dv(const ibmdem_ctx *c) {
+    return pow2_grid(c) ? DV_POW2 : c->cs.precision == IBMDEM_MIXED ? DV_EACH : DV_FOLD;
 }
 
 }  // namespace
@@ -1090,10 +1135,11 @@ int ibm_spread(ibmdem_ctx *c) {
     a.first = c->first_mdf ? 1 : 0;
     prof_begin(c, IBMDEM_K_SPREAD);
     const dim3 grid(c->act_grid);
-    if (pow2_grid(c))
-        hipLaunchKernelGGL((k_spread_tiles<true>), grid, dim3(64), 0, c->stream, a);
-    else
-        hipLaunchKernelGGL((k_spread_tiles<false>), grid, dim3(64), 0, c->stream, a);
+    switch (spread_dv(c)) {
+    case DV_POW2: hipLaunchKernelGGL((k_spread_tiles<DV_POW2>), grid, dim3(64), 0, c->stream, a); break;
+    case DV_FOLD: hipLaunchKernelGGL((k_spread_tiles<DV_FOLD>), grid, dim3(64), 0, c->stream, a); break;
+    default: hipLaunchKernelGGL((k_spread_tiles<DV_EACH>), grid, dim3(64), 0, c->stream, a);
+    }
     prof_end(c, IBMDEM_K_SPREAD, 0.0);
     CHECK_LAUNCH(c);
     if (c->prof.kernel == IBMDEM_K_SPREAD || c->prof.kernel == IBMDEM_K_INTERP) {
@@ -1270,7 +1316,7 @@ struct SpreadArg {
     SpreadArgs s;
 };
 // uniform argument: first (the step's first iteration)
-template <bool P2>
+template <int DV>
 __global__ __launch_bounds__(64) void kb_spread(BTable<SpreadArg> tab, int first) {
     batch_for(tab, [&](const SpreadArg &a, const Blk &kb) {
         SpreadArgs s = a.s;
@@ -1278,16 +1324,16 @@ __global__ __launch_bounds__(64) void kb_spread(BTable<SpreadArg> tab, int first
         s.rec = glb(s.rec); s.fac = glb(s.fac); s.fact = glb(s.fact); s.mask = glb(s.mask);
         s.u = glb(s.u); s.v = glb(s.v); s.w = glb(s.w);
         s.first = first;
-        spread_tiles_body<P2>(kb, s);
+        spread_tiles_body<DV>(kb, s);
     });
 }
 template <bool P2, bool OPEN>
 void launch_interp(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL((kb_interp<P2, OPEN>), dim3(o.blocks), dim3(T), 0, s, table<InterpArg>(o));
 }
-template <bool P2>
+template <int DV>
 void launch_spread(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_spread<P2>, dim3(o.blocks), dim3(64), 0, s, table<SpreadArg>(o), o.slot);
+    hipLaunchKernelGGL(kb_spread<DV>, dim3(o.blocks), dim3(64), 0, s, table<SpreadArg>(o), o.slot);
 }
 
 SpreadArgs spread_args(ibmdem_ctx *c) {
@@ -1318,7 +1364,7 @@ SpreadArgs spread_args(ibmdem_ctx *c) {
 // with markers (all share n_mdf; each at its current velocity parity)
 int ibm_plan_mdf(bk::BatchPlan &P, const std::vector<ibmdem_ctx *> &cs, std::string &err) {
     std::vector<InterpArg> ia[4];   // by (pow2, open)
-    std::vector<SpreadArg> sa[2];   // by pow2
+    std::vector<SpreadArg> sa[3];   // by spread_dv
     for (ibmdem_ctx *c : cs) {
         if (c->M == 0) continue;
         const int cur = c->vcur;
@@ -1340,11 +1386,11 @@ int ibm_plan_mdf(bk::BatchPlan &P, const std::vector<ibmdem_ctx *> &cs, std::str
         SpreadArg b{};
         b.g = bgrid(dim3(c->act_grid), dim3(64));
         b.s = spread_args(c);
-        sa[p2 ? 1 : 0].push_back(b);
+        sa[spread_dv(c)].push_back(b);
     }
     const BLaunch fi[4] = {launch_interp<false, false>, launch_interp<false, true>, launch_interp<true, false>,
                            launch_interp<true, true>};
-    const BLaunch fs[2] = {launch_spread<false>, launch_spread<true>};
+    const BLaunch fs[3] = {launch_spread<DV_POW2>, launch_spread<DV_FOLD>, launch_spread<DV_EACH>};
     const int n_mdf = cs.empty() ? 0 : cs[0]->cs.n_mdf;
     int rc;
     for (int it = 0; it < n_mdf; ++it) {
@@ -1352,7 +1398,7 @@ int ibm_plan_mdf(bk::BatchPlan &P, const std::vector<ibmdem_ctx *> &cs, std::str
             if ((rc = add_op(P.ar, P.ops, fi[v], T, ia[v], BOp(), err, true))) return rc;
         BOp o;
         o.slot = it == 0 ? 1 : 0;   // first
-        for (int v = 0; v < 2; ++v)
+        for (int v = 0; v < 3; ++v)
             if ((rc = add_op(P.ar, P.ops, fs[v], 64, sa[v], o, err, true))) return rc;
     }
     return IBMDEM_OK;
