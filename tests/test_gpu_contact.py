@@ -1,0 +1,33 @@
+"""The contact scan's two forms (32 lanes a marker, one thread a marker) against
+the oracle bit for bit: few and many scanning markers per block, more
+candidates in a row of cells or in all than the first form holds, rows that
+wrap in x, walls."""
+import numpy as np
+import pytest
+
+from ibmdem import cases
+from ibmdem.abi import BC_PERIODIC, BC_WALL, Simulation
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("markers", [40, 201, 900, 4000])
+@pytest.mark.parametrize("walls", [False, True])
+def test_contact_scan_forms(gpu_lib, oracle_lib, markers, walls):
+    n = (24, 20, 22)
+    case = cases.build_case(*n, [BC_WALL if walls else BC_PERIODIC] * 6, visc=0.05, kn_coeff=1e5, restitution=0.9,
+                            u_max=0.3, max_pairs=2000)
+    # shells overlap along x, also across the periodic face, and along z
+    cs = [(4.2, 9.8, 4.1), (12.1, 9.7, 4.4), (20.0, 9.9, 4.2), (12.3, 10.1, 12.0)]
+    mk, bd = cases.place_spheres(case, [cases.Sphere(c, 8.0, 2.0, markers) for c in cs])
+    rng = np.random.default_rng(4)
+    mk.v[:] = rng.normal(0.0, 0.02, size=mk.v.shape)
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        with Simulation(lib, case) as s:
+            s.upload_bodies(bd)
+            s.upload_markers(mk)
+            s.contact()
+            out.append(s.download_markers().fcol)
+    assert np.abs(out[1]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
