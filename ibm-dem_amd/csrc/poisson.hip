@@ -683,9 +683,13 @@ void launch_coarsest(hipStream_t s, const LevelDev &d, T *x, const T *b, T *tmp,
 // down to the coarsest, the whole V-cycle (smoothing, residual, restriction,
 // coarse sweeps, prolongation) runs in LDS with a barrier between phases, in
 // place of a few dozen launches that each cost more than their work. The
-// coarsest level sweeps on one wavefront from neighbour tables. Every cell's arithmetic is the multi-launch path's, so
-// the result is the same bit for bit; b of level `first` comes from global
-// memory and its x goes back there for the prolongation to the level above.
+// coarsest level sweeps on one wavefront from neighbour tables. Every cell's
+// arithmetic is the multi-launch path's, so the result is the same bit for
+// bit; b of level `first` comes from global memory and its x goes back there
+// for the prolongation to the level above. One CU's instruction issue bounds
+// the larger levels and a chain of LDS round trips the coarsest. With the
+// geometry in registers: levels 16^3, 8^3, 4^3, 2^3 in FP64 44 -> 31 us,
+// 16x12x20 down to 4x3x5 38 -> 27 us, FP32 43 -> 33 us.
 // ---------------------------------------------------------------------------
 constexpr int TAIL_T = 1024;
 constexpr int TAIL_BYTES = 112 * 1024;   // x (one extra zero slot on the coarsest level), b, r of the levels
@@ -695,48 +699,108 @@ static_assert(sizeof(LevelDev) % 4 == 0, "level descriptors copied by words");
 // divisions go through udiv_small)
 static_assert(TAIL_BYTES / 12 < (1 << 14), "tail levels small enough for udiv_small");
 
-// One half sweep of a level above the coarsest (split), by x-pairs. zero: x
-// is 0 before it, so the other colour takes part with 0 (a black sweep
-// follows, which reads red cells alone).
-template <typename T>
-__device__ __forceinline__ void tail_half(const LevelDev &L, T *x, const T *b, int color, bool zero) {
-    const int rl = L.nx >> 1;
-    T *own = x + color * L.half, *oth = x + (1 - color) * L.half;
-    for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
-        const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
-        const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
-        const int h = g.ca == color ? 0 : 1;
-        const T id = T(L.idiag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
-        const T bo = T(b[color * L.half + p]);
-        own[p] = zero ? (bo + T(0)) * id : (bo + nbsum_pair(oth, g, h, L)) * id;
-    }
-    __syncthreads();
-}
-
-// the residual after the last black sweep (in FP64 of the red cells alone, as
-// the passes of mgmarch.hpp); every level above the coarsest is split
-template <typename T>
-__device__ __forceinline__ void tail_residual(const LevelDev &L, const T *x, const T *b, T *r) {
-    const int rl = L.nx >> 1;
-    for (int p = threadIdx.x; p < L.half; p += TAIL_T) {
-        const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
-        const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
-        for (int c = 0; c < (RES_BLACK<T> ? 2 : 1); ++c) {
-            const int h = g.ca ^ c, own = c * L.half;   // the pair's cell of colour c
-            const T dg = T(L.diag[(h ? g.cx1 : g.cx0) * 16 + g.cyz]);
-            r[own + p] = T(b[own + p]) - (dg * x[own + p] - nbsum_pair(x + (1 - c) * L.half, g, h, L));
+// The x-pairs of a level above the coarsest (split) that one thread of NT
+// sweeps: pairs t, t + NT, .... Where a pair's neighbours stand and what its
+// cells are divided by is worked out once per visit and kept in registers, as
+// is b, so a half sweep is six LDS loads and the sum (index arithmetic and
+// table loads took two thirds of it). A missing neighbour is position `half`,
+// a zero word behind each colour's cells.
+template <typename T, int Q, int NT>
+struct TailPairs {
+    int o[Q][4], ox[Q][2];   // south, north, below, above; the other x neighbour of either colour's cell
+    int di[Q][2];
+    T id[Q][2], b[Q][2];
+    T ihx2, ihy2, ihz2;
+    const LevelDev &L;
+    __device__ __forceinline__ TailPairs(const LevelDev &lev, const T *bl) : L(lev) {
+        ihx2 = T(L.ihx2);
+        ihy2 = T(L.ihy2);
+        ihz2 = T(L.ihz2);
+        const int rl = L.nx >> 1, none = L.half;
+#pragma unroll
+        for (int u = 0; u < Q; ++u) {
+            const int p = threadIdx.x + u * NT;
+            if (p >= L.half) continue;
+            const int row = udiv_small(p, rl, L.m_row), kr = udiv_small(row, L.ny, L.m_ny);
+            const PairGeo g = pair_geo(L, p - row * rl, row - kr * L.ny, kr);
+            o[u][0] = g.hs ? p + g.ds : none;
+            o[u][1] = g.hn ? p + g.dn : none;
+            o[u][2] = g.hb ? p + g.db : none;
+            o[u][3] = g.ht ? p + g.dt : none;
+            const int w = g.hw ? p + g.dw : none, e = g.he ? p + g.de : none;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int h = g.ca ^ c;   // the pair's cell of colour c: even (0) or odd (1)
+                ox[u][c] = h ? e : w;
+                di[u][c] = (h ? g.cx1 : g.cx0) * 16 + g.cyz;
+                id[u][c] = T(L.idiag[di[u][c]]);
+                b[u][c] = bl[c * L.half + p];
+            }
         }
     }
-    __syncthreads();
+    // the black cells stand behind the red ones and their zero word
+    __device__ __forceinline__ int base(int c) const { return c ? L.half + 1 : 0; }
+    // nbsum_pair's value for the cell of colour c of pair u
+    __device__ __forceinline__ T nbsum(const T *x, int u, int c) const {
+        const T *oth = x + base(1 - c);
+        const T sx = (oth[threadIdx.x + u * NT] + oth[ox[u][c]]) * ihx2;
+        const T syy = (oth[o[u][0]] + oth[o[u][1]]) * ihy2;
+        const T szz = (oth[o[u][2]] + oth[o[u][3]]) * ihz2;
+        return sx + syy + szz;
+    }
+    template <typename F>
+    __device__ __forceinline__ void each(const F &f) const {
+#pragma unroll
+        for (int u = 0; u < Q; ++u)
+            if (threadIdx.x + u * NT < L.half) f(u, threadIdx.x + u * NT);
+    }
+    __device__ __forceinline__ void sync() const {
+        if (NT == 64) wave_barrier_lds();
+        else __syncthreads();
+    }
+    __device__ __forceinline__ void half_sweep(T *x, T (&own)[Q][2], int c) const {
+        each([&](int u, int p) {
+            own[u][c] = (b[u][c] + nbsum(x, u, c)) * id[u][c];
+            x[base(c) + p] = own[u][c];
+        });
+        sync();
+    }
+};
+
+// The way down through one level: the pre-smoothing from x = 0 (the first red
+// sweep reads no neighbour, the black one after it red cells alone) and the
+// residual after the last black sweep, in FP64 of the red cells alone as in
+// the passes of mgmarch.hpp.
+template <typename T, int Q, int NT>
+__device__ __forceinline__ void tail_down(const LevelDev &L, T *x, const T *bl, T *r, int pre) {
+    const TailPairs<T, Q, NT> P(L, bl);
+    T own[Q][2];
+    if (threadIdx.x < 2) x[P.base(threadIdx.x) + L.half] = T(0);
+    P.each([&](int u, int p) {
+        own[u][0] = (P.b[u][0] + T(0)) * P.id[u][0];
+        x[p] = own[u][0];
+    });
+    P.sync();
+    P.half_sweep(x, own, 1);
+    for (int q = 1; q < pre; ++q) {
+        P.half_sweep(x, own, 0);
+        P.half_sweep(x, own, 1);
+    }
+    P.each([&](int u, int p) {
+#pragma unroll
+        for (int c = 0; c < (RES_BLACK<T> ? 2 : 1); ++c)
+            r[c * L.half + p] = P.b[u][c] - (T(L.diag[P.di[u][c]]) * own[u][c] - P.nbsum(x, u, c));
+    });
+    P.sync();
 }
 
 // restrict_body's sum from the level's residual in LDS
-template <typename T>
+template <typename T, int NT>
 __device__ __forceinline__ void tail_restrict(const LevelDev &F, const T *rf, const LevelDev &Cl, T *bc) {
     const T wt[4] = {T(0.25), T(0.75), T(0.75), T(0.25)};
     const int n = Cl.nx * Cl.ny * Cl.nz, rl = F.nx >> 1;
     const bool px = F.bt[0] == IBMDEM_BC_PERIODIC;
-    for (int q = threadIdx.x; q < n; q += TAIL_T) {
+    for (int q = threadIdx.x; q < n; q += NT) {
         int I, J, K;
         lcell_small(Cl, q, I, J, K);
         const bool lo = I == 0 && !px, hi = I == Cl.nx - 1 && !px;
@@ -759,15 +823,21 @@ __device__ __forceinline__ void tail_restrict(const LevelDev &F, const T *rf, co
         }
         bc[q] = T(0.125) * s;
     }
-    __syncthreads();
+    if (NT == 64) wave_barrier_lds();
+    else __syncthreads();
 }
 
-// the correction of the red cells (the black ones are swept next)
-template <typename T>
-__device__ __forceinline__ void tail_prolong(const LevelDev &F, T *xf, const LevelDev &Cl, const T *xc) {
+// The way up: the correction of the red cells from the coarser level (hs:
+// words from its red to its black cells; the fine black cells are swept next)
+// and the post-smoothing. xg: the level's x in global memory, or null.
+template <typename T, int Q, int NT>
+__device__ __forceinline__ void tail_up(const LevelDev &F, T *xf, const T *bl, const LevelDev &Cl, const T *xc, int hs,
+                                        int post, T *xg) {
+    const TailPairs<T, Q, NT> P(F, bl);
     const T wt[2] = {T(0.75), T(0.25)};
-    const int rl = Cl.split ? Cl.nx >> 1 : Cl.nx, hs = Cl.split ? Cl.half : 0, fr = F.nx >> 1;
-    for (int q = threadIdx.x; q < F.half; q += TAIL_T) {
+    const int rl = Cl.split ? Cl.nx >> 1 : Cl.nx, fr = F.nx >> 1;
+    T own[Q][2];
+    P.each([&](int u, int q) {
         const int row = udiv_small(q, fr, F.m_row), k = udiv_small(row, F.ny, F.m_ny), j = row - k * F.ny;
         const int i = 2 * (q - row * fr) + ((j + k) & 1);
         int pi[2], pj[2], pk[2];
@@ -794,9 +864,20 @@ __device__ __forceinline__ void tail_prolong(const LevelDev &F, T *xf, const Lev
                     const int r = 2 * c3 + c2;
                     s = s + w * xc[(xp[c1] ^ rp[r]) * hs + ro[r] + xo[c1]];
                 }
-        xf[q] = xf[q] + s;
+        own[u][0] = xf[q] + s;
+        xf[q] = own[u][0];
+        own[u][1] = xf[P.base(1) + q];
+    });
+    P.sync();
+    for (int q = 0; q < post; ++q) {
+        P.half_sweep(xf, own, 1);
+        P.half_sweep(xf, own, 0);
     }
-    __syncthreads();
+    if (xg)
+        P.each([&](int u, int p) {
+            xg[p] = own[u][0];
+            xg[F.half + p] = own[u][1];
+        });
 }
 
 // The coarsest level (n <= COARSE_LDS cells, consistent red-black colouring)
@@ -850,7 +931,7 @@ __device__ __forceinline__ void vcycle_tail_body(const Blk &kb, const LevelDev *
                                                         int post, int coarse_sweeps,
                                                         const double *__restrict__ stop) {
     if (*stop != 0.0) return;
-    __shared__ T mem[TAIL_BYTES / sizeof(T)];
+    __shared__ T mem[TAIL_BYTES / sizeof(T) + 2 * TAIL_MAXLEV];
     __shared__ short s_nb[6][COARSE_LDS];
     __shared__ T s_id[COARSE_LDS];
     __shared__ unsigned char s_col[COARSE_LDS];
@@ -869,35 +950,44 @@ __device__ __forceinline__ void vcycle_tail_body(const Blk &kb, const LevelDev *
         int off = 0;
         for (int l = first; l <= last; ++l) {
             s_off[l] = off;
-            off += 3 * lev[l].nx * lev[l].ny * lev[l].nz + (l == last ? 1 : 0);
+            off += 3 * lev[l].nx * lev[l].ny * lev[l].nz + (l == last ? 1 : 2);
         }
     }
     __syncthreads();
+    constexpr int QM = (TAIL_BYTES / (3 * sizeof(T)) / 2 + TAIL_T - 1) / TAIL_T;   // pairs of the largest level
     auto LV = [&](int l) -> const LevelDev & { return s_lev[l - first]; };
     auto cells = [&](int l) { return LV(l).nx * LV(l).ny * LV(l).nz; };
     auto X = [&](int l) { return mem + s_off[l]; };
-    auto B = [&](int l) { return mem + s_off[l] + cells(l) + (l == last ? 1 : 0); };
+    auto B = [&](int l) { return mem + s_off[l] + cells(l) + (l == last ? 1 : 2); };
     auto R = [&](int l) { return B(l) + cells(l); };
-    for (int q = kb.tx; q < cells(first); q += TAIL_T) B(first)[q] = bg[q];
-    __syncthreads();
-    for (int l = first; l < last; ++l) {
-        for (int q = 0; q < pre; ++q) {
-            tail_half(LV(l), X(l), B(l), 0, q == 0);
-            tail_half(LV(l), X(l), B(l), 1, false);
-        }
-        tail_residual(LV(l), X(l), B(l), R(l));
-        tail_restrict(LV(l), R(l), LV(l + 1), B(l + 1));
+    auto HS = [&](int l) { return l == last ? LV(l).half : LV(l).half + 1; };   // red to black cells of x
+    // the levels from `wave` on have at most a pair per lane of one wavefront,
+    // which runs them without a work-group barrier
+    int wave = first;
+    while (wave < last && LV(wave).half > 64) ++wave;
+    for (int l = first; l < wave; ++l) {
+        const T *b = l == first ? bg : B(l);
+        if (LV(l).half > TAIL_T) tail_down<T, QM, TAIL_T>(LV(l), X(l), b, R(l), pre);
+        else tail_down<T, 1, TAIL_T>(LV(l), X(l), b, R(l), pre);
+        tail_restrict<T, TAIL_T>(LV(l), R(l), LV(l + 1), B(l + 1));
     }
-    if (kb.tx < 64) tail_coarse(LV(last), X(last), B(last), coarse_sweeps, s_nb, s_id, s_col);
-    __syncthreads();
-    for (int l = last - 1; l >= first; --l) {
-        tail_prolong(LV(l), X(l), LV(l + 1), X(l + 1));
-        for (int q = 0; q < post; ++q) {
-            tail_half(LV(l), X(l), B(l), 1, false);
-            tail_half(LV(l), X(l), B(l), 0, false);
+    if (kb.tx < 64) {
+        for (int l = wave; l < last; ++l) {
+            tail_down<T, 1, 64>(LV(l), X(l), l == first ? bg : B(l), R(l), pre);
+            tail_restrict<T, 64>(LV(l), R(l), LV(l + 1), B(l + 1));
         }
+        tail_coarse(LV(last), X(last), B(last), coarse_sweeps, s_nb, s_id, s_col);
+        for (int l = last - 1; l >= wave; --l)
+            tail_up<T, 1, 64>(LV(l), X(l), l == first ? bg : B(l), LV(l + 1), X(l + 1), HS(l + 1), post,
+                              l == first ? xg : nullptr);
     }
-    for (int q = kb.tx; q < cells(first); q += TAIL_T) xg[q] = X(first)[q];
+    __syncthreads();
+    for (int l = wave - 1; l >= first; --l) {
+        const T *b = l == first ? bg : B(l);
+        T *g = l == first ? xg : nullptr;
+        if (LV(l).half > TAIL_T) tail_up<T, QM, TAIL_T>(LV(l), X(l), b, LV(l + 1), X(l + 1), HS(l + 1), post, g);
+        else tail_up<T, 1, TAIL_T>(LV(l), X(l), b, LV(l + 1), X(l + 1), HS(l + 1), post, g);
+    }
 }
 template <typename T>
 __global__ __launch_bounds__(TAIL_T) void k_vcycle_tail(const LevelDev *__restrict__ lev, int first, int last,

@@ -90,3 +90,25 @@ def test_smoothing_counts(gpu_lib, oracle_lib, pre, post):
                 s.poisson()
             out.append(s.download_poisson()[0])
     _close(out[0], out[1], 1e-12)
+
+
+# the levels that one work-group runs: several pairs per thread, one, at most
+# a wavefront's, and hierarchies of those alone; the same operations as one
+# launch per operation, so equal bit for bit
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("n,bt", [
+    ((32, 24, 40), [W] * 6),
+    ((32, 32, 32), [P] * 6),
+    ((36, 34, 26), [P, P, W, W, I, O]),
+    ((48, 40, 36), [I, O, P, P, W, W]),
+    ((16, 12, 20), [W, W, P, P, W, W]),
+    ((8, 8, 16), [P, P, P, P, W, W]),
+    ((4, 12, 6), [P] * 6),
+])
+def test_small_levels_in_one_work_group(gpu_lib, monkeypatch, n, bt, precision):
+    out = []
+    for separate in ("1", "0"):
+        monkeypatch.setenv("IBMDEM_NO_TAIL", separate)
+        out.append(_iterate(gpu_lib, n, bt, precision))
+    assert np.abs(out[0]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
