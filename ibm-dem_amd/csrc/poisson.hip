@@ -443,58 +443,78 @@ __global__ __launch_bounds__(NT) void k_coarse_jac(LevelDev L, T *__restrict__ x
 // Tiles of CT_X x CT_Y x CT_Z cells, CT_H half sweeps (Jacobi: sweeps) s0 ..
 // s0 + ns - 1 from xin to xout (s0 = 0: from x = 0). The tile is loaded with a
 // halo of CT_H cells (wrapped across periodic sides, inactive zeros beyond
-// the others) and swept as a whole; the outermost layer is never updated, so
-// after s half sweeps the cells s layers in are exact, and the tile itself
-// is exact after CT_H. Halo cells are the neighbouring tiles' cells with
-// their own arithmetic, so the result does not depend on the tiling. At
-// 50x38x65 in FP64 a launch of four half sweeps takes 9.5 us on 180 blocks
-// (start, loads and stores ~7 us, ~0.6 us a half sweep), the solve 0.23 ms.
-constexpr int CT_X = 16, CT_Y = 8, CT_Z = 8, CT_H = 4, CT_T = 1024;
+// the others) and swept; after s half sweeps the cells s layers in are exact
+// (the planes further out are left alone), and the tile itself is exact after
+// CT_H. Halo cells are the neighbouring tiles' cells with their own
+// arithmetic, so the result does not depend on the tiling. Red-black launches
+// begin with a red sweep, which reads black cells alone: only those are
+// loaded, and only those are stored by all but the last launch (all_out).
+// A thread has CT_M pairs above each other, their values by colour in
+// registers: a neighbour in z is mostly a register, its plane's index
+// arithmetic the wavefront's, and LDS serves x and y. At 50x38x65 in FP64
+// (180 blocks): 7.3 us a launch of four half sweeps, the solve 0.18 ms; with
+// strided pairs and every neighbour from LDS 9.1 us, most of it index
+// arithmetic.
+constexpr int CT_X = 16, CT_Y = 8, CT_Z = 8, CT_H = 4, CT_M = 4;
 constexpr int CT_RL = (CT_X + 2 * CT_H) / 2, CT_EY = CT_Y + 2 * CT_H, CT_EZ = CT_Z + 2 * CT_H;
 constexpr int CT_NP = CT_RL * CT_EY * CT_EZ, CT_PL = CT_RL * CT_EY;   // x-pairs of a tile, of a plane
-constexpr int CT_M = CT_NP / CT_T;
-static_assert(CT_NP % CT_T == 0 && CT_X % 2 == 0 && CT_H % 2 == 0, "whole x-pairs and threads");
+constexpr int CT_T = CT_NP / CT_M;
+static_assert(CT_PL % 64 == 0 && CT_EZ % CT_M == 0 && CT_T <= 1024, "wavefronts within a plane");
+static_assert(CT_T % 256 == 0 && CT_X % 2 == 0 && CT_H % 2 == 0, "whole x-pairs, launches that begin with red");
 // the level's index of an unwrapped one, -1 beyond a side that is not periodic
 __device__ __forceinline__ int ct_map(int v, int n, int lo) {
     if (v >= 0 && v < n) return v;
     if (lo != IBMDEM_BC_PERIODIC) return -1;
-    v %= n;
-    return v < 0 ? v + n : v;
+    v += v < 0 ? n : -n;
+    if (v < 0 || v >= n) {   // levels smaller than the halo or the tile
+        v %= n;
+        v += v < 0 ? n : 0;
+    }
+    return v;
 }
 template <typename T, bool JAC>
 __device__ __forceinline__ void coarse_tile_body(const Blk &kb, const LevelDev &L, const T *__restrict__ xin,
                                                  T *__restrict__ xout, const T *__restrict__ bg, int s0, int ns,
-                                                 const double *__restrict__ stop) {
+                                                 bool all_out, const double *__restrict__ stop) {
     const double stopped = *stop;
     __shared__ T xs[2 * CT_NP];
     const int t = threadIdx.x;
+    const int seg = __builtin_amdgcn_readfirstlane(t / CT_PL), col = t - seg * CT_PL;
+    const int y = col / CT_RL, p = col - y * CT_RL, z0 = seg * CT_M, q0 = z0 * CT_PL + col;
     const int ox = kb.bx * CT_X - CT_H, oy = kb.by * CT_Y - CT_H, oz = kb.bz * CT_Z - CT_H;
     const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
-    int ca[CT_M];
-    bool upd[CT_M][2];
-    T bv[CT_M][2], id[CT_M][2], xv[CT_M][2];
-    const T id_int = T(L.idiag[DIAG_INTERIOR]);
+    const int ca0 = (oy + y + oz + z0) & 1;   // colour of the first pair's even cell (ox is even)
+    // cell (m, c): pair m's cell of colour c, even or odd as h(m, c) is 0 or 1
+    auto h = [&](int m, int c) { return (ca0 + m + c) & 1; };
+    T xv[CT_M][2], bv[CT_M][2], id[CT_M][2];
+    bool act[CT_M][2];
+    {
+        const int rl = L.split ? L.nx >> 1 : L.nx;
+        const int j = ct_map(oy + y, L.ny, L.bt[2]);
+        const int i0 = ct_map(ox + 2 * p, L.nx, L.bt[0]), i1 = ct_map(ox + 2 * p + 1, L.nx, L.bt[0]);
+        const int cy = 4 * diag_count(j, L.ny, L.bt[2], L.bt[3]);
+        const int cx0 = 16 * diag_count(i0, L.nx, L.bt[0], L.bt[1]), cx1 = 16 * diag_count(i1, L.nx, L.bt[0], L.bt[1]);
+        const T id_int = T(L.idiag[DIAG_INTERIOR]);
 #pragma unroll
-    for (int m = 0; m < CT_M; ++m) {
-        const int q = t + CT_T * m, z = q / CT_PL, y = (q - z * CT_PL) / CT_RL, p = q - z * CT_PL - y * CT_RL;
-        const int j = ct_map(oy + y, L.ny, L.bt[2]), k = ct_map(oz + z, L.nz, L.bt[4]);
-        ca[m] = (oy + y + oz + z) & 1;   // ox is even
-        const bool inner = y > 0 && y < CT_EY - 1 && z > 0 && z < CT_EZ - 1;
-        upd[m][0] = inner && p > 0;
-        upd[m][1] = inner && p < CT_RL - 1;
+        for (int m = 0; m < CT_M; ++m) {
+            const int k = ct_map(oz + z0 + m, L.nz, L.bt[4]);
+            const int cz = diag_count(k, L.nz, L.bt[4], L.bt[5]), row = (k * L.ny + j) * rl;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int i = ct_map(ox + 2 * p + e, L.nx, L.bt[0]);
-            const bool act = i >= 0 && j >= 0 && k >= 0;
-            const int g = act ? lidx(L, i, j, k) : 0;   // inactive cells load cell 0 and drop it
-            const int di = act ? diag_index(L, i, j, k) : DIAG_INTERIOR;
-            const T bl = bg[g], xl = s0 > 0 ? xin[g] : T(0);
-            T il = id_int;
-            if (di != DIAG_INTERIOR) il = T(L.idiag[di]);
-            bv[m][e] = act ? bl : T(0);
-            id[m][e] = act ? il : T(0);
-            xv[m][e] = act ? xl : T(0);
-            upd[m][e] = upd[m][e] && act;
+            for (int c = 0; c < 2; ++c) {
+                const int i = h(m, c) ? i1 : i0;
+                act[m][c] = i >= 0 && j >= 0 && k >= 0;
+                // lidx(L, i, j, k); inactive cells load cell 0 and drop it
+                int g = L.split ? (((i ^ j ^ k) & 1) ? L.half : 0) + row + (i >> 1) : row + i;
+                int d = (h(m, c) ? cx1 : cx0) + cy + cz;
+                g = act[m][c] ? g : 0;
+                d = act[m][c] ? d : DIAG_INTERIOR;
+                const T bl = bg[g], xl = s0 > 0 && (JAC || c == 1) ? xin[g] : T(0);
+                T il = id_int;
+                if (d != DIAG_INTERIOR) il = T(L.idiag[d]);
+                bv[m][c] = bl;
+                id[m][c] = il;
+                xv[m][c] = act[m][c] ? xl : T(0);
+            }
         }
     }
     // every load is in flight before the first is used
@@ -502,68 +522,83 @@ __device__ __forceinline__ void coarse_tile_body(const Blk &kb, const LevelDev &
 #pragma unroll
     for (int m = 0; m < CT_M; ++m)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) xs[((ca[m] + e) & 1) * CT_NP + t + CT_T * m] = xv[m][e];
+        for (int c = 0; c < 2; ++c) {
+            xs[c * CT_NP + q0 + m * CT_PL] = xv[m][c];
+            // the outermost layer in x and y is not updated
+            act[m][c] = act[m][c] && y > 0 && y < CT_EY - 1 && (h(m, c) ? p < CT_RL - 1 : p > 0);
+        }
     __syncthreads();
-    // nbsum of cell e of pair q from the other colour's half
-    auto nb = [&](const T *oth, int q, int e) {
-        const T xw = oth[e ? q : q - 1], xe = oth[e ? q + 1 : q];
-        const T sx = (xw + xe) * ihx2;
-        const T syy = (oth[q - CT_RL] + oth[q + CT_RL]) * ihy2;
-        const T szz = (oth[q - CT_PL] + oth[q + CT_PL]) * ihz2;
+    // nbsum of cell (m, c): its x neighbours are the pair's other cell and the
+    // same colour's cell of the pair beside
+    auto nb = [&](int m, int c) {
+        const T *oth = xs + (1 - c) * CT_NP + q0 + m * CT_PL;
+        const T sx = (xv[m][1 - c] + oth[h(m, c) ? 1 : -1]) * ihx2;
+        const T syy = (oth[-CT_RL] + oth[CT_RL]) * ihy2;
+        const T zb = m > 0 ? xv[m > 0 ? m - 1 : 0][1 - c] : oth[-CT_PL];
+        const T zt = m < CT_M - 1 ? xv[m < CT_M - 1 ? m + 1 : 0][1 - c] : oth[CT_PL];
+        const T szz = (zb + zt) * ihz2;
         return sx + syy + szz;
     };
-    for (int s = s0; s < s0 + ns; ++s) {
+    // planes s + 1 layers in and more take part in half sweep s
+    auto inner = [&](int m, int s) { return z0 + m > s && z0 + m < CT_EZ - 1 - s; };
+    for (int s = 0; s < ns; ++s) {
         if (JAC) {
             const T om = T(0.8);
             T nv[CT_M][2];
 #pragma unroll
             for (int m = 0; m < CT_M; ++m)
 #pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int q = t + CT_T * m, c = (ca[m] + e) & 1;
-                    const T x0 = xs[c * CT_NP + q];
-                    nv[m][e] = x0;
-                    if (upd[m][e]) {
-                        const T xn = (bv[m][e] + nb(xs + (1 - c) * CT_NP, q, e)) * id[m][e];
-                        nv[m][e] = x0 + om * (xn - x0);
+                for (int c = 0; c < 2; ++c) {
+                    nv[m][c] = xv[m][c];
+                    if (inner(m, s) && act[m][c]) {
+                        const T xn = (bv[m][c] + nb(m, c)) * id[m][c];
+                        nv[m][c] = xv[m][c] + om * (xn - xv[m][c]);
                     }
                 }
             __syncthreads();
 #pragma unroll
             for (int m = 0; m < CT_M; ++m)
 #pragma unroll
-                for (int e = 0; e < 2; ++e) xs[((ca[m] + e) & 1) * CT_NP + t + CT_T * m] = nv[m][e];
+                for (int c = 0; c < 2; ++c) {
+                    xv[m][c] = nv[m][c];
+                    xs[c * CT_NP + q0 + m * CT_PL] = nv[m][c];
+                }
+            __syncthreads();
         } else {
-            const int color = s & 1;
+            auto half = [&](int c) {
 #pragma unroll
-            for (int m = 0; m < CT_M; ++m) {
-                const int q = t + CT_T * m, e = ca[m] == color ? 0 : 1;
-                if (e ? upd[m][1] : upd[m][0])
-                    xs[color * CT_NP + q] = ((e ? bv[m][1] : bv[m][0]) + nb(xs + (1 - color) * CT_NP, q, e)) *
-                                            (e ? id[m][1] : id[m][0]);
-            }
+                for (int m = 0; m < CT_M; ++m)
+                    if (inner(m, s) && act[m][c]) {
+                        xv[m][c] = (bv[m][c] + nb(m, c)) * id[m][c];
+                        xs[c * CT_NP + q0 + m * CT_PL] = xv[m][c];
+                    }
+                __syncthreads();
+            };
+            half(0);
+            if (++s == ns) break;
+            half(1);
         }
-        __syncthreads();
     }
+    if (y < CT_H || y >= CT_Y + CT_H || p < CT_H / 2 || p >= (CT_X + CT_H) / 2) return;
+    const int j = oy + y;
+    if (j >= L.ny) return;
 #pragma unroll
     for (int m = 0; m < CT_M; ++m) {
-        const int q = t + CT_T * m, z = q / CT_PL, y = (q - z * CT_PL) / CT_RL, p = q - z * CT_PL - y * CT_RL;
-        if (p < CT_H / 2 || p >= (CT_X + CT_H) / 2 || y < CT_H || y >= CT_Y + CT_H || z < CT_H || z >= CT_Z + CT_H)
-            continue;
-        const int j = oy + y, k = oz + z;
-        if (j >= L.ny || k >= L.nz) continue;
+        const int z = z0 + m, k = oz + z;
+        if (z < CT_H || z >= CT_Z + CT_H || k >= L.nz) continue;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int i = ox + 2 * p + e;
-            if (i < L.nx) xout[lidx(L, i, j, k)] = xs[((ca[m] + e) & 1) * CT_NP + q];
+        for (int c = 0; c < 2; ++c) {
+            const int i = ox + 2 * p + h(m, c);
+            if (i < L.nx && (JAC || c == 1 || all_out)) xout[lidx(L, i, j, k)] = xv[m][c];
         }
     }
 }
 template <typename T, bool JAC>
-__global__ __launch_bounds__(CT_T) void k_coarse_tile(LevelDev L, const T *__restrict__ xin, T *__restrict__ xout,
-                                                      const T *__restrict__ bg, int s0, int ns,
+__global__ __launch_bounds__(CT_T) void k_coarse_tile(const LevelDev *__restrict__ lev,
+                                                      const T *__restrict__ xin, T *__restrict__ xout,
+                                                      const T *__restrict__ bg, int s0, int ns, bool all_out,
                                                       const double *__restrict__ stop) {
-    coarse_tile_body<T, JAC>(hw_blk(), L, xin, xout, bg, s0, ns, stop);
+    coarse_tile_body<T, JAC>(hw_blk(), *lev, xin, xout, bg, s0, ns, all_out, stop);
 }
 
 // Which form a coarsest level takes: one work-group where the level fits its
@@ -583,12 +618,12 @@ int coarse_threads(CoarseForm f) { return f == CF_WG256 ? 256 : f == CF_JAC512 ?
 // and reads what launch q - 1 wrote; the last one writes x (not tmp)
 struct CoarseTileStep {
     int s0, ns;
-    bool to_x;
+    bool to_x, all_out;
 };
 int coarse_tile_launches(bool jac, int sweeps) { return div_up(jac ? 2 * sweeps : 4 * sweeps - 1, CT_H); }
 CoarseTileStep coarse_tile_step(bool jac, int sweeps, int q) {
     const int total = jac ? 2 * sweeps : 4 * sweeps - 1, n = coarse_tile_launches(jac, sweeps);
-    return {q * CT_H, std::min(CT_H, total - q * CT_H), (n - 1 - q) % 2 == 0};
+    return {q * CT_H, std::min(CT_H, total - q * CT_H), (n - 1 - q) % 2 == 0, q == n - 1};
 }
 dim3 coarse_tile_grid(const LevelDev &d) { return dim3(div_up(d.nx, CT_X), div_up(d.ny, CT_Y), div_up(d.nz, CT_Z)); }
 
@@ -646,9 +681,10 @@ __device__ __forceinline__ bool coarse_sweeps_small(T *x, const T *b, const shor
     return true;
 }
 
-// the coarsest level's solve on the context's stream
+// the coarsest level's solve on the context's stream (dd: d on the device)
 template <typename T>
-void launch_coarsest(hipStream_t s, const LevelDev &d, T *x, const T *b, T *tmp, int sweeps, const double *stop) {
+void launch_coarsest(hipStream_t s, const LevelDev &d, const LevelDev *dd, T *x, const T *b, T *tmp, int sweeps,
+                     const double *stop) {
     const CoarseForm f = coarse_form(d);
     const dim3 one(1);
     switch (f) {
@@ -668,11 +704,11 @@ void launch_coarsest(hipStream_t s, const LevelDev &d, T *x, const T *b, T *tmp,
             const T *in = st.to_x ? tmp : x;
             T *out = st.to_x ? x : tmp;
             if (jac)
-                hipLaunchKernelGGL((k_coarse_tile<T, true>), coarse_tile_grid(d), dim3(CT_T), 0, s, d, in, out, b,
-                                   st.s0, st.ns, stop);
+                hipLaunchKernelGGL((k_coarse_tile<T, true>), coarse_tile_grid(d), dim3(CT_T), 0, s, dd, in, out, b,
+                                   st.s0, st.ns, st.all_out, stop);
             else
-                hipLaunchKernelGGL((k_coarse_tile<T, false>), coarse_tile_grid(d), dim3(CT_T), 0, s, d, in, out, b,
-                                   st.s0, st.ns, stop);
+                hipLaunchKernelGGL((k_coarse_tile<T, false>), coarse_tile_grid(d), dim3(CT_T), 0, s, dd, in, out, b,
+                                   st.s0, st.ns, st.all_out, stop);
         }
     }
     }
@@ -1525,7 +1561,7 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
         return IBMDEM_OK;
     }
     if (l == c->nlev - 1) {
-        launch_coarsest<T>(s, d, L.x, L.b, L.r, c->cs.mg_coarse_sweeps, c->scal + SC_CONV);
+        launch_coarsest<T>(s, d, c->dlev + l, L.x, L.b, L.r, c->cs.mg_coarse_sweeps, c->scal + SC_CONV);
         CHECK_LAUNCH(c);
         return IBMDEM_OK;
     }
@@ -2045,6 +2081,7 @@ struct BtArg {
     const LevelDev *lev;
     int first, last, pre, post, sweeps;
     int s0, ns;   // the tile form's half sweeps
+    bool all_out;
     T *x;
     const T *b;
     T *tmp;
@@ -2073,7 +2110,8 @@ __global__ __launch_bounds__(NT) void kb_coarse_wg(BTable<BtArg<T>> tab) {
 template <typename T, bool JAC>
 __global__ __launch_bounds__(CT_T) void kb_coarse_tile(BTable<BtArg<T>> tab) {
     batch_for(tab, [&](const BtArg<T> &a, const Blk &kb) {
-        coarse_tile_body<T, JAC>(kb, *cst(a.lev + a.last), glb(a.tmp), glb(a.x), glb(a.b), a.s0, a.ns, glb(a.stop));
+        coarse_tile_body<T, JAC>(kb, *cst(a.lev + a.last), glb(a.tmp), glb(a.x), glb(a.b), a.s0, a.ns, a.all_out,
+                                 glb(a.stop));
     });
 }
 
@@ -2360,11 +2398,12 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             const bool jac = f == CF_TILE_JAC;
             const int n = coarse_tile_launches(jac, a.sweeps);
             if ((int)tiles[jac].size() < n) tiles[jac].resize(n);
-            a.g = bgrid(coarse_tile_grid(L.d), dim3(CT_T));
+            a.g = bgrid(coarse_tile_grid(L.d), dim3(256, CT_T / 256));
             for (int q = 0; q < n; ++q) {
                 const CoarseTileStep st = coarse_tile_step(jac, a.sweeps, q);
                 a.s0 = st.s0;
                 a.ns = st.ns;
+                a.all_out = st.all_out;
                 a.x = st.to_x ? L.x : L.r;
                 a.tmp = st.to_x ? L.r : L.x;
                 tiles[jac][q].push_back(a);
