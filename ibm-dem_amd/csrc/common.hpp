@@ -358,6 +358,29 @@ struct LevelDev {
     unsigned m_row, m_ny, m_nxy;
 };
 
+// The sum of a block of NT threads (one value v each, t the thread's number)
+// in thread 0, in the order of the tree that adds element t + st to element t
+// for st = NT / 2 .. 1: the first wavefront takes the levels down to 64 from
+// LDS and the rest by shuffles, so one barrier serves in place of one a level.
+template <int NT>
+__device__ __forceinline__ double tree_sum(double v, int t, double *red) {
+    static_assert(NT >= 64 && (NT & (NT - 1)) == 0, "whole wavefronts, a full tree");
+    red[t] = v;
+    __syncthreads();
+    if (t >= 64) return 0.0;
+    double a[NT / 64];
+#pragma unroll
+    for (int w = 0; w < NT / 64; ++w) a[w] = red[t + 64 * w];
+#pragma unroll
+    for (int h = NT / 128; h > 0; h >>= 1)
+#pragma unroll
+        for (int w = 0; w < h; ++w) a[w] += a[w + h];
+    v = a[0];
+#pragma unroll
+    for (int st = 32; st > 0; st >>= 1) v += __shfl_down(v, st, 64);
+    return v;
+}
+
 // ceil(2^32 / d) (0 for d = 1): with it, udiv_small(p, d, m) = p / d exactly
 // for p * d < 2^32 (the error term p * (m d - 2^32) / 2^32 stays below p d /
 // 2^32 < 1 of the fractional part's room), in one multiply-high instead of

@@ -820,13 +820,8 @@ __device__ __forceinline__ void reduce_partial_body(const Blk &kb, const double 
     }
     for (; q < hi; q += RED_THREADS)
         if (q >= skip) s0 += term(q);
-    red[t] = (s0 + s1) + (s2 + s3);
-    __syncthreads();
-    for (int st = RED_THREADS / 2; st > 0; st >>= 1) {
-        if (t < st) red[t] += red[t + st];
-        __syncthreads();
-    }
-    if (t == 0) partial[kb.bx] = red[0];
+    const double sum = tree_sum<RED_THREADS>((s0 + s1) + (s2 + s3), t, red);
+    if (t == 0) partial[kb.bx] = sum;
 }
 __global__ __launch_bounds__(RED_THREADS) void k_reduce_partial(const double *__restrict__ a,
                                                                 const double *__restrict__ b, long n,
@@ -840,13 +835,8 @@ __device__ __forceinline__ void reduce_final_body(const Blk &kb, const double *_
     const int t = kb.tx;
     double s = 0.0;
     for (int q = t; q < np; q += RED_THREADS) s += partial[q];
-    red[t] = s;
-    __syncthreads();
-    for (int st = RED_THREADS / 2; st > 0; st >>= 1) {
-        if (t < st) red[t] += red[t + st];
-        __syncthreads();
-    }
-    if (t == 0) *out = red[0];
+    const double sum = tree_sum<RED_THREADS>(s, t, red);
+    if (t == 0) *out = sum;
 }
 __global__ __launch_bounds__(RED_THREADS) void k_reduce_final(const double *__restrict__ partial, int np,
                                                               double *__restrict__ out) {

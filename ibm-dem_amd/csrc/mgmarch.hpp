@@ -444,13 +444,8 @@ __device__ __forceinline__ void rz_half_body(const Blk &kb, const LevelDev &L, c
     }
     __shared__ double red[RB];
     const int t = kb.ty * kb.dx + kb.tx;
-    red[t] = dsum;
-    __syncthreads();
-    for (int st = RB / 2; st > 0; st >>= 1) {
-        if (t < st) red[t] += red[t + st];
-        __syncthreads();
-    }
-    if (t == 0) partial[pofs + ((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = red[0];
+    dsum = tree_sum<RB>(dsum, t, red);
+    if (t == 0) partial[pofs + ((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = dsum;
 }
 template <int PW>
 __global__ __launch_bounds__(RB) void k_rz_half(LevelDev L, const float *__restrict__ oth, float *__restrict__ own,

@@ -1036,16 +1036,6 @@ __global__ __launch_bounds__(TAIL_T) void k_vcycle_tail(const LevelDev *__restri
 // ---------------------------------------------------------------------------
 // CG kernels (FP64)
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double block_reduce(double s, double *red) {
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int st = RED_T / 2; st > 0; st >>= 1) {
-        if (threadIdx.x < st) red[threadIdx.x] += red[threadIdx.x + st];
-        __syncthreads();
-    }
-    return red[0];
-}
-
 // Ap = A p and one partial sum of p.Ap per block. A thread owns an x-pair
 // (both colours), a block 64 x 4 pairs of one plane: a block's plane
 // neighbours are read by the block
@@ -1129,14 +1119,9 @@ __device__ __forceinline__ void matvec_dot_body(const Blk &kb, const LevelDev &L
             }
         }
     }
-    const int nt = kb.dx * kb.dy, t = kb.ty * kb.dx + kb.tx;
-    red[t] = s;
-    __syncthreads();
-    for (int st = nt / 2; st > 0; st >>= 1) {
-        if (t < st) red[t] += red[t + st];
-        __syncthreads();
-    }
-    if (t == 0) partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = red[0];
+    const int t = kb.ty * kb.dx + kb.tx;
+    s = tree_sum<RB>(s, t, red);
+    if (t == 0) partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = s;
 }
 __global__ __launch_bounds__(RB) void k_matvec_dot(LevelDev L, const double *__restrict__ p,
                                                    double *__restrict__ Ap, double *__restrict__ partial,
@@ -1264,14 +1249,9 @@ __device__ __forceinline__ void matvec2_dot_body(const Blk &kb, const LevelDev &
             for (int c = 0; c < 2; ++c) s += v[r][hh][c] * a[hh][c];
         }
     }
-    const int nt = kb.dx * kb.dy, t = kb.ty * kb.dx + kb.tx;
-    red[t] = s;
-    __syncthreads();
-    for (int st = nt / 2; st > 0; st >>= 1) {
-        if (t < st) red[t] += red[t + st];
-        __syncthreads();
-    }
-    if (t == 0) partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = red[0];
+    const int t = kb.ty * kb.dx + kb.tx;
+    s = tree_sum<RB>(s, t, red);
+    if (t == 0) partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = s;
 }
 __global__ __launch_bounds__(RB) void k_matvec2_dot(LevelDev L, const double *__restrict__ p,
                                                     double *__restrict__ Ap, double *__restrict__ partial,
@@ -1302,19 +1282,28 @@ __global__ __launch_bounds__(RED_T) void k_cg_px(long n, double *__restrict__ p,
 __device__ __forceinline__ void cg_update_r_body(const Blk &kb, long n, double *__restrict__ r, const double *__restrict__ Ap,
                                                        const double *__restrict__ scal, double *__restrict__ partial,
                                                        float *__restrict__ r32) {
-    if (scal[SC_CONV] != 0.0) return;
     __shared__ double red[RED_T];
-    const double alpha = scal[SC_ALPHA];
+    const double conv = scal[SC_CONV], alpha = scal[SC_ALPHA];
     const long chunk = (n + kb.gx - 1) / kb.gx;
     const long lo = (long)kb.bx * chunk, hi = min(n, lo + chunk);
-    double s = 0.0;
-    for (long q = lo + kb.tx; q < hi; q += RED_T) {
-        double rq = r[q] - alpha * Ap[q];
+    double s = 0.0, ro = 0.0, ap = 0.0;
+    // a round's loads before the round ahead of it is stored, the first
+    // before the wait for the scalars
+    auto load = [&](long a) {
+        if (a < hi) { ro = r[a]; ap = Ap[a]; }
+    };
+    long q = lo + kb.tx;
+    load(q);
+    if (conv != 0.0) return;
+    while (q < hi) {
+        const double rq = ro - alpha * ap;
+        load(q + RED_T);
         r[q] = rq;
         if (r32) r32[q] = float(rq);
         s += rq * rq;
+        q += RED_T;
     }
-    double t = block_reduce(s, red);
+    const double t = tree_sum<RED_T>(s, kb.tx, red);
     if (kb.tx == 0) partial[kb.bx] = t;
 }
 __global__ __launch_bounds__(RED_T) void k_cg_update_r(long n, double *__restrict__ r, const double *__restrict__ Ap,
@@ -1343,7 +1332,7 @@ __device__ __forceinline__ void dot_body(const Blk &kb, long n, const double *__
         s3 += a[q + 3 * RED_T] * b[q + 3 * RED_T];
     }
     for (; q < hi; q += RED_T) s0 += a[q] * b[q];
-    double t = block_reduce((s0 + s1) + (s2 + s3), red);
+    const double t = tree_sum<RED_T>((s0 + s1) + (s2 + s3), kb.tx, red);
     if (kb.tx == 0) partial[kb.bx] = t;
 }
 __global__ __launch_bounds__(RED_T) void k_dot(long n, const double *__restrict__ a, const double *__restrict__ b,
@@ -1359,26 +1348,25 @@ __global__ __launch_bounds__(RED_T) void k_dot(long n, const double *__restrict_
 constexpr int FIN_T = 1024;
 __device__ __forceinline__ void final_body(const Blk &kb, const double *__restrict__ partial, int np, double *__restrict__ scal,
                                                  int slot, int op, int it, double rtol) {
-    if (scal[SC_CONV] != 0.0) return;
     __shared__ double red[FIN_T];
+    // one block, bound by its chain of latencies: the stop flag and the
+    // scalars are waited for with the partial sums (at 128^3 in FP64 the
+    // solve's three reductions an iteration take 1 to 1.5 % of a step less
+    // than with a wait of its own for the flag and a barrier per tree level)
+    const double conv = scal[SC_CONV], rz = scal[SC_RZ], tol = scal[SC_TOL];
     double a[4] = {0.0, 0.0, 0.0, 0.0};
     int q = kb.tx;
     for (; q + 3 * FIN_T < np; q += 4 * FIN_T)
         for (int u = 0; u < 4; ++u) a[u] += partial[q + u * FIN_T];
     for (int u = 0; q < np; q += FIN_T, ++u) a[u] += partial[q];
-    red[kb.tx] = (a[0] + a[1]) + (a[2] + a[3]);
-    __syncthreads();
-    for (int st = FIN_T / 2; st > 0; st >>= 1) {
-        if (kb.tx < st) red[kb.tx] += red[kb.tx + st];
-        __syncthreads();
-    }
-    const double t = red[0];
+    const double t = tree_sum<FIN_T>((a[0] + a[1]) + (a[2] + a[3]), kb.tx, red);
+    if (conv != 0.0) return;
     if (kb.tx == 0) {
         scal[slot] = t;
-        if (op == 1) scal[SC_ALPHA] = scal[SC_RZ] / t;
-        if (op == 2) { scal[SC_BETA] = t / scal[SC_RZ]; scal[SC_RZ] = t; }
+        if (op == 1) scal[SC_ALPHA] = rz / t;
+        if (op == 2) { scal[SC_BETA] = t / rz; scal[SC_RZ] = t; }
         if (op == 3) scal[SC_DONE] = it;
-        if (op == 3 && (sqrt(t) <= scal[SC_TOL] || !(t == t))) { scal[SC_CONV] = 1.0; scal[SC_ITER] = it; }
+        if (op == 3 && (sqrt(t) <= tol || !(t == t))) { scal[SC_CONV] = 1.0; scal[SC_ITER] = it; }
         if (op == 4) {
             scal[SC_TOL] = rtol * sqrt(t);
             if (t == 0.0) { scal[SC_CONV] = 1.0; scal[SC_ITER] = 0; scal[SC_RR] = 0.0; }
