@@ -370,16 +370,17 @@ __global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void k_march(LevelDev L
 }
 
 // The last black and red sweeps at level 0 of the mixed form, one launch each:
-// x of the other colour (FP32) in, the FP64 z = double(x) of the cells of
-// `color` out and (black) their x, with one partial sum of r.z per block over
-// its cells. Each thread has PW pairs of two adjacent rows. These two are not
+// x of the other colour in, the x of the cells of `color` out, with one partial
+// sum of r.z, z = double(x), per block over its cells. Each thread has PW pairs of two adjacent rows. These two are not
 // fused: their partial sums keep one association (this block shape, a tree
 // over its threads), since a change in the last bit of r.z reaches r's
 // conversion to FP32 and from there the solution at the solve's tolerance.
+// Bound by memory: 30 us a launch at 256^3 (35 us when an FP64 copy of z was
+// written as well).
 template <int PW>
 __device__ __forceinline__ void rz_half_body(const Blk &kb, const LevelDev &L, const float *__restrict__ oth,
                                              float *__restrict__ own, int color, const double *__restrict__ r64,
-                                             double *__restrict__ z64, double *__restrict__ partial, long pofs,
+                                             double *__restrict__ partial, long pofs,
                                              const double *__restrict__ stop) {
     const double stopped = *stop;   // waited for with the first loads
     const int rl = L.nx >> 1, pl = rl * L.ny;
@@ -424,7 +425,6 @@ __device__ __forceinline__ void rz_half_body(const Blk &kb, const LevelDev &L, c
         if (j >= L.ny || p0 >= rl) continue;
         const int cyz = diag_count(j, L.ny, L.bt[2], L.bt[3]) * 4 + cz;
         float x[PW];
-        double z[PW];
 #pragma unroll
         for (int c = 0; c < PW; ++c) {
             const bool outer = h[rr] ? c == PW - 1 : c == 0;
@@ -436,11 +436,9 @@ __device__ __forceinline__ void rz_half_body(const Blk &kb, const LevelDev &L, c
             float id = id_int;
             if (di != DIAG_INTERIOR) id = float(L.idiag[di]);
             x[c] = (float(r[rr][c]) + (sx + syy + szz)) * id;
-            z[c] = double(x[c]);
-            dsum += r[rr][c] * z[c];
+            dsum += r[rr][c] * double(x[c]);
         }
-        if (own) stp<float, PW>(own + pos[rr], x);
-        stp<double, PW>(z64 + (long)color * L.half + pos[rr], z);
+        stp<float, PW>(own + pos[rr], x);
     }
     __shared__ double red[RB];
     const int t = kb.ty * kb.dx + kb.tx;
@@ -449,10 +447,10 @@ __device__ __forceinline__ void rz_half_body(const Blk &kb, const LevelDev &L, c
 }
 template <int PW>
 __global__ __launch_bounds__(RB) void k_rz_half(LevelDev L, const float *__restrict__ oth, float *__restrict__ own,
-                                                int color, const double *__restrict__ r64, double *__restrict__ z64,
+                                                int color, const double *__restrict__ r64,
                                                 double *__restrict__ partial, long pofs,
                                                 const double *__restrict__ stop) {
-    rz_half_body<PW>(hw_blk(), L, oth, own, color, r64, z64, partial, pofs, stop);
+    rz_half_body<PW>(hw_blk(), L, oth, own, color, r64, partial, pofs, stop);
 }
 
 // b_c = (1/8) sum w r_f over the 4x4x4 fine cells of a coarse cell, w =

@@ -1261,17 +1261,21 @@ __global__ __launch_bounds__(RB) void k_matvec2_dot(LevelDev L, const double *__
 
 // CG iteration k >= 2, first kernel: p_k = z_k + beta_{k-1} p_{k-1} in place,
 // and the deferred x_k = x_{k-1} + alpha_{k-1} p_{k-1}
-__device__ __forceinline__ void cg_px_body(const Blk &kb, long n, double *__restrict__ p, const double *__restrict__ z,
-                                                 double *__restrict__ x, const double *__restrict__ scal) {
+// (z in the V-cycle's precision; bound by memory: 104 us at 256^3 in FP64,
+// 89 us with the mixed form's FP32 z read as it is)
+template <typename T>
+__device__ __forceinline__ void cg_px_body(const Blk &kb, long n, double *__restrict__ p, const T *__restrict__ z,
+                                           double *__restrict__ x, const double *__restrict__ scal) {
     if (scal[SC_CONV] != 0.0) return;
     const double beta = scal[SC_BETA], alpha = scal[SC_ALPHA];
     for (long q = (long)kb.bx * RED_T + kb.tx; q < n; q += (long)kb.gx * RED_T) {
         const double po = p[q];
-        p[q] = z[q] + beta * po;
+        p[q] = double(z[q]) + beta * po;
         x[q] = x[q] + alpha * po;
     }
 }
-__global__ __launch_bounds__(RED_T) void k_cg_px(long n, double *__restrict__ p, const double *__restrict__ z,
+template <typename T>
+__global__ __launch_bounds__(RED_T) void k_cg_px(long n, double *__restrict__ p, const T *__restrict__ z,
                                                  double *__restrict__ x, const double *__restrict__ scal) {
     cg_px_body(hw_blk(), n, p, z, x, scal);
 }
@@ -1413,10 +1417,12 @@ __global__ __launch_bounds__(RB) void k_cg_init(LevelDev L, const double *__rest
     cg_init_body(hw_blk(), L, rhs, r, x, scal, r32);
 }
 
-__device__ __forceinline__ void copy_body(const Blk &kb, long n, double *__restrict__ d, const double *__restrict__ s) {
+template <typename T>
+__device__ __forceinline__ void copy_body(const Blk &kb, long n, double *__restrict__ d, const T *__restrict__ s) {
     for (long q = (long)kb.bx * RED_T + kb.tx; q < n; q += (long)kb.gx * RED_T) d[q] = s[q];
 }
-__global__ __launch_bounds__(RED_T) void k_copy(long n, double *__restrict__ d, const double *__restrict__ s) {
+template <typename T>
+__global__ __launch_bounds__(RED_T) void k_copy(long n, double *__restrict__ d, const T *__restrict__ s) {
     copy_body(hw_blk(), n, d, s);
 }
 template <typename TD, typename TS>
@@ -1519,21 +1525,19 @@ void launch_march(hipStream_t s, const LevelDev &d, const T *xin, const T *b, T 
         hipLaunchKernelGGL((k_march<T, 1, MODE, FROMB>), grid, block, 0, s, d, xin, b, out, out2, partial, stop);
 }
 
-// the mixed form's last two sweeps at level 0: x of the red cells in, the
-// black ones' x kept in x1
-void launch_rz(hipStream_t s, const LevelDev &d, const float *xr, float *x1, const double *r64, double *z64,
+// the mixed form's last two sweeps at level 0: the red cells' x from xr, the
+// black ones' to x1 and the red ones' to x0
+void launch_rz(hipStream_t s, const LevelDev &d, const float *xr, float *x0, float *x1, const double *r64,
                double *partial, const double *stop) {
     const SweepShape sw = sweep_shape(d);
     const long nb = (long)sw.grid.x * sw.grid.y * sw.grid.z;
     for (int q = 0; q < 2; ++q) {   // black, red
         const float *oth = q ? x1 : xr;
-        float *own = q ? nullptr : x1;
+        float *own = q ? x0 : x1;
         if (sw.x2)
-            hipLaunchKernelGGL(k_rz_half<2>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, z64, partial, q * nb,
-                               stop);
+            hipLaunchKernelGGL(k_rz_half<2>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, partial, q * nb, stop);
         else
-            hipLaunchKernelGGL(k_rz_half<1>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, z64, partial, q * nb,
-                               stop);
+            hipLaunchKernelGGL(k_rz_half<1>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, partial, q * nb, stop);
     }
 }
 
@@ -1623,14 +1627,13 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
             cur = to;
         } else if (dot && l == 0) {
             // the last pass at level 0 finalizes z and leaves the partial
-            // sums of r.z (the mixed form reads the FP64 r and writes the
-            // FP64 z)
+            // sums of r.z (the mixed form reads the FP64 r)
             if constexpr (std::is_same<T, double>::value) {
                 launch_march<T, 2, false>(s, d, cur, L.b, x0, x1, c->partial, stop);
                 bytes += 2.5 * cell;
             } else {
-                launch_rz(s, d, cur, x1, c->cg_r, c->cg_z, c->partial, stop);
-                bytes += 1.5 * cell + 16.0 * (double)L.n;
+                launch_rz(s, d, cur, x0, x1, c->cg_r, c->partial, stop);
+                bytes += 2.0 * cell + 8.0 * (double)L.n;
             }
         } else {
             launch_march<T, 3, false>(s, d, cur, L.b, x0, x1, nullptr, stop);
@@ -1690,7 +1693,7 @@ int precondition_dot(ibmdem_ctx *c, int slot, int op) {
     int rc;
     if (c->cs.precision == IBMDEM_MIXED) {
         // the FP32 copy of r was written with r (k_cg_init, k_cg_update_r);
-        // the last level-0 sweeps write the FP64 z
+        // the last level-0 sweeps read the FP64 r
         rc = vcycle<float>(c, c->lev32, 0, true);
     } else {
         c->lev64[0].b = c->cg_r;
@@ -1812,8 +1815,12 @@ int cg_iteration(ibmdem_ctx *c, int it) {
     const SweepShape mv = sweep_shape(L0);   // two rows per thread, two pairs where the level allows
     const int mv_blocks = (int)(mv.grid.x * mv.grid.y * mv.grid.z);
     if (it > 1) {
-        hipLaunchKernelGGL(k_cg_px, dim3(stream_blocks(n)), dim3(RED_T), 0, s, n, c->cg_p, c->cg_z, c->cg_x,
-                           c->scal);
+        if (c->cs.precision == IBMDEM_MIXED)
+            hipLaunchKernelGGL(k_cg_px<float>, dim3(stream_blocks(n)), dim3(RED_T), 0, s, n, c->cg_p, c->lev32[0].x,
+                               c->cg_x, c->scal);
+        else
+            hipLaunchKernelGGL(k_cg_px<double>, dim3(stream_blocks(n)), dim3(RED_T), 0, s, n, c->cg_p, c->cg_z,
+                               c->cg_x, c->scal);
         CHECK_LAUNCH(c);
     }
     prof_begin(c, IBMDEM_K_MATVEC);
@@ -1860,7 +1867,12 @@ int poisson_begin_rhs(ibmdem_ctx *c) {
 int poisson_begin_precondition(ibmdem_ctx *c) {
     int rc;
     if ((rc = precondition_dot(c, SC_RZ, 0))) return rc;
-    hipLaunchKernelGGL(k_copy, dim3(stream_blocks(c->n)), dim3(RED_T), 0, c->stream, c->n, c->cg_p, c->cg_z);
+    if (c->cs.precision == IBMDEM_MIXED)
+        hipLaunchKernelGGL(k_copy<float>, dim3(stream_blocks(c->n)), dim3(RED_T), 0, c->stream, c->n, c->cg_p,
+                           c->lev32[0].x);
+    else
+        hipLaunchKernelGGL(k_copy<double>, dim3(stream_blocks(c->n)), dim3(RED_T), 0, c->stream, c->n, c->cg_p,
+                           c->cg_z);
     CHECK_LAUNCH(c);
     return IBMDEM_OK;
 }
@@ -1991,15 +2003,15 @@ struct RzArg {
     const float *oth;
     float *own;
     const double *r64;
-    double *z64, *partial;
+    double *partial;
     long pofs;
     const double *stop;
 };
 template <int PW>
 __global__ __launch_bounds__(RB) void kb_rz_half(BTable<RzArg> tab, int color) {
     batch_for(tab, [&](const RzArg &a, const Blk &kb) {
-        rz_half_body<PW>(kb, *cst(a.L), glb(a.oth), color ? glb(a.own) : (float *)nullptr, color, glb(a.r64),
-                         glb(a.z64), glb(a.partial), a.pofs, glb(a.stop));
+        rz_half_body<PW>(kb, *cst(a.L), glb(a.oth), glb(a.own), color, glb(a.r64), glb(a.partial), a.pofs,
+                         glb(a.stop));
     });
 }
 
@@ -2108,7 +2120,8 @@ struct CgArg {
     BGrid g;
     const LevelDev *L;
     long n;
-    double *p, *z, *x, *r, *Ap;
+    double *p, *x, *r, *Ap;
+    const void *z;   // FP32 in the mixed form
     double *partial;
     double *scal;
     float *r32;
@@ -2126,16 +2139,20 @@ __global__ __launch_bounds__(RB) void kb_matvec2_dot(BTable<CgArg> tab) {
         matvec2_dot_body(kb, *cst(a.L), glb(a.p), glb(a.Ap), glb(a.partial), glb(a.scal));
     });
 }
+template <typename T>
 __global__ __launch_bounds__(RED_T) void kb_cg_px(BTable<CgArg> tab) {
-    batch_for(tab, [&](const CgArg &a, const Blk &kb) { cg_px_body(kb, a.n, glb(a.p), glb(a.z), glb(a.x), glb(a.scal)); });
+    batch_for(tab, [&](const CgArg &a, const Blk &kb) {
+        cg_px_body(kb, a.n, glb(a.p), glb((const T *)a.z), glb(a.x), glb(a.scal));
+    });
 }
 __global__ __launch_bounds__(RED_T) void kb_cg_update_r(BTable<CgArg> tab) {
     batch_for(tab, [&](const CgArg &a, const Blk &kb) {
         cg_update_r_body(kb, a.n, glb(a.r), glb(a.Ap), glb(a.scal), glb(a.partial), glb(a.r32));
     });
 }
+template <typename T>
 __global__ __launch_bounds__(RED_T) void kb_copy(BTable<CgArg> tab) {
-    batch_for(tab, [&](const CgArg &a, const Blk &kb) { copy_body(kb, a.n, glb(a.p), glb(a.z)); });
+    batch_for(tab, [&](const CgArg &a, const Blk &kb) { copy_body(kb, a.n, glb(a.p), glb((const T *)a.z)); });
 }
 __global__ __launch_bounds__(FIN_T) void kb_final(BTable<CgArg> tab, int slot, int op, int it) {
     batch_for(tab, [&](const CgArg &a, const Blk &kb) {
@@ -2208,14 +2225,16 @@ void launch_matvec(const BOp &o, hipStream_t s, int) {
 void launch_matvec2(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_matvec2_dot, dim3(o.blocks), dim3(RB), 0, s, table<CgArg>(o));
 }
+template <typename T>
 void launch_px(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_cg_px, dim3(o.blocks), dim3(RED_T), 0, s, table<CgArg>(o));
+    hipLaunchKernelGGL(kb_cg_px<T>, dim3(o.blocks), dim3(RED_T), 0, s, table<CgArg>(o));
 }
 void launch_update_r(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_cg_update_r, dim3(o.blocks), dim3(RED_T), 0, s, table<CgArg>(o));
 }
+template <typename T>
 void launch_copy(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_copy, dim3(o.blocks), dim3(RED_T), 0, s, table<CgArg>(o));
+    hipLaunchKernelGGL(kb_copy<T>, dim3(o.blocks), dim3(RED_T), 0, s, table<CgArg>(o));
 }
 void launch_final(const BOp &o, hipStream_t s, int it) {
     hipLaunchKernelGGL(kb_final, dim3(o.blocks), dim3(FIN_T), 0, s, table<CgArg>(o), o.slot, o.op,
@@ -2310,14 +2329,13 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
                 a.g = bgrid(sw.grid, sw.block);
                 a.L = c->dlev;
                 a.oth = q ? L.x + L.d.half : L.r + (in - 2) * (long)L.d.half;
-                a.own = L.x + L.d.half;
+                a.own = L.x + (q ? 0 : L.d.half);
                 a.r64 = c->cg_r;
-                a.z64 = c->cg_z;
                 a.partial = c->partial;
                 a.pofs = q * (long)sw.grid.x * sw.grid.y * sw.grid.z;
                 a.stop = c->scal + SC_CONV;
                 args[sw.x2].push_back(a);
-                o[sw.x2].bytes += (q ? 10.0 : 12.0) * (double)c->n;
+                o[sw.x2].bytes += 8.0 * (double)c->n;
             }
             for (int v = 1; v >= 0; --v) {
                 o[v].color = 1 - q;
@@ -2510,7 +2528,8 @@ CgArg cg_arg(ibmdem_ctx *c, dim3 grid, dim3 block, int np) {
     a.g = bgrid(grid, block);
     a.L = c->dlev;
     a.n = c->n;
-    a.p = c->cg_p; a.z = c->cg_z; a.x = c->cg_x; a.r = c->cg_r; a.Ap = c->cg_Ap;
+    a.z = c->cs.precision == IBMDEM_MIXED ? (const void *)c->lev32[0].x : c->cg_z;
+    a.p = c->cg_p; a.x = c->cg_x; a.r = c->cg_r; a.Ap = c->cg_Ap;
     a.partial = c->partial;
     a.scal = c->scal;
     a.r32 = c->cs.precision == IBMDEM_MIXED ? c->lev32[0].b : nullptr;
@@ -2543,12 +2562,12 @@ int plan_all(Arena &ar, std::vector<BOp> &begin, std::vector<BOp> &iter, const s
     const bool mixed = !std::is_same<T, double>::value;
     BOp o;
     o.kind = IBMDEM_BK_VECTOR;
-    o.bytes = 16.0 * cells;   // z read, p written
-    if ((rc = add_op(ar, begin, launch_copy, RED_T, cp, o, err))) return rc;
+    o.bytes = (8.0 + sizeof(T)) * cells;   // z read, p written
+    if ((rc = add_op(ar, begin, launch_copy<T>, RED_T, cp, o, err))) return rc;
     // cg_iteration
     o.skip_first = true;
-    o.bytes = 40.0 * cells;   // p, x read and written, z read
-    if ((rc = add_op(ar, iter, launch_px, RED_T, px, o, err))) return rc;
+    o.bytes = (32.0 + sizeof(T)) * cells;   // p, x read and written, z read
+    if ((rc = add_op(ar, iter, launch_px<T>, RED_T, px, o, err))) return rc;
     o = BOp();
     o.kind = IBMDEM_BK_MATVEC;
     o.bytes = 16.0 * mv_cells[1];   // p read, Ap written
