@@ -31,3 +31,24 @@ def test_contact_scan_forms(gpu_lib, oracle_lib, markers, walls):
             out.append(s.download_markers().fcol)
     assert np.abs(out[1]).max() > 0
     np.testing.assert_array_equal(out[0], out[1])
+
+
+# the bodies in reach: fewer and more bodies than a block and than a chunk of
+# either length, several in reach at once and across a periodic side, and none
+@pytest.mark.parametrize("bodies", [2, 17, 65, 130, 4097, 4160])
+def test_bodies_in_reach(gpu_lib, oracle_lib, bodies):
+    n = (40, 36, 44)
+    case = cases.build_case(*n, [BC_PERIODIC] * 4 + [BC_WALL] * 2, visc=0.05, kn_coeff=1e5, restitution=0.9, u_max=0.3,
+                            max_pairs=500)
+    rng = np.random.default_rng(bodies)
+    cs = [tuple(c) for c in rng.uniform(1.5, np.array(n) - 1.5, (bodies, 3))]
+    mk, bd = cases.place_spheres(case, [cases.Sphere(c, 1.0, 2.0, 3) for c in cs])
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        with Simulation(lib, case) as s:
+            s.upload_bodies(bd)
+            s.upload_markers(mk)
+            s.contact()
+            out.append(s.download_markers().fcol)
+    assert bodies < 100 or np.abs(out[1]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
