@@ -25,7 +25,13 @@
 //   MODE 2  stage B relaxes and both colours are written, with the partial
 //           sums of r.z (last post-smoothing pass at level 0 in FP64: x is z,
 //           b is r); MODE 3 the same without the sums (other levels)
-// FROMB passes take their red input from b (first pre-smoothing pass).
+// FROMB passes take their red input from b (first pre-smoothing pass). PRO
+// passes (FP64, the first post-smoothing pass) add the coarse correction to
+// it as they load it: a thread interpolates each coarse plane in x and y once,
+// to either side of its pairs, and two of those planes in z per fine plane,
+// so the corrected red cells are neither written nor read again. (In FP32 the
+// prolongation keeps its launch and with it its order of summation, for the
+// reason above.)
 // A level then moves 1.5 + 2 + 2 + 2.5 of its cells per V-cycle (pre = post
 // = 2) where one launch per half sweep and one for the residual moved 14.5,
 // in 4 launches instead of 9. At 256^3 in FP64 the four take 41, 41, 42 and
@@ -102,10 +108,10 @@ __device__ __forceinline__ void stp(T *p, const T (&v)[PW]) {
     else p[0] = v[0];
 }
 
-template <typename T, int PW, int MODE, bool FROMB>
+template <typename T, int PW, int MODE, bool FROMB, bool PRO>
 __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, const T *__restrict__ xin,
                                            const T *__restrict__ b, T *__restrict__ out, T *__restrict__ out2,
-                                           double *__restrict__ partial, int nzp,
+                                           double *__restrict__ partial, int nzp, const T *__restrict__ xc,
                                            const double *__restrict__ stop) {
     const double stopped = *stop;   // waited for with the first loads
     __shared__ T s_r[2][MT * PW], s_b[2][MT * PW], s_id[64], s_dg[64];
@@ -235,10 +241,93 @@ __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, con
         if (inA) ldp<T, PW>(bb + pa, n.b);
         if (!FROMB && own) ldp<T, PW>(b + pb, n.q);
     };
+    // PRO: the coarse correction of the thread's red cells. The coarse level
+    // has half the cells per dimension; columns p - 1 .. p + PW of rows J[0]
+    // (the parent) and J[1] (the neighbour on the row's side), a missing one
+    // beyond a side the parent's (parents()). In an even plane the red cell of
+    // a pair lies to side A (east where j is odd), in an odd one to side B.
+    struct Coarse {
+        int nx, ny, nz, rl, half;
+        int ic[PW + 2], J[2];
+        T raw[2][PW + 2], a[PW], ap[PW], b[PW];   // interpolated: side A of planes K, K - 1, side B of K
+    } cg;
+    if constexpr (PRO) {
+        cg.nx = L.nx >> 1;
+        cg.ny = L.ny >> 1;
+        cg.nz = L.nz >> 1;
+        const bool split = (cg.nx & 1) == 0;
+        cg.rl = split ? cg.nx >> 1 : cg.nx;
+        cg.half = split ? cg.rl * cg.ny * cg.nz : 0;
+        for (int c = 0; c < PW + 2; ++c) {
+            const int i = p + c - 1;
+            cg.ic[c] = i < 0 ? (px ? i + cg.nx : 0) : (i < cg.nx ? i : (px ? i - cg.nx : cg.nx - 1));
+        }
+        cg.J[0] = jr >> 1;
+        const int jn = cg.J[0] + ((jr & 1) ? 1 : -1);
+        cg.J[1] = jn < 0 ? (py ? jn + cg.ny : 0) : (jn < cg.ny ? jn : (py ? jn - cg.ny : cg.ny - 1));
+    }
+    auto coarse_load = [&](int K, T (&raw)[2][PW + 2]) {
+        K = K < 0 ? (pz ? K + cg.nz : 0) : (K < cg.nz ? K : (pz ? K - cg.nz : cg.nz - 1));
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int o = (K * cg.ny + cg.J[q]) * cg.rl;
+            if constexpr (PW == 2) {
+                // p is even (and the coarse row split): columns p and p + 2 lie
+                // in one colour half, p - 1 and p + 1 in the other
+                const int h = ((cg.J[q] + K) & 1) ? cg.half : 0, even = o + h, odd = o + cg.half - h;
+                raw[q][1] = xc[even + (p >> 1)];
+                raw[q][2] = xc[odd + (p >> 1)];
+                const T w = xc[odd + (cg.ic[0] >> 1)], e = xc[even + (cg.ic[PW + 1] >> 1)];
+                raw[q][0] = cg.ic[0] == p ? raw[q][1] : w;
+                raw[q][PW + 1] = cg.ic[PW + 1] == p + 1 ? raw[q][2] : e;
+            } else {
+#pragma unroll
+                for (int c = 0; c < PW + 2; ++c) {
+                    const int i = cg.ic[c];
+                    raw[q][c] = xc[o + (cg.half ? (((i + cg.J[q] + K) & 1) ? cg.half : 0) + (i >> 1) : i)];
+                }
+            }
+        }
+    };
+    // plane K interpolated in x and y, to side A and side B of each pair
+    auto coarse_xy = [&](const T (&raw)[2][PW + 2], T (&a)[PW], T (&bs)[PW]) {
+        const T w0 = T(0.75), w1 = T(0.25);
+        const bool east = (j & 1) != 0;
+#pragma unroll
+        for (int c = 0; c < PW; ++c) {
+            T lo[2], hi[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const T m = w0 * raw[q][c + 1];
+                lo[q] = m + w1 * raw[q][c];
+                hi[q] = m + w1 * raw[q][c + 2];
+            }
+            const T vw = w0 * lo[0] + w1 * lo[1], ve = w0 * hi[0] + w1 * hi[1];
+            a[c] = east ? ve : vw;
+            bs[c] = east ? vw : ve;
+        }
+    };
     // two steps' loads are in flight (each step reuses its own registers for
     // the step after the next), so a step does not wait for the memory latency
     fetch(z0 - 2, n0);
     fetch(z0 - 1, n1);
+    if constexpr (PRO) {
+        const int K = (z0 - 2) >> 1;
+        T before[2][PW + 2];
+#pragma unroll
+        for (int c = 0; c < PW; ++c) cg.a[c] = cg.ap[c] = cg.b[c] = T(0);
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int c = 0; c < PW + 2; ++c) before[q][c] = cg.raw[q][c] = T(0);
+        if (valid) {
+            coarse_load(K - 1, before);
+            coarse_load(K, cg.raw);
+            coarse_xy(before, cg.ap, cg.b);
+            coarse_xy(cg.raw, cg.a, cg.b);
+            if (z0 & 1) coarse_load(K + 1, cg.raw);
+        }
+    }
     if (stopped != 0.0) return;
     double dsum = 0.0;
     if (ty < sh.ry && !inA) {   // black values beyond a side stay 0
@@ -268,6 +357,26 @@ __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, con
             }
             cb[c] = n.b[c];
             r2[c] = n.r[c];
+        }
+        if constexpr (PRO) {
+            // s = 3/4 of the parent plane K = P / 2 and 1/4 of K - 1 (P even)
+            // or K + 1, whose values were loaded in the step before
+            const T w0 = T(0.75), w1 = T(0.25);
+            if (P & 1) {
+                T a[PW], bs[PW];
+                coarse_xy(cg.raw, a, bs);
+#pragma unroll
+                for (int c = 0; c < PW; ++c) {
+                    r2[c] = r2[c] + (w0 * cg.b[c] + w1 * bs[c]);
+                    cg.ap[c] = cg.a[c];
+                    cg.a[c] = a[c];
+                    cg.b[c] = bs[c];
+                }
+            } else {
+#pragma unroll
+                for (int c = 0; c < PW; ++c) r2[c] = r2[c] + (w0 * cg.a[c] + w1 * cg.ap[c]);
+                if (valid && P + 1 < z1 + 2) coarse_load((P >> 1) + 1, cg.raw);
+            }
         }
         if (FROMB) {
             ids(y, kr, y.id, s_id, idv);
@@ -359,14 +468,17 @@ __device__ __forceinline__ Blk march_blk(const MarchShape &sh) {
     kb.bz = (int)blockIdx.x >> 3 < per && q < nb ? q / (sh.ntx * sh.nty) : -1;
     return kb;
 }
-template <typename T, int PW, int MODE, bool FROMB>
-__global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void k_march(LevelDev L, const T *__restrict__ xin, const T *__restrict__ b,
-                                              T *__restrict__ out, T *__restrict__ out2,
-                                              double *__restrict__ partial, const double *__restrict__ stop) {
+template <typename T, int PW, int MODE, bool FROMB, bool PRO>
+__global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void k_march(LevelDev L, const T *__restrict__ xin,
+                                                                      const T *__restrict__ b, T *__restrict__ out,
+                                                                      T *__restrict__ out2,
+                                                                      double *__restrict__ partial,
+                                                                      const T *__restrict__ xc,
+                                                                      const double *__restrict__ stop) {
     const MarchShape sh = march_shape<T>(L, PW);
     const Blk kb = march_blk(sh);
     if (kb.bz < 0) return;
-    march_body<T, PW, MODE, FROMB>(kb, L, xin, b, out, out2, partial, sh.nzp, stop);
+    march_body<T, PW, MODE, FROMB, PRO>(kb, L, xin, b, out, out2, partial, sh.nzp, xc, stop);
 }
 
 // The last black and red sweeps at level 0 of the mixed form, one launch each:

@@ -261,6 +261,28 @@ __global__ __launch_bounds__(TileDown::NT) void k_tile_down(LevelDev L, const T 
     tile_down_body<T>(hw_blk(), L, bg, xr, Cl, bc, stop);
 }
 
+// whether pair m of a thread lies in the tile itself (not its halo)
+template <typename G, typename C>
+__device__ __forceinline__ bool tile_owns(const C &c, const LevelDev &L, int ox, int oy, int oz, int m) {
+    const int j = oy + c.y, k = oz + c.z + m, i = ox + 2 * c.p;
+    return c.act && c.p >= 2 && c.p < 2 + TL_X / 2 && c.y >= 4 && c.y < 4 + TL_Y && c.z + m >= 4 &&
+           c.z + m < 4 + TL_Z && i < L.nx && j < L.ny && k < L.nz;
+}
+// the block's partial sum: wavefronts by shuffles, then in order
+template <typename G>
+__device__ __forceinline__ void tile_partial(const Blk &kb, double dsum, double *__restrict__ partial) {
+    const int t = threadIdx.x;
+    __shared__ double red[G::NT / 64];
+    for (int st = 32; st > 0; st >>= 1) dsum += __shfl_down(dsum, st, 64);
+    if ((t & 63) == 0) red[t >> 6] = dsum;
+    __syncthreads();
+    if (t == 0) {
+        double a = 0.0;
+        for (int w = 0; w < G::NT / 64; ++w) a += red[w];
+        partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = a;
+    }
+}
+
 // The correction of the red cells and two post-smoothing sweeps: the red
 // cells' x of tile_down and the coarse level's x in, x (both halves) out;
 // with partial, one partial sum of b.x per block (level 0: r.z).
@@ -346,25 +368,14 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
     double dsum = 0.0;
 #pragma unroll
     for (int m = 0; m < G::M; ++m) {
-        const int j = oy + c.y, k = oz + c.z + m, i = ox + 2 * c.p;
-        if (c.act && c.p >= 2 && c.p < 2 + TL_X / 2 && c.y >= 4 && c.y < 4 + TL_Y && c.z + m >= 4 &&
-            c.z + m < 4 + TL_Z && i < L.nx && j < L.ny && k < L.nz) {
+        if (tile_owns<G>(c, L, ox, oy, oz, m)) {
             x[c.pos[m]] = c.r[m];
             x[L.half + c.pos[m]] = c.b[m];
             dsum += double(c.fr[m]) * double(c.r[m]);
             dsum += double(c.fb[m]) * double(c.b[m]);
         }
     }
-    if (!partial) return;
-    __shared__ double red[G::NT / 64];
-    for (int st = 32; st > 0; st >>= 1) dsum += __shfl_down(dsum, st, 64);
-    if ((t & 63) == 0) red[t >> 6] = dsum;
-    __syncthreads();
-    if (t == 0) {
-        double a = 0.0;
-        for (int w = 0; w < G::NT / 64; ++w) a += red[w];
-        partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = a;
-    }
+    if (partial) tile_partial<G>(kb, dsum, partial);
 }
 template <typename T>
 __global__ __launch_bounds__(TileUp::NT) void k_tile_up(LevelDev L, const T *__restrict__ bg,
@@ -372,6 +383,27 @@ __global__ __launch_bounds__(TileUp::NT) void k_tile_up(LevelDev L, const T *__r
                                                         const T *__restrict__ xc, double *__restrict__ partial,
                                                         const double *__restrict__ stop) {
     tile_up_body<T>(hw_blk(), L, bg, xr, x, Cl, xc, partial, stop);
+}
+
+// tile_up_body's partial sums of b.x from an x that is there already: a batch
+// whose level 0 marches still sums r.z as each case's own launch does.
+template <typename T>
+__device__ __forceinline__ void tile_rz_body(const Blk &kb, const LevelDev &L, const T *__restrict__ bg,
+                                             const T *__restrict__ x, double *__restrict__ partial,
+                                             const double *__restrict__ stop) {
+    using G = TileUp;
+    if (*stop != 0.0) return;
+    const int ox = kb.bx * TL_X - 4, oy = kb.by * TL_Y - 4, oz = kb.bz * TL_Z - 4;
+    TileCells<T, G> c;
+    tile_init(c, L, ox, oy, oz);
+    double dsum = 0.0;
+#pragma unroll
+    for (int m = 0; m < G::M; ++m)
+        if (tile_owns<G>(c, L, ox, oy, oz, m)) {
+            dsum += double(bg[c.pos[m]]) * double(x[c.pos[m]]);
+            dsum += double(bg[L.half + c.pos[m]]) * double(x[L.half + c.pos[m]]);
+        }
+    tile_partial<G>(kb, dsum, partial);
 }
 
 dim3 tile_grid(const LevelDev &d) { return dim3(div_up(d.nx, TL_X), div_up(d.ny, TL_Y), div_up(d.nz, TL_Z)); }

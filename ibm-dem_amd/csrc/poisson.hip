@@ -1513,16 +1513,18 @@ bool tile_level(const ibmdem_ctx *c, int l) {
     return tile_level<T>(c->lev64[l].d, l, c->cs.mg_pre, c->cs.mg_post);
 }
 
-template <typename T, int MODE, bool FROMB>
+template <typename T, int MODE, bool FROMB, bool PRO = false>
 void launch_march(hipStream_t s, const LevelDev &d, const T *xin, const T *b, T *out, T *out2, double *partial,
-                  const double *stop) {
+                  const double *stop, const T *xc = nullptr) {
     const int pw = march_pw(d);
     const MarchShape sh = march_shape<T>(d, pw);
     const dim3 grid(8 * div_up(sh.ntx * sh.nty * sh.nzc, 8)), block(MT);
     if (pw == 2)
-        hipLaunchKernelGGL((k_march<T, 2, MODE, FROMB>), grid, block, 0, s, d, xin, b, out, out2, partial, stop);
+        hipLaunchKernelGGL((k_march<T, 2, MODE, FROMB, PRO>), grid, block, 0, s, d, xin, b, out, out2, partial, xc,
+                           stop);
     else
-        hipLaunchKernelGGL((k_march<T, 1, MODE, FROMB>), grid, block, 0, s, d, xin, b, out, out2, partial, stop);
+        hipLaunchKernelGGL((k_march<T, 1, MODE, FROMB, PRO>), grid, block, 0, s, d, xin, b, out, out2, partial, xc,
+                           stop);
 }
 
 // the mixed form's last two sweeps at level 0: the red cells' x from xr, the
@@ -1539,6 +1541,17 @@ void launch_rz(hipStream_t s, const LevelDev &d, const float *xr, float *x0, flo
         else
             hipLaunchKernelGGL(k_rz_half<1>, sw.grid, sw.block, 0, s, d, oth, own, 1 - q, r64, partial, q * nb, stop);
     }
+}
+
+// Whether a marching level's prolongation is part of its first post-smoothing
+// pass (in FP64, when another pass follows that finalizes x). The pass's steps
+// take half as long again, which the launch and the traffic saved outweigh on
+// large levels: 66 us in place of 41 + 41 at 256^3, 20 in place of 12.7 + 8.7
+// at 128^3; on the smallest that march they meet: 19.7 and 12.0 + 7.9 at
+// 100x76x130, 18.5 and 11.3 + 6.7 at 64x64x256, with one launch less.
+template <typename T>
+constexpr bool prolong_fused(int post) {
+    return std::is_same<T, double>::value && post >= 2;
 }
 
 template <typename T>
@@ -1610,19 +1623,28 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
     CHECK_LAUNCH(c);
     int rc = vcycle<T>(c, lev, l + 1);
     if (rc) return rc;
+    const bool fused = prolong_fused<T>(c->cs.mg_post);
     const LaunchShape ps = shape_for(d.nx / 2 / march_pw(d), d.ny, d.nz);
-    if (march_pw(d) == 2)
-        hipLaunchKernelGGL((k_prolong_red<T, 2>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
-    else
-        hipLaunchKernelGGL((k_prolong_red<T, 1>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
-    CHECK_LAUNCH(c);
+    if (!fused) {
+        if (march_pw(d) == 2)
+            hipLaunchKernelGGL((k_prolong_red<T, 2>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
+        else
+            hipLaunchKernelGGL((k_prolong_red<T, 1>), ps.grid, ps.block, 0, s, d, cur, r0, C.d, C.x, stop);
+        CHECK_LAUNCH(c);
+    }
+    const T *uncorrected = cur;
     cur = r0;
     bytes = 0.0;
     if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
     for (int q = 0; q < c->cs.mg_post; ++q) {
         if (q < c->cs.mg_post - 1) {
             T *to = cur == r0 ? r1 : r0;
-            launch_march<T, 0, false>(s, d, cur, L.b, to, nullptr, nullptr, stop);
+            if (q == 0 && fused) {
+                if constexpr (std::is_same<T, double>::value)
+                    launch_march<T, 0, false, true>(s, d, uncorrected, L.b, to, nullptr, nullptr, stop, C.x);
+            } else {
+                launch_march<T, 0, false>(s, d, cur, L.b, to, nullptr, nullptr, stop);
+            }
             bytes += 2.0 * cell;
             cur = to;
         } else if (dot && l == 0) {
@@ -1987,13 +2009,14 @@ struct MaArg {
     T *out, *out2;
     double *partial;
     int nzp;   // planes of a chunk
+    const T *xc;
     const double *stop;
 };
-template <typename T, int PW, int MODE, bool FROMB>
+template <typename T, int PW, int MODE, bool FROMB, bool PRO>
 __global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void kb_march(BTable<MaArg<T>> tab) {
     batch_for(tab, [&](const MaArg<T> &a, const Blk &kb) {
-        march_body<T, PW, MODE, FROMB>(kb, *cst(a.L), glb(a.xin), glb(a.b), glb(a.out), glb(a.out2),
-                                       glb(a.partial), a.nzp, glb(a.stop));
+        march_body<T, PW, MODE, FROMB, PRO>(kb, *cst(a.L), glb(a.xin), glb(a.b), glb(a.out), glb(a.out2),
+                                            glb(a.partial), a.nzp, glb(a.xc), glb(a.stop));
     });
 }
 
@@ -2039,6 +2062,12 @@ __global__ __launch_bounds__(TileUp::NT) void kb_tile_up(BTable<TlArg<T>> tab) {
     batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
         tile_up_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xr), glb(a.x), *cst(a.C), glb(a.xc),
                         a.partial ? glb(a.partial) : (double *)nullptr, glb(a.stop));
+    });
+}
+template <typename T>
+__global__ __launch_bounds__(TileUp::NT) void kb_tile_rz(BTable<TlArg<T>> tab) {
+    batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
+        tile_rz_body<T>(kb, *cst(a.L), glb(a.b), glb((const T *)a.x), glb(a.partial), glb(a.stop));
     });
 }
 
@@ -2179,9 +2208,9 @@ struct BProf {
     std::vector<double> bytes;
     int n = 0;                          // launches recorded
 };
-template <typename T, int PW, int MODE, bool FROMB>
+template <typename T, int PW, int MODE, bool FROMB, bool PRO = false>
 void launch_ma(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL((kb_march<T, PW, MODE, FROMB>), dim3(o.blocks), dim3(MT), 0, s, table<MaArg<T>>(o));
+    hipLaunchKernelGGL((kb_march<T, PW, MODE, FROMB, PRO>), dim3(o.blocks), dim3(MT), 0, s, table<MaArg<T>>(o));
 }
 template <int PW>
 void launch_rzb(const BOp &o, hipStream_t s, int) {
@@ -2190,6 +2219,10 @@ void launch_rzb(const BOp &o, hipStream_t s, int) {
 template <typename T>
 void launch_down(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_tile_down<T>, dim3(o.blocks), dim3(TileDown::NT), 0, s, table<TlArg<T>>(o));
+}
+template <typename T>
+void launch_tile_rz(const BOp &o, hipStream_t s, int) {
+    hipLaunchKernelGGL(kb_tile_rz<T>, dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
 }
 template <typename T>
 void launch_up(const BOp &o, hipStream_t s, int) {
@@ -2261,10 +2294,12 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
     int depth = 0;
     for (ibmdem_ctx *c : cs) depth = std::max(depth, bottom_level(c));
     int rc;
-    // The cells that smooth on level l, over the cases. Below level 0 tiles or
-    // passes (the same values) are chosen by them, as for one level of that
-    // size: a batch fills the chip, and the tiles' halo then costs time.
-    // Level 0 takes each case's own form, whose r.z sums are the form's.
+    // The cells that smooth on level l, over the cases. Tiles or passes (the
+    // same values) are chosen by them, as for one level of that size: a batch
+    // fills the chip, and the tiles' halo then costs time (40 cases of
+    // 96x80x64 in FP64: BATCH_T in tiles, BATCH_M in passes). What the form
+    // decides in a case's own run stays as it is there: the order of the r.z
+    // sums (TlRz below) and whether the prolongation is part of a pass.
     auto cells_at = [&](int l) {
         double n = 0.0;
         for (ibmdem_ctx *c : cs)
@@ -2272,12 +2307,13 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         return n;
     };
     auto tiled = [&](const ibmdem_ctx *c, int l) {
-        return tile_level<T>(c, l) && (l == 0 || cells_at(l) <= (double)TILE_CELLS);
+        return tile_level<T>(c, l) && cells_at(l) <= (double)TILE_CELLS;
     };
     // The pass of level l (vcycle's, MODE and FROMB by mode and fromb) of every
     // case whose V-cycle goes below l: one launch for the cases with two-pair
     // threads, one for the others. in and out: 0, 1 the halves of x, 2, 3 of r
-    auto pass = [&](int l, int mode, bool fromb, int in, int to, int to2) {
+    // (own_tile: 1 the cases whose own form is tiles alone, 0 the others alone)
+    auto pass = [&](int l, int mode, bool fromb, int in, int to, int to2, int own_tile = -1, bool pro = false) {
         std::vector<MaArg<T>> args[2];
         BOp o[2];
         const double total = cells_at(l);
@@ -2287,6 +2323,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
                                                        : 2.0 * sizeof(T);
         for (ibmdem_ctx *c : cs) {
             if (l >= bottom_level(c) || tiled(c, l)) continue;
+            if (own_tile >= 0 && tile_level<T>(c, l) != (own_tile == 1)) continue;
             MGLevel<T> &L = levels<T>(c)[l];
             T *buf[4] = {L.x, L.x + L.d.half, L.r, L.r + L.d.half};
             const int pw = march_pw(L.d);
@@ -2300,10 +2337,12 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             a.out2 = to2 >= 0 ? buf[to2] : nullptr;
             a.partial = mode == 2 ? c->partial : nullptr;
             a.nzp = sh.nzp;
+            a.xc = pro ? levels<T>(c)[l + 1].x : nullptr;
             a.stop = c->scal + SC_CONV;
             args[pw - 1].push_back(a);
             if (l == 0) o[pw - 1].bytes += per * (double)c->n;
         }
+        const BLaunch fp[2] = {launch_ma<double, 1, 0, false, true>, launch_ma<double, 2, 0, false, true>};
         const BLaunch fn[2][5] = {
             {launch_ma<T, 1, 0, false>, launch_ma<T, 1, 0, true>, launch_ma<T, 1, 1, false>, launch_ma<T, 1, 1, true>,
              mode == 2 ? launch_ma<double, 1, 2, false> : launch_ma<T, 1, 3, false>},
@@ -2311,7 +2350,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
              mode == 2 ? launch_ma<double, 2, 2, false> : launch_ma<T, 2, 3, false>}};
         for (int v = 1; v >= 0; --v) {
             o[v].kind = l == 0 ? IBMDEM_BK_SMOOTH0 : IBMDEM_BK_SMOOTH;
-            const int r2 = add_op(ar, ops, fn[v][mode >= 2 ? 4 : 2 * mode + fromb], MT, args[v], o[v], err);
+            const int r2 = add_op(ar, ops, pro ? fp[v] : fn[v][mode >= 2 ? 4 : 2 * mode + fromb], MT, args[v], o[v], err);
             if (r2) return r2;
         }
         return (int)IBMDEM_OK;
@@ -2369,6 +2408,26 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             if (l == 0) o.bytes += (up ? 2.5 : 1.5) * sizeof(T) * (double)c->n;
         }
         return add_op(ar, ops, up ? launch_up<T> : launch_down<T>, up ? TileUp::NT : TileDown::NT, args, o, err);
+    };
+    // r.z of the cases whose own level-0 form is tiles, after passes
+    auto tile_rz = [&]() {
+        std::vector<TlArg<T>> args;
+        BOp o;
+        o.kind = IBMDEM_BK_SMOOTH0;
+        for (ibmdem_ctx *c : cs) {
+            if (tiled(c, 0) || !tile_level<T>(c, 0)) continue;
+            MGLevel<T> &L = levels<T>(c)[0];
+            TlArg<T> a{};
+            a.g = bgrid(tile_grid(L.d), dim3(256, TileUp::NT / 256));
+            a.L = c->dlev;
+            a.b = L.b;
+            a.x = L.x;
+            a.partial = c->partial;
+            a.stop = c->scal + SC_CONV;
+            args.push_back(a);
+            o.bytes += 2.0 * sizeof(T) * (double)c->n;
+        }
+        return add_op(ar, ops, launch_tile_rz<T>, TileUp::NT, args, o, err);
     };
     // the bottoms at level l
     auto bottoms = [&](int l) {
@@ -2469,11 +2528,12 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         if ((rc = add_op(ar, ops, launch_restrict<T>, RB, rs, ors, err))) return rc;
         if ((rc = bottoms(l + 1))) return rc;
     }
+    const bool fused = prolong_fused<T>(post);
     for (int l = depth - 1; l >= 0; --l) {
         std::vector<PrArg<T>> pr[2];
         BOp opr[2];
         for (ibmdem_ctx *c : cs) {
-            if (l >= bottom_level(c) || tiled(c, l)) continue;
+            if (l >= bottom_level(c) || tiled(c, l) || (fused && !tile_level<T>(c, l))) continue;
             MGLevel<T> &F = levels<T>(c)[l], &C = levels<T>(c)[l + 1];
             const int pw = march_pw(F.d);
             const LaunchShape sh = shape_for(F.d.nx / 2 / pw, F.d.ny, F.d.nz);
@@ -2501,7 +2561,17 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
                 if ((rc = rz(cur))) return rc;
                 break;
             }
-            if ((rc = pass(l, last ? (l == 0 ? 2 : 3) : 0, false, cur, last ? 0 : to, last ? 1 : -1))) return rc;
+            if (!last) {
+                const bool pro = q == 0 && fused;
+                if (pro && (rc = pass(l, 0, false, last_in, to, -1, 0, true))) return rc;
+                if ((rc = pass(l, 0, false, cur, to, -1, pro ? 1 : -1))) return rc;
+            } else if (l == 0) {
+                if ((rc = pass(l, 2, false, cur, 0, 1, 0))) return rc;
+                if ((rc = pass(l, 3, false, cur, 0, 1, 1))) return rc;
+                if ((rc = tile_rz())) return rc;
+            } else if ((rc = pass(l, 3, false, cur, 0, 1))) {
+                return rc;
+            }
             cur = to;
         }
     }

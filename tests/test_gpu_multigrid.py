@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from ibmdem import cases
-from ibmdem.abi import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, ERR_NOT_CONVERGED, IbmdemError, Simulation)
+from ibmdem.abi import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, ERR_NOT_CONVERGED, IbmdemError, Batch, Simulation)
 
 pytestmark = pytest.mark.gpu
 P, W, I, O = BC_PERIODIC, BC_WALL, BC_INFLOW, BC_OUTFLOW
@@ -112,3 +112,46 @@ def test_small_levels_in_one_work_group(gpu_lib, monkeypatch, n, bt, precision):
         out.append(_iterate(gpu_lib, n, bt, precision))
     assert np.abs(out[0]).max() > 0
     np.testing.assert_array_equal(out[0], out[1])
+
+
+# levels whose prolongation is part of a smoothing pass: one pair per thread
+# and two, rows in one tile and in several, chunks that begin in odd planes,
+# coarse rows of odd length, every side type
+@pytest.mark.parametrize("n,bt", [
+    ((64, 118, 200), [W] * 6),
+    ((130, 90, 78), [P, P, W, W, W, W]),
+    ((130, 108, 110), [P] * 6),
+    ((130, 100, 118), [W, W, P, P, I, O]),
+    ((262, 90, 66), [I, O, W, W, P, P]),
+    ((520, 60, 50), [P, P, W, W, W, W]),
+])
+def test_prolongation_in_a_pass(gpu_lib, oracle_lib, n, bt):
+    _close(_iterate(gpu_lib, n, bt), _iterate(oracle_lib, n, bt), 1e-12)
+
+
+# batches whose levels march where each case's own run takes tiles: several
+# equal cases, uneven ones, and one that marches by itself among them
+@pytest.mark.parametrize("sizes", [
+    [(64, 48, 56)] * 6,
+    [(96, 64, 40), (50, 80, 64), (72, 72, 64), (64, 36, 128)],
+    [(32, 32, 32), (130, 90, 80), (48, 64, 32)],
+])
+def test_batch_marches_where_cases_tile(gpu_lib, sizes):
+    setups = [cases.small_periodic(n=n, n_spheres=2) for n in sizes]
+
+    def out(s):
+        return s.download_fields()
+
+    with Batch(gpu_lib, [s.case for s in setups]) as b:
+        for q, s in enumerate(setups):
+            cases.load(b[q], s)
+        infos = b.run(3)
+        got = [(out(b[q]), infos[q].iterations) for q in range(len(b))]
+    for s, (fields, iterations) in zip(setups, got):
+        with Simulation(gpu_lib, s.case) as one:
+            cases.load(one, s)
+            for _ in range(3):
+                info = one.step()
+            assert info.iterations == iterations
+            for a, c in zip(fields, out(one)):
+                np.testing.assert_array_equal(a, c)
