@@ -114,8 +114,8 @@ def timed_run(setup, precision, steps, warmup, profile):
 
 KERNEL_NAMES = {
     "spread": "k_spread_tiles (IBM spread + multi-direct-forcing update)",
-    "mg_smooth": "k_rb_half, all level-0 variants (red-black Gauss-Seidel half-sweeps: plain, "
-                 "first sweep, residual, r.z)",
+    "mg_smooth": "k_march, all level-0 passes (two fused red-black Gauss-Seidel half sweeps each: first, "
+                 "residual, with the prolongation, r.z)",
     "interp": "k_interp (IBM interpolation)",
     "predictor": "k_predictor_lds (fused advection-diffusion predictor, LDS z-marching)",
 }

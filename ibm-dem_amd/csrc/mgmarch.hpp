@@ -34,9 +34,9 @@
 // reason above.)
 // A level then moves 1.5 + 2 + 2 + 2.5 of its cells per V-cycle (pre = post
 // = 2) where one launch per half sweep and one for the residual moved 14.5,
-// in 4 launches instead of 9. At 256^3 in FP64 the four take 41, 41, 42 and
-// 51 us (6.1 TB/s on those bytes but for the first, 4.9; the separate ones
-// took 311 us), bound by HBM; on small levels by the steps (0.8 us each).
+// in 4 launches instead of 9. At 256^3 in FP64 the four take 41, 44, 66
+// (with the prolongation, 41 without) and 50 us (about 6 TB/s on those bytes
+// but for the first, 4.9; the separate ones took 311 us), bound by HBM; on small levels by the steps (0.8 us each).
 //
 // A work-group owns a tile of rows (whole rows up to 64 x-pair groups, ranges
 // of a row above) and marches up a chunk of planes, each thread with one
@@ -70,7 +70,10 @@ constexpr bool RES_BLACK = std::is_same<T, float>::value;   // the black cells' 
 // loads four halo planes).
 constexpr int MARCH_MIN = 4;
 // `share`: the part of the chip the launch has for this level (a launch over a
-// batch of cases: the level's part of its cells).
+// batch of cases: the level's part of its cells). There the cases' work-groups
+// are of uneven length and rounded per case, so in FP64, where one fills a CU,
+// two rounds of them are made (40 uneven cases of 96x80x64 cells on average:
+// 4.9 in place of 5.3 ms a step at level 0; 64 cases in FP32 lose 1 % by it).
 template <typename T>
 __host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw, double share = 1.0) {
     MarchShape s;
@@ -83,7 +86,8 @@ __host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw, dou
     s.ty = (d.ny + s.nty - 1) / s.nty;
     s.ry = s.ty + 4;
     const int tiles = s.ntx * s.nty, slots = (int)((sizeof(T) == 8 ? 256 : 512) * share);
-    const int want = tiles < slots ? slots / tiles : 1;
+    const int want = sizeof(T) == 8 && share < 1.0 ? (int)(2.0 * 256 * share / tiles + 1.0)
+                                                   : (tiles < slots ? slots / tiles : 1);
     int per = (d.nz + want - 1) / want;
     per = per < MARCH_MIN ? MARCH_MIN : per;
     s.nzc = (d.nz + per - 1) / per;

@@ -605,7 +605,7 @@ __global__ __launch_bounds__(CT_T) void k_coarse_tile(const LevelDev *__restrict
 // LDS and registers, with as few wavefronts as hold the level in one or two
 // rounds (a barrier of four is faster than one of sixteen), tiles above. At
 // the line, CWG_PAIRS pairs in FP64, one work-group takes 137 us and the
-// tiles' 24 launches 190 us.
+// tiles' 24 launches took 190 us (at 9.5 us each; 7.3 now).
 enum CoarseForm { CF_WG256, CF_WG1, CF_WG2, CF_WG4, CF_WG8, CF_JAC512, CF_JAC2, CF_JAC8, CF_TILE, CF_TILE_JAC };
 CoarseForm coarse_form(const LevelDev &d) {
     const long n = (long)d.nx * d.ny * d.nz, pairs = (long)((d.nx + 1) / 2) * d.ny * d.nz;
@@ -1497,7 +1497,8 @@ LevelDev make_level(int nx, int ny, int nz, const int bt[6], const double h[3]) 
 int march_pw(const LevelDev &d) { return (d.nx >> 1) % 2 == 0 ? 2 : 1; }
 
 // Levels of up to TILE_CELLS cells smooth in tiles (mgtile.hpp: two launches a
-// visit), larger ones in marching passes (mgmarch.hpp: six). In FP64 a visit's
+// visit), larger ones in marching passes (mgmarch.hpp: five, six
+// in FP32). In FP64 a visit's
 // launches take 18 us in tiles and 61 us in passes at 64^3, 66 and 63 us at
 // 64x64x256, 94 and 72 us at 128^3; the line lies where they meet, less the
 // gaps between four more launches. The mixed form's level 0 always marches
@@ -2296,8 +2297,9 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
     int rc;
     // The cells that smooth on level l, over the cases. Tiles or passes (the
     // same values) are chosen by them, as for one level of that size: a batch
-    // fills the chip, and the tiles' halo then costs time (40 cases of
-    // 96x80x64 in FP64: BATCH_T in tiles, BATCH_M in passes). What the form
+    // fills the chip, and the tiles' halo then costs time (40 uneven
+    // cases of 96x80x64 cells on average in FP64: 104 ms a pass of four steps
+    // and download with level 0 in tiles, 73 ms in passes). What the form
     // decides in a case's own run stays as it is there: the order of the r.z
     // sums (TlRz below) and whether the prolongation is part of a pass.
     auto cells_at = [&](int l) {

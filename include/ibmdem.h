@@ -331,8 +331,8 @@ int ibmdem_batch_stats(const ibmdem_batch *batch, int64_t *fused_solves, double 
  * and the launches' run times are added up per kind. profile_read gives a
  * kind's total ms, launches and total algorithmic HBM bytes (0 where not
  * stated). */
-#define IBMDEM_BK_SMOOTH0   1   /* level-0 red-black half sweeps, all variants */
-#define IBMDEM_BK_SMOOTH    2   /* half sweeps of the coarser levels           */
+#define IBMDEM_BK_SMOOTH0   1   /* level-0 smoothing launches, all forms       */
+#define IBMDEM_BK_SMOOTH    2   /* those of the coarser levels                 */
 #define IBMDEM_BK_RESTRICT  3
 #define IBMDEM_BK_PROLONG   4
 #define IBMDEM_BK_BOTTOM    5   /* one-work-group tails, coarsest-level solves */
@@ -348,7 +348,7 @@ int ibmdem_batch_profile_read(const ibmdem_batch *batch, int32_t kind, double *t
  * kernel on the context stream; the level-0 smoother's pre- and post-smoothing
  * sweeps are timed as two groups of back-to-back launches). */
 #define IBMDEM_K_PREDICTOR   1
-#define IBMDEM_K_MG_SMOOTH   2   /* level-0 red-black half sweeps      */
+#define IBMDEM_K_MG_SMOOTH   2   /* level-0 smoothing passes           */
 #define IBMDEM_K_MATVEC      3   /* CG matrix-vector product           */
 #define IBMDEM_K_SPREAD      4
 #define IBMDEM_K_INTERP      5
