@@ -6,8 +6,9 @@
 // their work: smoothing, residual and restriction of a level take five
 // launches, correction and smoothing as many. Here each of the two halves is
 // one launch over tiles of TL_X x TL_Y x TL_Z cells: a work-group loads its
-// tile with a halo as deep as the half has half sweeps, keeps it in LDS and
-// registers, and sweeps the whole extended tile a barrier apart. A sweep's
+// tile with a halo as deep as the half has half sweeps (up to two sweeps; a
+// half of more is led by launches that smooth alone, tile_smooths), keeps it
+// in LDS and registers, and sweeps the whole extended tile a barrier apart. A sweep's
 // values are exact one layer further in than its input's, so the tile itself
 // is exact at the end; halo cells are the neighbouring tiles' cells with the
 // same arithmetic, so the result does not depend on the tiling and each
@@ -38,6 +39,10 @@ struct TileGeoC {
 };
 using TileDown = TileGeoC<6, 5, 5>;   // two sweeps, the residual, one layer for the restriction
 using TileUp = TileGeoC<4, 4, 4>;     // two sweeps
+
+// Where a launch's red cells come from: b / diag (the first red sweep from x =
+// 0), a launch before it, or that and the correction from the coarse level.
+enum TileSrc { TS_B, TS_X, TS_PROLONG };
 
 // level index of an unwrapped one: wrapped across a periodic side (however
 // often the halo goes round a small level), -1 beyond another
@@ -145,12 +150,16 @@ __device__ __forceinline__ void tile_sweep(TileCells<T, G> &c, bool red, int lay
     }
 }
 
-// Two pre-smoothing sweeps from x = 0, the residual and its restriction: b of
-// the level in, the red cells' x (xr, a half) and the coarse level's b out.
-template <typename T>
+// The last pre-smoothing sweeps, the residual and its restriction: b of the
+// level (and, TS_X, the red cells' x) in, the red cells' x (xr, a half) and
+// the coarse level's b out. From the first red sweep on (TS_B) or from xin:
+// black and red once more if `more`, then black.
+template <typename T, int SRC>
 __device__ __forceinline__ void tile_down_body(const Blk &kb, const LevelDev &L, const T *__restrict__ bg,
-                                               T *__restrict__ xr, const LevelDev &Cl, T *__restrict__ bc,
+                                               const T *__restrict__ xin, bool more, T *__restrict__ xr,
+                                               const LevelDev &Cl, T *__restrict__ bc,
                                                const double *__restrict__ stop) {
+    static_assert(SRC != TS_PROLONG, "the way down has no correction");
     using G = TileDown;
     const double stopped = *stop;   // waited for with the first loads
     __shared__ T sr[G::SLOTS], sb[G::SLOTS], s_id[64], s_dg[64];
@@ -168,6 +177,7 @@ __device__ __forceinline__ void tile_down_body(const Blk &kb, const LevelDev &L,
         const int g = max(c.pos[m], 0);
         c.fr[m] = bg[g];
         c.fb[m] = bg[L.half + g];
+        if (SRC == TS_X) c.r[m] = xin[g];
     }
     const bool plain = tile_plain(L, ox, oy, oz, 2 * G::RL, G::EY, G::EZ);
     __syncthreads();   // the tables
@@ -179,7 +189,8 @@ __device__ __forceinline__ void tile_down_body(const Blk &kb, const LevelDev &L,
     for (int m = 0; m < G::M; ++m) {
         c.fr[m] = c.pos[m] >= 0 ? c.fr[m] : T(0);
         c.fb[m] = c.pos[m] >= 0 ? c.fb[m] : T(0);
-        c.r[m] = (c.fr[m] + T(0)) * c.ir[m];
+        if (SRC == TS_X) c.r[m] = c.pos[m] >= 0 ? c.r[m] : T(0);
+        else c.r[m] = (c.fr[m] + T(0)) * c.ir[m];
         c.b[m] = T(0);
         if (c.act) {
             sr[c.q + m * G::PL] = c.r[m];
@@ -187,10 +198,12 @@ __device__ __forceinline__ void tile_down_body(const Blk &kb, const LevelDev &L,
         }
     }
     __syncthreads();
-    tile_sweep(c, false, 1, sr, sb, ihx2, ihy2, ihz2);
-    __syncthreads();
-    tile_sweep(c, true, 2, sr, sb, ihx2, ihy2, ihz2);
-    __syncthreads();
+    if (more) {
+        tile_sweep(c, false, 1, sr, sb, ihx2, ihy2, ihz2);
+        __syncthreads();
+        tile_sweep(c, true, 2, sr, sb, ihx2, ihy2, ihz2);
+        __syncthreads();
+    }
     T rb[G::M];   // the black cells' residual (FP32)
     const T dg_int = T(L.diag[DIAG_INTERIOR]);
 #pragma unroll
@@ -254,11 +267,12 @@ __device__ __forceinline__ void tile_down_body(const Blk &kb, const LevelDev &L,
     }
     bc[lidx(Cl, I, J, K)] = T(0.125) * s;
 }
-template <typename T>
-__global__ __launch_bounds__(TileDown::NT) void k_tile_down(LevelDev L, const T *__restrict__ bg, T *__restrict__ xr,
+template <typename T, int SRC>
+__global__ __launch_bounds__(TileDown::NT) void k_tile_down(LevelDev L, const T *__restrict__ bg,
+                                                            const T *__restrict__ xin, bool more, T *__restrict__ xr,
                                                             LevelDev Cl, T *__restrict__ bc,
                                                             const double *__restrict__ stop) {
-    tile_down_body<T>(hw_blk(), L, bg, xr, Cl, bc, stop);
+    tile_down_body<T, SRC>(hw_blk(), L, bg, xin, more, xr, Cl, bc, stop);
 }
 
 // whether pair m of a thread lies in the tile itself (not its halo)
@@ -283,14 +297,16 @@ __device__ __forceinline__ void tile_partial(const Blk &kb, double dsum, double 
     }
 }
 
-// The correction of the red cells and two post-smoothing sweeps: the red
-// cells' x of tile_down and the coarse level's x in, x (both halves) out;
+// One or two (`two`) sweeps, each black and then red: after the correction of
+// the red cells (TS_PROLONG: the red cells' x of tile_down and the coarse
+// level's x in), on a launch before this one (TS_X), or after the first red
+// sweep from x = 0 (TS_B). The red cells' x out, and with xb the black ones';
 // with partial, one partial sum of b.x per block (level 0: r.z).
-template <typename T>
+template <typename T, int SRC>
 __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, const T *__restrict__ bg,
-                                             const T *__restrict__ xr, T *__restrict__ x, const LevelDev &Cl,
-                                             const T *__restrict__ xc, double *__restrict__ partial,
-                                             const double *__restrict__ stop) {
+                                             const T *__restrict__ xr, T *__restrict__ x, T *__restrict__ xb, bool two,
+                                             const LevelDev &Cl, const T *__restrict__ xc,
+                                             double *__restrict__ partial, const double *__restrict__ stop) {
     using G = TileUp;
     const double stopped = *stop;
     __shared__ T sr[G::SLOTS], sb[G::SLOTS], s_id[64];
@@ -306,12 +322,12 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
 #pragma unroll
     for (int m = 0; m < G::M; ++m) {
         const int g = max(c.pos[m], 0);
-        c.r[m] = xr[g];
+        if (SRC != TS_B) c.r[m] = xr[g];
         c.fr[m] = bg[g];
         c.fb[m] = bg[L.half + g];
     }
     constexpr int CM = (CN + G::NT - 1) / G::NT;
-    T cv[CM];
+    T cv[CM];   // (TS_PROLONG)
     // a coarse coordinate beyond the level: wrapped, or the edge cell again
     auto cmap = [](int v, int n, int lo) {
         if (v >= 0 && v < n) return v;
@@ -320,14 +336,14 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
         return v < 0 ? v + n : v;
     };
 #pragma unroll
-    for (int u = 0; u < CM; ++u) {
+    for (int u = 0; u < (SRC == TS_PROLONG ? CM : 0); ++u) {
         const int q = min(t + u * G::NT, CN - 1), zz = q / (CX * CY), yy = q / CX % CY, xx = q % CX;
         cv[u] = xc[lidx(Cl, cmap((ox >> 1) - 1 + xx, Cl.nx, Cl.bt[0]), cmap((oy >> 1) - 1 + yy, Cl.ny, Cl.bt[2]),
                         cmap((oz >> 1) - 1 + zz, Cl.nz, Cl.bt[4]))];
     }
     const bool plain = tile_plain(L, ox, oy, oz, 2 * G::RL, G::EY, G::EZ);
 #pragma unroll
-    for (int u = 0; u < CM; ++u)
+    for (int u = 0; u < (SRC == TS_PROLONG ? CM : 0); ++u)
         if (t + u * G::NT < CN) sc[t + u * G::NT] = cv[u];
     __syncthreads();
     if (stopped != 0.0) return;
@@ -337,6 +353,14 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
     for (int m = 0; m < G::M; ++m) {
         c.fr[m] = c.pos[m] >= 0 ? c.fr[m] : T(0);
         c.fb[m] = c.pos[m] >= 0 ? c.fb[m] : T(0);
+        c.b[m] = T(0);
+        if (c.act) sb[c.q + m * G::PL] = T(0);
+        if (SRC != TS_PROLONG) {
+            if (SRC == TS_X) c.r[m] = c.pos[m] >= 0 ? c.r[m] : T(0);
+            else c.r[m] = (c.fr[m] + T(0)) * c.ir[m];
+            if (c.act) sr[c.q + m * G::PL] = c.r[m];
+            continue;
+        }
         // parents: the own coarse cell and the neighbour on the cell's side
         const int xx[2] = {c.p + 1, c.p + 1 + ((m & 1) ? -c.s0 : c.s0)};
         const int yo = oy + c.y, zo = oz + c.z + m;
@@ -351,38 +375,37 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
                 for (int c1 = 0; c1 < 2; ++c1)
                     s = s + wt[c3] * wt[c2] * wt[c1] * sc[(zz[c3] * CY + yy[c2]) * CX + xx[c1]];
         c.r[m] = c.pos[m] >= 0 ? c.r[m] + s : T(0);
-        c.b[m] = T(0);
-        if (c.act) {
-            sr[c.q + m * G::PL] = c.r[m];
-            sb[c.q + m * G::PL] = T(0);
-        }
+        if (c.act) sr[c.q + m * G::PL] = c.r[m];
     }
     __syncthreads();
     tile_sweep(c, false, 1, sr, sb, ihx2, ihy2, ihz2);
     __syncthreads();
     tile_sweep(c, true, 2, sr, sb, ihx2, ihy2, ihz2);
-    __syncthreads();
-    tile_sweep(c, false, 3, sr, sb, ihx2, ihy2, ihz2);
-    __syncthreads();
-    tile_sweep(c, true, 4, sr, sb, ihx2, ihy2, ihz2);
+    if (two) {
+        __syncthreads();
+        tile_sweep(c, false, 3, sr, sb, ihx2, ihy2, ihz2);
+        __syncthreads();
+        tile_sweep(c, true, 4, sr, sb, ihx2, ihy2, ihz2);
+    }
     double dsum = 0.0;
 #pragma unroll
     for (int m = 0; m < G::M; ++m) {
         if (tile_owns<G>(c, L, ox, oy, oz, m)) {
             x[c.pos[m]] = c.r[m];
-            x[L.half + c.pos[m]] = c.b[m];
+            if (xb) xb[c.pos[m]] = c.b[m];
             dsum += double(c.fr[m]) * double(c.r[m]);
             dsum += double(c.fb[m]) * double(c.b[m]);
         }
     }
     if (partial) tile_partial<G>(kb, dsum, partial);
 }
-template <typename T>
+template <typename T, int SRC>
 __global__ __launch_bounds__(TileUp::NT) void k_tile_up(LevelDev L, const T *__restrict__ bg,
-                                                        const T *__restrict__ xr, T *__restrict__ x, LevelDev Cl,
+                                                        const T *__restrict__ xr, T *__restrict__ x,
+                                                        T *__restrict__ xb, bool two, LevelDev Cl,
                                                         const T *__restrict__ xc, double *__restrict__ partial,
                                                         const double *__restrict__ stop) {
-    tile_up_body<T>(hw_blk(), L, bg, xr, x, Cl, xc, partial, stop);
+    tile_up_body<T, SRC>(hw_blk(), L, bg, xr, x, xb, two, Cl, xc, partial, stop);
 }
 
 // tile_up_body's partial sums of b.x from an x that is there already: a batch
@@ -405,5 +428,12 @@ __device__ __forceinline__ void tile_rz_body(const Blk &kb, const LevelDev &L, c
         }
     tile_partial<G>(kb, dsum, partial);
 }
+
+// The launches of a visit. Before tile_down (q = 0 ..) and from tile_down's
+// coarse level back up, each of one or two sweeps; the last one up writes x.
+int tile_smooths(int pre) { return pre > 2 ? div_up(pre - 2, 2) : 0; }
+bool tile_smooth_two(int pre, int q) { return pre - 2 - 2 * q >= 2; }
+int tile_ups(int post) { return div_up(post, 2); }
+bool tile_up_two(int post, int q) { return post - 2 * q >= 2; }
 
 dim3 tile_grid(const LevelDev &d) { return dim3(div_up(d.nx, TL_X), div_up(d.ny, TL_Y), div_up(d.nz, TL_Z)); }

@@ -1496,22 +1496,25 @@ LevelDev make_level(int nx, int ny, int nz, const int bt[6], const double h[3]) 
 // pairs per thread of a level's passes: two where its rows hold an even number
 int march_pw(const LevelDev &d) { return (d.nx >> 1) % 2 == 0 ? 2 : 1; }
 
-// Levels of up to TILE_CELLS cells smooth in tiles (mgtile.hpp: two launches a
-// visit), larger ones in marching passes (mgmarch.hpp: five, six
-// in FP32). In FP64 a visit's
-// launches take 18 us in tiles and 61 us in passes at 64^3, 66 and 63 us at
-// 64x64x256, 94 and 72 us at 128^3; the line lies where they meet, less the
-// gaps between four more launches. The mixed form's level 0 always marches
-// (its r.z sums, rz_half_body).
-constexpr long TILE_CELLS = 900000;
-template <typename T>
-bool tile_level(const LevelDev &d, int l, int pre, int post) {
-    return pre == 2 && post == 2 && (l > 0 || std::is_same<T, double>::value) &&
-           (long)d.nx * d.ny * d.nz <= TILE_CELLS;
-}
+// Levels of up to tile_cells() cells smooth in tiles (mgtile.hpp: two launches
+// a visit with up to two sweeps each way), larger ones in marching passes
+// (mgmarch.hpp: five, six in FP32). Tiles save launches and gaps, passes the
+// halo's work. A CG iteration with the level in tiles and in passes, us, by
+// (pre, post), in FP64 with 0.51 M cells (80^3), 0.74 M (80x96x96), 0.88 M
+// (96^3), 1.05 M (64x64x256) and 1.12 M (104^3):
+//   (2,2)  152/187  182/193  185/193  196/187  210/205
+//   (4,4)  224/290  267/291  273/298  290/286  306/306
+//   (1,1)  140/147  168/160  168/156  177/152  194/167
+//   (2,1)  148/168  178/178  179/176  189/170  205/186
+//   (3,3)  215/254  256/256  261/259  277/251  294/269
+// A launch of one sweep has the halo of two, so odd counts end earlier. Level 1
+// in FP32 meets later (0.51 M 327/362, 0.88 M 433/452, 1.12 M 518/523, 1.40 M
+// 680/677, 2.10 M 781/732), by 1 % or less where the line would differ. The
+// mixed form's level 0 always marches (its r.z sums, rz_half_body).
+long tile_cells(int pre, int post) { return (pre | post) & 1 ? 600000 : 900000; }
 template <typename T>
 bool tile_level(const ibmdem_ctx *c, int l) {
-    return tile_level<T>(c->lev64[l].d, l, c->cs.mg_pre, c->cs.mg_post);
+    return (l > 0 || std::is_same<T, double>::value) && c->lev64[l].n <= tile_cells(c->cs.mg_pre, c->cs.mg_post);
 }
 
 template <typename T, int MODE, bool FROMB, bool PRO = false>
@@ -1526,6 +1529,29 @@ void launch_march(hipStream_t s, const LevelDev &d, const T *xin, const T *b, T 
     else
         hipLaunchKernelGGL((k_march<T, 1, MODE, FROMB, PRO>), grid, block, 0, s, d, xin, b, out, out2, partial, xc,
                            stop);
+}
+
+// the launches of a level in tiles (mgtile.hpp)
+template <typename T>
+void launch_tile_down(hipStream_t s, TileSrc src, const MGLevel<T> &L, const MGLevel<T> &C, const T *xin, bool more,
+                      T *xr, const double *stop) {
+    const dim3 grid = tile_grid(L.d), block(TileDown::NT);
+    if (src == TS_B)
+        hipLaunchKernelGGL((k_tile_down<T, TS_B>), grid, block, 0, s, L.d, L.b, xin, more, xr, C.d, C.b, stop);
+    else
+        hipLaunchKernelGGL((k_tile_down<T, TS_X>), grid, block, 0, s, L.d, L.b, xin, more, xr, C.d, C.b, stop);
+}
+template <typename T>
+void launch_tile_up(hipStream_t s, TileSrc src, const MGLevel<T> &L, const MGLevel<T> &C, const T *xr, T *x, T *xb,
+                    bool two, double *partial, const double *stop) {
+    const dim3 grid = tile_grid(L.d), block(TileUp::NT);
+    if (src == TS_PROLONG)
+        hipLaunchKernelGGL((k_tile_up<T, TS_PROLONG>), grid, block, 0, s, L.d, L.b, xr, x, xb, two, C.d, C.x, partial,
+                           stop);
+    else if (src == TS_X)
+        hipLaunchKernelGGL((k_tile_up<T, TS_X>), grid, block, 0, s, L.d, L.b, xr, x, xb, two, C.d, C.x, partial, stop);
+    else
+        hipLaunchKernelGGL((k_tile_up<T, TS_B>), grid, block, 0, s, L.d, L.b, xr, x, xb, two, C.d, C.x, partial, stop);
 }
 
 // the mixed form's last two sweeps at level 0: the red cells' x from xr, the
@@ -1584,19 +1610,32 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
     double bytes = 0.0;
     MGLevel<T> &C = lev[l + 1];
     if (tile_level<T>(c, l)) {
-        // profiled at level 0: b read, the red cells' x written; b, x read,
-        // x written
+        // profiled at level 0: b (and from the second launch on the red
+        // cells' x) read, the red cells' x written; on the way up b, x read
+        // and the red cells' x written, the last time both colours'
+        const int pre = c->cs.mg_pre, post = c->cs.mg_post, ns = tile_smooths(pre), nu = tile_ups(post);
         if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
-        hipLaunchKernelGGL((k_tile_down<T>), tile_grid(d), dim3(TileDown::NT), 0, s, d, L.b, r0, C.d, C.b, stop);
+        for (int q = 0; q < ns; ++q) {
+            T *to = q & 1 ? x1 : x0;
+            launch_tile_up<T>(s, q ? TS_X : TS_B, L, C, cur, to, nullptr, tile_smooth_two(pre, q), nullptr, stop);
+            CHECK_LAUNCH(c);
+            cur = to;
+        }
+        launch_tile_down<T>(s, ns ? TS_X : TS_B, L, C, cur, pre > 1, r0, stop);
         CHECK_LAUNCH(c);
-        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, 1.5 * cell, 1);
+        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, (1.5 + 2.0 * ns) * cell, 1 + ns);
         const int rc = vcycle<T>(c, lev, l + 1);
         if (rc) return rc;
         if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
-        hipLaunchKernelGGL((k_tile_up<T>), tile_grid(d), dim3(TileUp::NT), 0, s, d, L.b, r0, x0, C.d, C.x,
-                           dot && l == 0 ? c->partial : (double *)nullptr, stop);
-        CHECK_LAUNCH(c);
-        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, 2.5 * cell, 1);
+        for (int q = 0; q < nu; ++q) {
+            const bool last = q == nu - 1;
+            T *from = q & 1 ? r1 : r0;
+            launch_tile_up<T>(s, q ? TS_X : TS_PROLONG, L, C, from, last ? x0 : (q & 1 ? r0 : r1),
+                              last ? x1 : (T *)nullptr, tile_up_two(post, q),
+                              dot && l == 0 && last ? c->partial : (double *)nullptr, stop);
+            CHECK_LAUNCH(c);
+        }
+        if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, (2.0 * nu + 0.5) * cell, nu);
         return IBMDEM_OK;
     }
     if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
@@ -2039,36 +2078,37 @@ __global__ __launch_bounds__(RB) void kb_rz_half(BTable<RzArg> tab, int color) {
     });
 }
 
-// a tile half of a level (down: b to the red cells' x and the coarse b; up:
-// from the coarse x to x)
+// a launch of a level in tiles (k_tile_down's and k_tile_up's arguments)
 template <typename T>
 struct TlArg {
     BGrid g;
     const LevelDev *L, *C;
-    const T *b;
-    T *xr, *x;
+    const T *b, *xin;
+    T *x, *xb;
+    bool more;   // k_tile_down's more, k_tile_up's two
     T *bc;
     const T *xc;
     double *partial;
     const double *stop;
 };
-template <typename T>
+template <typename T, int SRC>
 __global__ __launch_bounds__(TileDown::NT) void kb_tile_down(BTable<TlArg<T>> tab) {
     batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
-        tile_down_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xr), *cst(a.C), glb(a.bc), glb(a.stop));
+        tile_down_body<T, SRC>(kb, *cst(a.L), glb(a.b), glb(a.xin), a.more, glb(a.x), *cst(a.C), glb(a.bc),
+                               glb(a.stop));
     });
 }
-template <typename T>
+template <typename T, int SRC>
 __global__ __launch_bounds__(TileUp::NT) void kb_tile_up(BTable<TlArg<T>> tab) {
     batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
-        tile_up_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xr), glb(a.x), *cst(a.C), glb(a.xc),
-                        a.partial ? glb(a.partial) : (double *)nullptr, glb(a.stop));
+        tile_up_body<T, SRC>(kb, *cst(a.L), glb(a.b), glb(a.xin), glb(a.x), a.xb ? glb(a.xb) : (T *)nullptr, a.more,
+                             *cst(a.C), glb(a.xc), a.partial ? glb(a.partial) : (double *)nullptr, glb(a.stop));
     });
 }
 template <typename T>
 __global__ __launch_bounds__(TileUp::NT) void kb_tile_rz(BTable<TlArg<T>> tab) {
     batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
-        tile_rz_body<T>(kb, *cst(a.L), glb(a.b), glb((const T *)a.x), glb(a.partial), glb(a.stop));
+        tile_rz_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xin), glb(a.partial), glb(a.stop));
     });
 }
 
@@ -2217,17 +2257,17 @@ template <int PW>
 void launch_rzb(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_rz_half<PW>, dim3(o.blocks), dim3(RB), 0, s, table<RzArg>(o), o.color);
 }
-template <typename T>
+template <typename T, int SRC>
 void launch_down(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_tile_down<T>, dim3(o.blocks), dim3(TileDown::NT), 0, s, table<TlArg<T>>(o));
+    hipLaunchKernelGGL((kb_tile_down<T, SRC>), dim3(o.blocks), dim3(TileDown::NT), 0, s, table<TlArg<T>>(o));
 }
 template <typename T>
 void launch_tile_rz(const BOp &o, hipStream_t s, int) {
     hipLaunchKernelGGL(kb_tile_rz<T>, dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
 }
-template <typename T>
+template <typename T, int SRC>
 void launch_up(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_tile_up<T>, dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
+    hipLaunchKernelGGL((kb_tile_up<T, SRC>), dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
 }
 template <typename T>
 void launch_restrict(const BOp &o, hipStream_t s, int) {
@@ -2309,7 +2349,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         return n;
     };
     auto tiled = [&](const ibmdem_ctx *c, int l) {
-        return tile_level<T>(c, l) && cells_at(l) <= (double)TILE_CELLS;
+        return tile_level<T>(c, l) && cells_at(l) <= (double)tile_cells(pre, post);
     };
     // The pass of level l (vcycle's, MODE and FROMB by mode and fromb) of every
     // case whose V-cycle goes below l: one launch for the cases with two-pair
@@ -2387,29 +2427,57 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         }
         return (int)IBMDEM_OK;
     };
-    // the tile half of level l of every case that takes it
-    auto tile = [&](int l, bool up) {
+    // one launch in tiles on level l, of every case that takes them: in and
+    // to as pass's, src and more the kernel's
+    auto tile = [&](int l, bool up, TileSrc src, int in, int to, int to2, bool more, bool rzsum) {
         std::vector<TlArg<T>> args;
         BOp o;
         o.kind = l == 0 ? IBMDEM_BK_SMOOTH0 : IBMDEM_BK_SMOOTH;
         for (ibmdem_ctx *c : cs) {
             if (l >= bottom_level(c) || !tiled(c, l)) continue;
             MGLevel<T> &L = levels<T>(c)[l], &C = levels<T>(c)[l + 1];
+            T *buf[4] = {L.x, L.x + L.d.half, L.r, L.r + L.d.half};
             TlArg<T> a{};
             a.g = bgrid(tile_grid(L.d), dim3(256, (up ? TileUp::NT : TileDown::NT) / 256));
             a.L = c->dlev + l;
             a.C = c->dlev + l + 1;
             a.b = L.b;
-            a.xr = L.r;
-            a.x = L.x;
+            a.xin = in >= 0 ? buf[in] : nullptr;
+            a.x = buf[to];
+            a.xb = to2 >= 0 ? buf[to2] : nullptr;
+            a.more = more;
             a.bc = C.b;
             a.xc = C.x;
-            a.partial = up && l == 0 ? c->partial : nullptr;
+            a.partial = rzsum ? c->partial : nullptr;
             a.stop = c->scal + SC_CONV;
             args.push_back(a);
-            if (l == 0) o.bytes += (up ? 2.5 : 1.5) * sizeof(T) * (double)c->n;
+            if (l == 0) o.bytes += (src == TS_B ? 1.5 : to2 >= 0 ? 2.5 : 2.0) * sizeof(T) * (double)c->n;
         }
-        return add_op(ar, ops, up ? launch_up<T> : launch_down<T>, up ? TileUp::NT : TileDown::NT, args, o, err);
+        const BLaunch fu[3] = {launch_up<T, TS_B>, launch_up<T, TS_X>, launch_up<T, TS_PROLONG>};
+        const BLaunch fd[2] = {launch_down<T, TS_B>, launch_down<T, TS_X>};
+        return add_op(ar, ops, up ? fu[src] : fd[src], up ? TileUp::NT : TileDown::NT, args, o, err);
+    };
+    // the halves of a visit in tiles, as vcycle's
+    auto tile_down = [&](int l) {
+        const int ns = tile_smooths(pre);
+        int in = -1, r2;
+        for (int q = 0; q < ns; ++q) {
+            const int to = q & 1;
+            if ((r2 = tile(l, true, q ? TS_X : TS_B, in, to, -1, tile_smooth_two(pre, q), false))) return r2;
+            in = to;
+        }
+        return tile(l, false, ns ? TS_X : TS_B, in, 2, -1, pre > 1, false);
+    };
+    auto tile_up = [&](int l) {
+        const int nu = tile_ups(post);
+        for (int q = 0; q < nu; ++q) {
+            const bool last = q == nu - 1;
+            const int from = 2 + (q & 1);
+            const int r2 = tile(l, true, q ? TS_X : TS_PROLONG, from, last ? 0 : 5 - from, last ? 1 : -1,
+                                tile_up_two(post, q), l == 0 && last);
+            if (r2) return r2;
+        }
+        return (int)IBMDEM_OK;
     };
     // r.z of the cases whose own level-0 form is tiles, after passes
     auto tile_rz = [&]() {
@@ -2423,7 +2491,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             a.g = bgrid(tile_grid(L.d), dim3(256, TileUp::NT / 256));
             a.L = c->dlev;
             a.b = L.b;
-            a.x = L.x;
+            a.xin = L.x;
             a.partial = c->partial;
             a.stop = c->scal + SC_CONV;
             args.push_back(a);
@@ -2508,7 +2576,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             }
         }
         last_in = cur;
-        if ((rc = tile(l, false))) return rc;
+        if ((rc = tile_down(l))) return rc;
         std::vector<RsArg<T>> rs;
         BOp ors;
         ors.kind = IBMDEM_BK_RESTRICT;
@@ -2554,7 +2622,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
         opr[0].kind = opr[1].kind = IBMDEM_BK_PROLONG;
         if ((rc = add_op(ar, ops, launch_prolong<T, 2>, RB, pr[1], opr[1], err))) return rc;
         if ((rc = add_op(ar, ops, launch_prolong<T, 1>, RB, pr[0], opr[0], err))) return rc;
-        if ((rc = tile(l, true))) return rc;
+        if ((rc = tile_up(l))) return rc;
         int cur = 2;
         for (int q = 0; q < post; ++q) {
             const bool last = q == post - 1;

@@ -1,0 +1,68 @@
+"""Multigrid levels in tiles at edge shapes with every smoothing count, against
+the oracle: one CG iteration from x = 0 exposes one V-cycle."""
+import numpy as np
+import pytest
+
+from ibmdem import cases
+from ibmdem.abi import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, ERR_NOT_CONVERGED, K_MG_SMOOTH, IbmdemError,
+                        Simulation)
+
+pytestmark = pytest.mark.gpu
+P, W, I, O = BC_PERIODIC, BC_WALL, BC_INFLOW, BC_OUTFLOW
+
+# one and two pairs per thread, rows in one tile and in several, partial tiles
+# in every dimension, levels smaller than a halo, every side type
+GRIDS = [
+    ((4, 4, 4), [W] * 6),
+    ((6, 4, 10), [P, P, P, P, W, W]),
+    ((12, 20, 4), [W, W, P, P, P, P]),
+    ((26, 14, 22), [P] * 6),
+    ((62, 4, 8), [W] * 6),
+    ((34, 58, 18), [W, W, W, W, I, O]),
+    ((8, 130, 40), [P, P, W, W, P, P]),
+    ((260, 28, 16), [P] * 6),
+    ((264, 12, 20), [W] * 6),
+    ((130, 44, 12), [I, O, P, P, W, W]),
+    ((386, 8, 6), [P, P, W, W, W, W]),
+    ((520, 30, 8), [I, O, W, W, P, P]),
+    ((24, 40, 152), [W, W, I, O, P, P]),
+]
+
+
+def _iterate(lib, n, bt, **kw):
+    """One CG iteration from x = 0: one V-cycle applied to the right-hand side."""
+    case = cases.build_case(*n, bt, rtol=1e-30, max_iter=1, **kw)
+    rhs = np.random.default_rng(5).normal(size=n[::-1])
+    rhs -= rhs.mean()
+    with Simulation(lib, case) as s:
+        s.upload_poisson_rhs(rhs)
+        with pytest.raises(IbmdemError) as e:
+            s.poisson()
+        assert e.value.code == ERR_NOT_CONVERGED
+        return s.download_poisson()[0]
+
+
+def _close(a, b, tol):
+    assert np.abs(b).max() > 0
+    assert np.abs(a - b).max() < tol * np.abs(b).max()
+
+
+# tolerance as test_gpu_multigrid's: the rounding of two inner products
+@pytest.mark.parametrize("pre,post", [(1, 1), (1, 2), (2, 1), (2, 3), (3, 2), (3, 4), (5, 5), (8, 6)])
+@pytest.mark.parametrize("n,bt", [GRIDS[q] for q in (0, 2, 3, 5, 8, 9, 12)])
+def test_smoothing_counts_in_tiles(gpu_lib, oracle_lib, n, bt, pre, post):
+    kw = dict(mg_pre=pre, mg_post=post)
+    _close(_iterate(gpu_lib, n, bt, **kw), _iterate(oracle_lib, n, bt, **kw), 1e-12)
+
+
+# a visit in tiles is a launch for every two sweeps each way (marching passes
+# would be one for each)
+@pytest.mark.parametrize("pre,post,launches", [(2, 2, 2), (1, 1, 2), (3, 3, 4), (4, 4, 4), (7, 2, 5)])
+def test_launches_of_a_visit_in_tiles(gpu_lib, pre, post, launches):
+    case = cases.build_case(48, 40, 56, [W] * 6, rtol=1e-30, max_iter=3, mg_pre=pre, mg_post=post)
+    with Simulation(gpu_lib, case) as s:
+        s.upload_poisson_rhs(np.random.default_rng(2).normal(size=(56, 40, 48)))
+        s.profile_kernel(K_MG_SMOOTH)
+        with pytest.raises(IbmdemError):
+            s.poisson()
+        assert s.profile_read()[1] == 4 * launches   # z = M^-1 r at the start and in each iteration
