@@ -282,17 +282,17 @@ __device__ __forceinline__ bool tile_owns(const C &c, const LevelDev &L, int ox,
     return c.act && c.p >= 2 && c.p < 2 + TL_X / 2 && c.y >= 4 && c.y < 4 + TL_Y && c.z + m >= 4 &&
            c.z + m < 4 + TL_Z && i < L.nx && j < L.ny && k < L.nz;
 }
-// the block's partial sum: wavefronts by shuffles, then in order
-template <typename G>
+// the block's partial sum: NW wavefronts by shuffles, then in order
+template <int NW>
 __device__ __forceinline__ void tile_partial(const Blk &kb, double dsum, double *__restrict__ partial) {
     const int t = threadIdx.x;
-    __shared__ double red[G::NT / 64];
+    __shared__ double red[NW];
     for (int st = 32; st > 0; st >>= 1) dsum += __shfl_down(dsum, st, 64);
     if ((t & 63) == 0) red[t >> 6] = dsum;
     __syncthreads();
     if (t == 0) {
         double a = 0.0;
-        for (int w = 0; w < G::NT / 64; ++w) a += red[w];
+        for (int w = 0; w < NW; ++w) a += red[w];
         partial[((long)kb.bz * kb.gy + kb.by) * kb.gx + kb.bx] = a;
     }
 }
@@ -397,7 +397,7 @@ __device__ __forceinline__ void tile_up_body(const Blk &kb, const LevelDev &L, c
             dsum += double(c.fb[m]) * double(c.b[m]);
         }
     }
-    if (partial) tile_partial<G>(kb, dsum, partial);
+    if (partial) tile_partial<G::NT / 64>(kb, dsum, partial);
 }
 template <typename T, int SRC>
 __global__ __launch_bounds__(TileUp::NT) void k_tile_up(LevelDev L, const T *__restrict__ bg,
@@ -409,24 +409,42 @@ __global__ __launch_bounds__(TileUp::NT) void k_tile_up(LevelDev L, const T *__r
 }
 
 // tile_up_body's partial sums of b.x from an x that is there already: a batch
-// whose level 0 marches still sums r.z as each case's own launch does.
+// whose level 0 marches still sums r.z as each case's own launch does, so
+// this is bound by memory. It runs the two groups of wavefronts that hold the
+// tile's planes (the outer two's are halo and add 0), the loads ahead of the
+// stop flag: a step of 20 cases of 64^3 takes 5.95 ms, 6.23 ms with all four
+// groups, which left half of the CUs' wavefronts idle.
+constexpr int TRZ_NT = 2 * TileUp::GT;
+static_assert(TileUp::GT % 64 == 0 && TL_Z == 2 * TileUp::M && TileUp::NG == 4, "the tile is the middle two groups");
 template <typename T>
 __device__ __forceinline__ void tile_rz_body(const Blk &kb, const LevelDev &L, const T *__restrict__ bg,
                                              const T *__restrict__ x, double *__restrict__ partial,
                                              const double *__restrict__ stop) {
     using G = TileUp;
-    if (*stop != 0.0) return;
-    const int ox = kb.bx * TL_X - 4, oy = kb.by * TL_Y - 4, oz = kb.bz * TL_Z - 4;
-    TileCells<T, G> c;
-    tile_init(c, L, ox, oy, oz);
+    const double stopped = *stop;   // waited for with the loads
+    const int g = __builtin_amdgcn_readfirstlane((int)threadIdx.x / G::GT), col = threadIdx.x - g * G::GT;
+    const int y = col / G::RL, p = col - y * G::RL;   // tile_init's column
+    const int i = kb.bx * TL_X + 2 * (p - 2), j = kb.by * TL_Y + y - 4, k0 = kb.bz * TL_Z + g * G::M;
+    const bool own = col < G::PL && p >= 2 && p < 2 + TL_X / 2 && y >= 4 && y < 4 + TL_Y && i < L.nx && j < L.ny;
+    const int pl = (L.nx >> 1) * L.ny, pos = own ? k0 * pl + j * (L.nx >> 1) + (i >> 1) : 0;
+    T v[G::M][4];
+#pragma unroll
+    for (int m = 0; m < G::M; ++m) {
+        const int q = own && k0 + m < L.nz ? pos + m * pl : 0;
+        v[m][0] = bg[q];
+        v[m][1] = x[q];
+        v[m][2] = bg[L.half + q];
+        v[m][3] = x[L.half + q];
+    }
+    if (stopped != 0.0) return;
     double dsum = 0.0;
 #pragma unroll
     for (int m = 0; m < G::M; ++m)
-        if (tile_owns<G>(c, L, ox, oy, oz, m)) {
-            dsum += double(bg[c.pos[m]]) * double(x[c.pos[m]]);
-            dsum += double(bg[L.half + c.pos[m]]) * double(x[L.half + c.pos[m]]);
+        if (own && k0 + m < L.nz) {
+            dsum += double(v[m][0]) * double(v[m][1]);
+            dsum += double(v[m][2]) * double(v[m][3]);
         }
-    tile_partial<G>(kb, dsum, partial);
+    tile_partial<TRZ_NT / 64>(kb, dsum, partial);
 }
 
 // The launches of a visit. Before tile_down (q = 0 ..) and from tile_down's

@@ -2106,7 +2106,7 @@ __global__ __launch_bounds__(TileUp::NT) void kb_tile_up(BTable<TlArg<T>> tab) {
     });
 }
 template <typename T>
-__global__ __launch_bounds__(TileUp::NT) void kb_tile_rz(BTable<TlArg<T>> tab) {
+__global__ __launch_bounds__(TRZ_NT) void kb_tile_rz(BTable<TlArg<T>> tab) {
     batch_for(tab, [&](const TlArg<T> &a, const Blk &kb) {
         tile_rz_body<T>(kb, *cst(a.L), glb(a.b), glb(a.xin), glb(a.partial), glb(a.stop));
     });
@@ -2263,7 +2263,7 @@ void launch_down(const BOp &o, hipStream_t s, int) {
 }
 template <typename T>
 void launch_tile_rz(const BOp &o, hipStream_t s, int) {
-    hipLaunchKernelGGL(kb_tile_rz<T>, dim3(o.blocks), dim3(TileUp::NT), 0, s, table<TlArg<T>>(o));
+    hipLaunchKernelGGL(kb_tile_rz<T>, dim3(o.blocks), dim3(TRZ_NT), 0, s, table<TlArg<T>>(o));
 }
 template <typename T, int SRC>
 void launch_up(const BOp &o, hipStream_t s, int) {
@@ -2488,7 +2488,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             if (tiled(c, 0) || !tile_level<T>(c, 0)) continue;
             MGLevel<T> &L = levels<T>(c)[0];
             TlArg<T> a{};
-            a.g = bgrid(tile_grid(L.d), dim3(256, TileUp::NT / 256));
+            a.g = bgrid(tile_grid(L.d), dim3(128, TRZ_NT / 128));
             a.L = c->dlev;
             a.b = L.b;
             a.xin = L.x;
@@ -2497,7 +2497,7 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             args.push_back(a);
             o.bytes += 2.0 * sizeof(T) * (double)c->n;
         }
-        return add_op(ar, ops, launch_tile_rz<T>, TileUp::NT, args, o, err);
+        return add_op(ar, ops, launch_tile_rz<T>, TRZ_NT, args, o, err);
     };
     // the bottoms at level l
     auto bottoms = [&](int l) {

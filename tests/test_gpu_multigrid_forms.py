@@ -1,11 +1,13 @@
-"""Multigrid levels in tiles at edge shapes with every smoothing count, against
-the oracle: one CG iteration from x = 0 exposes one V-cycle."""
+"""Every form of a multigrid level at edge shapes: tiles with all smoothing
+counts against the oracle (one CG iteration from x = 0 exposes one V-cycle), and
+the marching passes of small levels (a batch whose cells add up takes them) bit
+for bit against the tiles of each case's own run."""
 import numpy as np
 import pytest
 
 from ibmdem import cases
-from ibmdem.abi import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, ERR_NOT_CONVERGED, K_MG_SMOOTH, IbmdemError,
-                        Simulation)
+from ibmdem.abi import (BC_INFLOW, BC_OUTFLOW, BC_PERIODIC, BC_WALL, ERR_NOT_CONVERGED, FP64, K_MG_SMOOTH, MIXED,
+                        Batch, IbmdemError, Simulation)
 
 pytestmark = pytest.mark.gpu
 P, W, I, O = BC_PERIODIC, BC_WALL, BC_INFLOW, BC_OUTFLOW
@@ -66,3 +68,40 @@ def test_launches_of_a_visit_in_tiles(gpu_lib, pre, post, launches):
         with pytest.raises(IbmdemError):
             s.poisson()
         assert s.profile_read()[1] == 4 * launches   # z = M^-1 r at the start and in each iteration
+
+
+def _fluid(n, bt, precision, pre, post):
+    inflow = [0.0, 0.0, 0.0]
+    for d in range(3):
+        if bt[2 * d] == I:
+            inflow[d] = 0.05
+    case = cases.build_case(*n, bt, visc=0.05, u_max=0.3, precision=precision, mg_pre=pre, mg_post=post,
+                            inflow=tuple(inflow))
+    mk, bd = cases.place_spheres(case, [])
+    rng = np.random.default_rng(sum(n))
+    f = [0.02 * rng.normal(size=n[::-1]) for _ in range(4)]
+    for d in range(3):
+        if bt[2 * d] == I:
+            f[d] += 0.05
+    return cases.Setup("fluid", case, mk, bd, f)
+
+
+# with the large case's, the cells of levels 0 and 1 are more than tiles take,
+# so every case marches there; in FP64 the small ones' own runs take tiles
+@pytest.mark.parametrize("precision", [FP64, MIXED])
+@pytest.mark.parametrize("pre,post", [(2, 2), (1, 1), (3, 2), (2, 5)])
+def test_small_levels_march_in_a_batch(gpu_lib, precision, pre, post):
+    sets = [_fluid(n, bt, precision, pre, post) for n, bt in [((200, 200, 200), [W] * 6)] + GRIDS]
+    with Batch(gpu_lib, [s.case for s in sets]) as b:
+        for q, s in enumerate(sets):
+            cases.load(b[q], s)
+        infos = b.run(3)
+        assert b.fused_solves() > 0
+        got = [b[q].download_fields() for q in range(len(b))]
+    for s, fields, info in list(zip(sets, got, infos))[1:]:
+        with Simulation(gpu_lib, s.case) as one:
+            cases.load(one, s)
+            assert one.run(3).iterations == info.iterations
+            for x, y in zip(fields, one.download_fields()):
+                assert np.isfinite(x).all()
+                np.testing.assert_array_equal(x, y)
