@@ -82,6 +82,16 @@ struct BTable {
 // z neighbours are then read through one XCD's L2, whatever a plane's block
 // count. A barrier separates a physical block's blocks, as bodies reuse
 // their LDS.
+// (range [lo, hi) of a case of 8 or more blocks on XCD xs: xcd_range)
+__host__ __device__ __forceinline__ void xcd_range(int plane, int gz, int xs, int &lo, int &hi) {
+    if (gz >= 8) {
+        lo = (xs * gz >> 3) * plane;
+        hi = ((xs + 1) * gz >> 3) * plane;
+    } else {
+        lo = (int)((long)xs * plane * gz >> 3);
+        hi = (int)((long)(xs + 1) * plane * gz >> 3);
+    }
+}
 template <class A, class F>
 __device__ __forceinline__ void batch_for(const BTable<A> &tab, F &&f) {
     const int bid = blockIdx.x, lane = threadIdx.x & 63;
@@ -106,13 +116,7 @@ __device__ __forceinline__ void batch_for(const BTable<A> &tab, F &&f) {
     } else if (nb >= 8) {
         const int xs = p & 7, per = g.pb >> 3;
         int lo;
-        if (g.gz >= 8) {
-            lo = (xs * g.gz >> 3) * plane;
-            hi = ((xs + 1) * g.gz >> 3) * plane;
-        } else {
-            lo = (int)((long)xs * nb >> 3);
-            hi = (int)((long)(xs + 1) * nb >> 3);
-        }
+        xcd_range(plane, g.gz, xs, lo, hi);
         lb0 = lo + (p >> 3);
         step = per;
     } else {

@@ -69,13 +69,8 @@ constexpr bool RES_BLACK = std::is_same<T, float>::value;   // the black cells' 
 // a CU's registers; two in FP32), at least MARCH_MIN planes each (a chunk also
 // loads four halo planes).
 constexpr int MARCH_MIN = 4;
-// `share`: the part of the chip the launch has for this level (a launch over a
-// batch of cases: the level's part of its cells). There the cases' work-groups
-// are of uneven length and rounded per case, so in FP64, where one fills a CU,
-// two rounds of them are made (40 uneven cases of 96x80x64 cells on average:
-// 4.9 in place of 5.3 ms a step at level 0; 64 cases in FP32 lose 1 % by it).
 template <typename T>
-__host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw, double share = 1.0) {
+__host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw) {
     MarchShape s;
     const int groups = (d.nx >> 1) / pw;
     s.ntx = groups <= 64 ? 1 : (groups + 63) / 64;
@@ -85,14 +80,49 @@ __host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw, dou
     s.nty = (d.ny + most - 1) / most;
     s.ty = (d.ny + s.nty - 1) / s.nty;
     s.ry = s.ty + 4;
-    const int tiles = s.ntx * s.nty, slots = (int)((sizeof(T) == 8 ? 256 : 512) * share);
-    const int want = sizeof(T) == 8 && share < 1.0 ? (int)(2.0 * 256 * share / tiles + 1.0)
-                                                   : (tiles < slots ? slots / tiles : 1);
+    const int tiles = s.ntx * s.nty, slots = sizeof(T) == 8 ? 256 : 512, want = tiles < slots ? slots / tiles : 1;
     int per = (d.nz + want - 1) / want;
     per = per < MARCH_MIN ? MARCH_MIN : per;
     s.nzc = (d.nz + per - 1) / per;
     s.nzp = (d.nz + s.nzc - 1) / s.nzc;
     return s;
+}
+// The chunk length of a launch over a batch of cases (their levels d, all of
+// pw pairs): the one whose work-groups are through in the fewest steps. A chunk
+// of `per` planes is per + 4 steps, and an XCD, whose 32 CUs hold `wgs`
+// work-groups each, takes the case's chunks in batch_for's ranges. Chunks that
+// gave each case its share of one or two rounds left some XCDs a round behind:
+// a step of 20 cases of 64^3 in FP64 took 5.90 ms with them and takes 5.47, two
+// of 128^3 4.59 and 4.22, 64 uneven settling cases 28.5 and 25.8 (mixed 26.2
+// and 23.8).
+template <typename T>
+int march_planes(const std::vector<LevelDev> &d, int pw, int wgs) {
+    int best = MARCH_MIN, most = MARCH_MIN;
+    long cost = LONG_MAX;
+    std::vector<int> plane;
+    for (const LevelDev &l : d) {
+        const MarchShape s = march_shape<T>(l, pw);
+        plane.push_back(s.ntx * s.nty);
+        most = std::max(most, l.nz);
+    }
+    for (int per = MARCH_MIN; per <= most; ++per) {
+        double n[8] = {};
+        for (size_t q = 0; q < d.size(); ++q) {
+            const int nb = plane[q] * div_up(d[q].nz, per);
+            for (int x = 0; x < 8; ++x) {
+                int lo, hi;
+                xcd_range(nb, 1, x, lo, hi);
+                n[x] += nb >= 8 ? hi - lo : nb / 8.0;
+            }
+        }
+        const long c = (long)std::ceil(*std::max_element(n, n + 8) / (32 * wgs)) * (per + 4);
+        if (c < cost) {
+            cost = c;
+            best = per;
+        }
+        if (c <= per + 4) break;   // one round: longer chunks take longer
+    }
+    return best;
 }
 
 // wavefronts per SIMD the registers are held to: two work-groups per CU for

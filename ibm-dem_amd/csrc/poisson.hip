@@ -30,6 +30,8 @@
 #include "common.hpp"
 #include "batched.hpp"
 
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -2031,10 +2033,13 @@ int poisson_solve(ibmdem_ctx *c, ibmdem_solve_info *info) {
 //
 // A group's cases share the precision, the smoothing counts and the
 // iteration cap; grids, level counts, where the one-work-group tail starts
-// and the coarsest-level sweeps are per case. A launch runs each member's
-// blocks with the body, block decomposition and arguments of the member's
-// own launch, and a member sees its operations in the order its own solve
-// queues them, so its arithmetic is bitwise that of solving it alone. A
+// and the coarsest-level sweeps are per case. A launch runs the body of the
+// members' own launches, and a member sees its operations in the order its own
+// solve queues them. Where a sum's association follows the decomposition (the
+// inner products, the last pass with r.z) that is the member's own; the level
+// passes, whose cells do not depend on it, choose tiles or marching and the
+// chunk length by the whole launch. So a member's arithmetic is bitwise that
+// of solving it alone. A
 // block finds its case in a table of first blocks (each a multiple of 8, so
 // a case's blocks keep the XCD placement of its own launch); a member that
 // has converged returns at once, as it does alone.
@@ -2049,12 +2054,17 @@ struct MaArg {
     T *out, *out2;
     double *partial;
     int nzp;   // planes of a chunk
+    int nty;   // the grid's y holds the rows' tiles chunk after chunk, so that
+               // batch_for deals the blocks evenly (by planes, a chunk more or less an XCD)
     const T *xc;
     const double *stop;
 };
 template <typename T, int PW, int MODE, bool FROMB, bool PRO>
 __global__ __launch_bounds__(MT, (MARCH_WAVES<T, MODE>)) void kb_march(BTable<MaArg<T>> tab) {
-    batch_for(tab, [&](const MaArg<T> &a, const Blk &kb) {
+    batch_for(tab, [&](const MaArg<T> &a, const Blk &kt) {
+        Blk kb = kt;
+        kb.bz = kt.by / a.nty;
+        kb.by = kt.by - kb.bz * a.nty;
         march_body<T, PW, MODE, FROMB, PRO>(kb, *cst(a.L), glb(a.xin), glb(a.b), glb(a.out), glb(a.out2),
                                             glb(a.partial), a.nzp, glb(a.xc), glb(a.stop));
     });
@@ -2357,8 +2367,8 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
     // (own_tile: 1 the cases whose own form is tiles alone, 0 the others alone)
     auto pass = [&](int l, int mode, bool fromb, int in, int to, int to2, int own_tile = -1, bool pro = false) {
         std::vector<MaArg<T>> args[2];
+        std::vector<LevelDev> lev[2];
         BOp o[2];
-        const double total = cells_at(l);
         const double per = mode >= 2        ? 2.5 * sizeof(T)
                            : mode == 0 && fromb ? 1.5 * sizeof(T)
                            : mode == 1 && RES_BLACK<T> ? 2.5 * sizeof(T)
@@ -2369,9 +2379,10 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             MGLevel<T> &L = levels<T>(c)[l];
             T *buf[4] = {L.x, L.x + L.d.half, L.r, L.r + L.d.half};
             const int pw = march_pw(L.d);
-            const MarchShape sh = march_shape<T>(L.d, pw, mode == 2 ? 1.0 : (double)L.n / total);
+            const MarchShape sh = march_shape<T>(L.d, pw);
             MaArg<T> a{};
-            a.g = bgrid(dim3(sh.ntx, sh.nty, sh.nzc), dim3(MT));
+            a.g = bgrid(dim3(sh.ntx, sh.nty * sh.nzc), dim3(MT));
+            a.nty = sh.nty;
             a.L = c->dlev + l;
             a.xin = in >= 0 ? buf[in] : nullptr;
             a.b = L.b;
@@ -2382,7 +2393,19 @@ int plan_precondition_dot(Arena &ar, std::vector<BOp> &ops, const std::vector<ib
             a.xc = pro ? levels<T>(c)[l + 1].x : nullptr;
             a.stop = c->scal + SC_CONV;
             args[pw - 1].push_back(a);
+            lev[pw - 1].push_back(L.d);
             if (l == 0) o[pw - 1].bytes += per * (double)c->n;
+        }
+        // chunks for the launch, except where the r.z sums follow the case's own
+        for (int v = 0; v < (mode == 2 ? 0 : 2); ++v) {
+            if (args[v].empty()) continue;
+            const int planes = march_planes<T>(lev[v], v + 1, sizeof(T) == 4 && mode != 1 ? 2 : 1);
+            for (size_t q = 0; q < args[v].size(); ++q) {
+                MaArg<T> &a = args[v][q];
+                const int nzc = div_up(lev[v][q].nz, planes);
+                a.nzp = div_up(lev[v][q].nz, nzc);
+                a.g = bgrid(dim3(a.g.gx, a.nty * nzc), dim3(MT));
+            }
         }
         const BLaunch fp[2] = {launch_ma<double, 1, 0, false, true>, launch_ma<double, 2, 0, false, true>};
         const BLaunch fn[2][5] = {
