@@ -460,10 +460,14 @@ __device__ __forceinline__ void contact_body(const Blk &kb, int M, GridDev g, co
         // COOP_MAX of them are scanned by half-wavefronts in turn, more by
         // their own threads, 64 side by side.
         constexpr int COOP_MAX = 64;
-        __shared__ int s_n, s_list[T], s_cnt[T];
+        // A marker whose candidates do not fit was scanned in vain: the block's
+        // markers are alike, so the first such one sends the rest to their own
+        // threads (two spheres of 4,000 markers, 9 times the usual density: 236 us
+        // a contact call, 249 us with every marker tried, 226 us with none).
+        __shared__ int s_n, s_over, s_list[T], s_cnt[T];
         __shared__ double s_f[3][T];
         __shared__ uint32_t s_cand[T / 32][CANDC];
-        if (kb.tx == 0) s_n = 0;
+        if (kb.tx == 0) s_n = s_over = 0;
         __syncthreads();
         if (scan) s_list[atomicAdd(&s_n, 1)] = kb.tx;
         __syncthreads();
@@ -471,10 +475,14 @@ __device__ __forceinline__ void contact_body(const Blk &kb, int M, GridDev g, co
         if (n > 0 && n <= COOP_MAX) {
             for (int e = kb.tx >> 5; e < n; e += T / 32) {
                 const int o = s_list[e];
-                double s0, s1, s2;
-                const int k = contact_scan32(kb.bx * T + o, M, g, mx, mv, mmass, mrad, mbody, mcell, bin_start,
-                                             bin_items, cp, s_cand[kb.tx >> 5], s0, s1, s2);
+                double s0 = 0.0, s1 = 0.0, s2 = 0.0;
+                const int over = __hip_atomic_load(&s_over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                const int k = __shfl(over, 0, 32) ? -1
+                                                  : contact_scan32(kb.bx * T + o, M, g, mx, mv, mmass, mrad, mbody,
+                                                                   mcell, bin_start, bin_items, cp,
+                                                                   s_cand[kb.tx >> 5], s0, s1, s2);
                 if ((kb.tx & 31) == 0) {
+                    if (k < 0) __hip_atomic_store(&s_over, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     s_cnt[o] = k;
                     s_f[0][o] = s0;
                     s_f[1][o] = s1;

@@ -52,3 +52,23 @@ def test_bodies_in_reach(gpu_lib, oracle_lib, bodies):
             out.append(s.download_markers().fcol)
     assert bodies < 100 or np.abs(out[1]).max() > 0
     np.testing.assert_array_equal(out[0], out[1])
+
+
+# shells denser than the first form holds in some blocks and not in others, and
+# blocks where some of the scanning markers fit and the rest do not
+@pytest.mark.parametrize("markers", [(2000, 2000), (4000, 201), (60, 6000), (1000, 3000)])
+def test_contact_scan_overflow(gpu_lib, oracle_lib, markers):
+    case = cases.build_case(40, 36, 34, [BC_PERIODIC] * 6, visc=0.05, kn_coeff=1e5, restitution=0.9, u_max=0.3,
+                            max_pairs=4000)
+    cs = [(8.2, 17.8, 17.1), (20.6, 17.7, 17.4)]
+    mk, bd = cases.place_spheres(case, [cases.Sphere(c, 12.0, 2.0, m) for c, m in zip(cs, markers)])
+    mk.v[:] = np.random.default_rng(6).normal(0.0, 0.02, size=mk.v.shape)
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        with Simulation(lib, case) as s:
+            s.upload_bodies(bd)
+            s.upload_markers(mk)
+            s.contact()
+            out.append(s.download_markers().fcol)
+    assert np.abs(out[1]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
