@@ -747,6 +747,7 @@ __device__ __forceinline__ void stage_entry(const SpreadArgs &a, const EntryIn &
         const int q = lane + 64 * r, e = q / 12;
         s_w[e][q - 12 * e] = in.fw[r];
     }
+    wave_sync();   // an image entry's lane overwrites what other lanes wrote of its row
     u.mlo = u.mhi = 0u;
     if (!in.valid) return;
     const uint32_t code = in.en & ((1u << SBITS) - 1);

@@ -39,3 +39,35 @@ def test_spread_forms(gpu_lib, oracle_lib, h, precision, walls):
     for a, b in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
         assert np.abs(b).max() > 0
         assert np.abs(a - b).max() < 1e-14 * np.abs(b).max()
+
+
+# staged chunks that are images throughout, in one, two and three dimensions:
+# their rows are written by all lanes and then overwritten in part by the lane
+# that stages the entry
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("h", [1.0, 0.3])
+@pytest.mark.parametrize("bt", [[BC_PERIODIC] * 6, [BC_WALL] * 6, [BC_PERIODIC] * 2 + [BC_WALL] * 2 + [BC_PERIODIC] * 2])
+def test_spread_of_images(gpu_lib, oracle_lib, bt, h, precision):
+    n = (16, 24, 17)
+    case = cases.build_case(*n, bt, h=h, visc=0.05, dt=0.1, precision=precision)
+    lo, hi = 1.4, [m - 1.4 for m in n]
+    cs = [(x, y, z) for z in (lo, hi[2]) for y in (lo, hi[1]) for x in (lo, hi[0])]   # corners
+    cs += [(lo, 12.0, hi[2]), (8.0, lo, 8.5), (8.0, 12.0, hi[2])]                     # an edge and faces
+    mk, bd = cases.place_spheres(case, [cases.Sphere(tuple(h * x for x in c), 2.4 * h, 1.5, 40 + 9 * q)
+                                        for q, c in enumerate(cs)], h)
+    rng = np.random.default_rng(8)
+    mk.v[:] = rng.normal(size=mk.v.shape)
+    u = [rng.normal(size=n[::-1]) for _ in range(3)]
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        with Simulation(lib, case) as s:
+            s.upload_bodies(bd)
+            s.upload_markers(mk)
+            s.upload_fields(*u, None)
+            s.begin_step()
+            s.interpolate()
+            s.spread()
+            out.append((s.download_force(), s.download_fields()[:3]))
+    for a, b in zip(out[0][0] + out[0][1], out[1][0] + out[1][1]):
+        assert np.abs(b).max() > 0
+        assert np.abs(a - b).max() < 1e-13 * np.abs(b).max()
