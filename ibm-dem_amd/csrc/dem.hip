@@ -353,14 +353,18 @@ __device__ __forceinline__ int contact_scan32(int i, int M, const GridDev &g, co
     f0 = f1 = f2 = 0.0;
     if (most > ROWC || total > CANDC) return -1;
     off -= n;
+    // (the lanes are one half of a wavefront: their LDS operations complete
+    // in program order)
+    auto lanes_sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    lanes_sync();   // the last marker's candidates have been read
 #pragma unroll
     for (int s = 0; s < ROWC; ++s)
         if (s < n) cand[off + s] = (uint32_t)c[s];
-    // (the lanes are one half of a wavefront: their LDS operations complete
-    // in program order)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    lanes_sync();
     for (int e0 = 0; e0 < total; e0 += 32) {
         double g1 = 0.0, g2 = 0.0, g3 = 0.0;
         if (e0 + l < total) {

@@ -72,3 +72,24 @@ def test_contact_scan_overflow(gpu_lib, oracle_lib, markers):
             out.append(s.download_markers().fcol)
     assert np.abs(out[1]).max() > 0
     np.testing.assert_array_equal(out[0], out[1])
+
+
+# several scanning markers one after the other on the same lanes, each with
+# another number of candidates than the one before it (none among them)
+@pytest.mark.parametrize("seed", [1, 2])
+def test_contact_scan_turns(gpu_lib, oracle_lib, seed):
+    case = cases.build_case(30, 28, 26, [BC_PERIODIC] * 6, visc=0.05, kn_coeff=1e5, restitution=0.9, u_max=0.3,
+                            max_pairs=500)
+    rng = np.random.default_rng(seed)
+    cs = [tuple(c) for c in rng.uniform(0.0, 26.0, (40, 3))]
+    mk, bd = cases.place_spheres(case, [cases.Sphere(c, 5.0, 2.0, 30 + q) for q, c in enumerate(cs)])
+    mk.v[:] = rng.normal(0.0, 0.02, size=mk.v.shape)
+    out = []
+    for lib in (gpu_lib, oracle_lib):
+        with Simulation(lib, case) as s:
+            s.upload_bodies(bd)
+            s.upload_markers(mk)
+            s.contact()
+            out.append(s.download_markers().fcol)
+    assert np.abs(out[1]).max() > 0
+    np.testing.assert_array_equal(out[0], out[1])
