@@ -1,7 +1,7 @@
 """Every form of a multigrid level at edge shapes: tiles with all smoothing
-counts against the oracle (one CG iteration from x = 0 exposes one V-cycle), and
-the marching passes of small levels (a batch whose cells add up takes them) bit
-for bit against the tiles of each case's own run."""
+counts and the mixed form's FP32 levels against the oracle (one CG iteration from
+x = 0 exposes one V-cycle), and the marching passes of small levels (a batch whose
+cells add up takes them) bit for bit against the tiles of each case's own run."""
 import numpy as np
 import pytest
 
@@ -68,6 +68,23 @@ def test_launches_of_a_visit_in_tiles(gpu_lib, pre, post, launches):
         with pytest.raises(IbmdemError):
             s.poisson()
         assert s.profile_read()[1] == 4 * launches   # z = M^-1 r at the start and in each iteration
+
+
+# FP32 levels: a V-cycle commits about 8 roundings of 6e-8 in each of the 95
+# half sweeps of its coarsest level and in fewer above it, 5e-5 of the scale
+@pytest.mark.parametrize("pre,post", [(2, 2), (1, 1), (3, 2)])
+@pytest.mark.parametrize("n,bt", GRIDS + [
+    ((2, 2, 3), [W] * 6),             # the coarsest level alone, in all its forms
+    ((11, 13, 14), [W, W, W, W, I, O]),
+    ((3, 5, 7), [P] * 6),
+    ((16, 16, 33), [P, P, P, P, W, W]),
+    ((34, 27, 45), [W] * 6),
+    ((49, 37, 21), [I, O, W, W, W, W]),
+    ((25, 33, 19), [P, P, W, W, P, P]),
+])
+def test_mixed_levels(gpu_lib, oracle_lib, n, bt, pre, post):
+    kw = dict(mg_pre=pre, mg_post=post)
+    _close(_iterate(gpu_lib, n, bt, precision=MIXED, **kw), _iterate(oracle_lib, n, bt, **kw), 5e-5)
 
 
 def _fluid(n, bt, precision, pre, post):
