@@ -281,7 +281,7 @@ __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, con
     // beyond a side the parent's (parents()). In an even plane the red cell of
     // a pair lies to side A (east where j is odd), in an odd one to side B.
     struct Coarse {
-        int nx, ny, nz, rl, half;
+        int nx, ny, nz, rl, half;   // (two pairs per thread: a split coarse row, one: an odd one)
         int ic[PW + 2], J[2];
         T raw[2][PW + 2], a[PW], ap[PW], b[PW];   // interpolated: side A of planes K, K - 1, side B of K
     } cg;
@@ -289,9 +289,8 @@ __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, con
         cg.nx = L.nx >> 1;
         cg.ny = L.ny >> 1;
         cg.nz = L.nz >> 1;
-        const bool split = (cg.nx & 1) == 0;
-        cg.rl = split ? cg.nx >> 1 : cg.nx;
-        cg.half = split ? cg.rl * cg.ny * cg.nz : 0;
+        cg.rl = PW == 2 ? cg.nx >> 1 : cg.nx;
+        cg.half = PW == 2 ? cg.rl * cg.ny * cg.nz : 0;
         for (int c = 0; c < PW + 2; ++c) {
             const int i = p + c - 1;
             cg.ic[c] = i < 0 ? (px ? i + cg.nx : 0) : (i < cg.nx ? i : (px ? i - cg.nx : cg.nx - 1));
@@ -316,10 +315,7 @@ __device__ __forceinline__ void march_body(const Blk &kb, const LevelDev &L, con
                 raw[q][PW + 1] = cg.ic[PW + 1] == p + 1 ? raw[q][2] : e;
             } else {
 #pragma unroll
-                for (int c = 0; c < PW + 2; ++c) {
-                    const int i = cg.ic[c];
-                    raw[q][c] = xc[o + (cg.half ? (((i + cg.J[q] + K) & 1) ? cg.half : 0) + (i >> 1) : i)];
-                }
+                for (int c = 0; c < PW + 2; ++c) raw[q][c] = xc[o + cg.ic[c]];
             }
         }
     };

@@ -45,7 +45,9 @@ using TileUp = TileGeoC<4, 4, 4>;     // two sweeps
 enum TileSrc { TS_B, TS_X, TS_PROLONG };
 
 // level index of an unwrapped one: wrapped across a periodic side (however
-// often the halo goes round a small level), -1 beyond another
+// often the halo goes round a small level), -1 beyond another. (ct_map's
+// values; its step ahead of the remainder costs these kernels 2 % of a CG
+// iteration at 96^3.)
 __device__ __forceinline__ int tl_map(int v, int n, int lo) {
     if (v >= 0 && v < n) return v;
     if (lo != IBMDEM_BC_PERIODIC) return -1;

@@ -145,49 +145,11 @@ __device__ __forceinline__ PairGeo pair_geo(const LevelDev &L, int p, int j, int
     g.cyz = diag_count(j, L.ny, L.bt[2], L.bt[3]) * 4 + diag_count(k, L.nz, L.bt[4], L.bt[5]);
     return g;
 }
-// nbsum of the pair's even (h = 0) or odd (h = 1) cell; q(d) is the value
-// at offset d from the pair's position in the other cell's colour half
-template <typename T, typename F>
-__device__ __forceinline__ T nbsum_pair_f(const F &q, const PairGeo &g, int h, const LevelDev &L) {
-    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
-    T xw, xe;
-    if (h == 0) {
-        xw = g.hw ? q(g.dw) : T(0);
-        xe = q(0);
-    } else {
-        xw = q(0);
-        xe = g.he ? q(g.de) : T(0);
-    }
-    const T xs = g.hs ? q(g.ds) : T(0), xn = g.hn ? q(g.dn) : T(0);
-    const T xb = g.hb ? q(g.db) : T(0), xt = g.ht ? q(g.dt) : T(0);
-    const T sx = (xw + xe) * ihx2;
-    const T syy = (xs + xn) * ihy2;
-    const T szz = (xb + xt) * ihz2;
-    return sx + syy + szz;
-}
-// nbsum_pair_f's value from an array. Every neighbour is loaded without a
-// branch (an absent one from offset 0, the pair's own position, and then
-// replaced by 0), so a thread's loads can all be in flight at once.
-template <typename T>
-__device__ __forceinline__ T nbsum_pair(const T *__restrict__ oth, const PairGeo &g, int h, const LevelDev &L) {
-    const T *q = oth + g.pos;
-    const T ihx2 = T(L.ihx2), ihy2 = T(L.ihy2), ihz2 = T(L.ihz2);
-    const bool pw = h == 0 ? g.hw : true, pe = h == 0 ? true : g.he;
-    const T vw = q[h == 0 && g.hw ? g.dw : 0], ve = q[h != 0 && g.he ? g.de : 0];
-    const T vs = q[g.hs ? g.ds : 0], vn = q[g.hn ? g.dn : 0];
-    const T vb = q[g.hb ? g.db : 0], vt = q[g.ht ? g.dt : 0];
-    const T xw = pw ? vw : T(0), xe = pe ? ve : T(0);
-    const T xs = g.hs ? vs : T(0), xn = g.hn ? vn : T(0);
-    const T xb = g.hb ? vb : T(0), xt = g.ht ? vt : T(0);
-    const T sx = (xw + xe) * ihx2;
-    const T syy = (xs + xn) * ihy2;
-    const T szz = (xb + xt) * ihz2;
-    return sx + syy + szz;
-}
-
-// nbsum_pair from the loaded values: the pair value, the other x neighbour
-// (west for h = 0, east for h = 1), south, north, below, above (each read
-// at offset 0 when absent, and replaced by 0 here)
+// nbsum of the pair's even (h = 0) or odd (h = 1) cell from the loaded values:
+// the pair's other one, the other x neighbour (west for h = 0, east for h = 1),
+// south, north, below, above (each read at offset 0, the pair's own position,
+// when absent, and replaced by 0 here: loads without a branch are all in flight
+// at once)
 template <typename T>
 __device__ __forceinline__ T nbsum_pair_vals(const PairGeo &g, int h, T part, T xo, T ys, T yn, T zb, T zt,
                                              const LevelDev &L) {
@@ -778,7 +740,7 @@ struct TailPairs {
     }
     // the black cells stand behind the red ones and their zero word
     __device__ __forceinline__ int base(int c) const { return c ? L.half + 1 : 0; }
-    // nbsum_pair's value for the cell of colour c of pair u
+    // nbsum of the cell of colour c of pair u
     __device__ __forceinline__ T nbsum(const T *x, int u, int c) const {
         const T *oth = x + base(1 - c);
         const T sx = (oth[threadIdx.x + u * NT] + oth[ox[u][c]]) * ihx2;
