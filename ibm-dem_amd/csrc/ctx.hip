@@ -88,7 +88,7 @@ int alloc_all(ibmdem_ctx *c) {
         for (int d = 0; d < 3; ++d)
             if (c->g.bt[2 * d + 1] == IBMDEM_BC_OUTFLOW) A(c->g.plane[d], pn[d]);
     }
-    A(c->cg_x, n); A(c->cg_r, n); A(c->cg_z, n); A(c->cg_p, n); A(c->cg_Ap, n);
+    A(c->cg_x, n); A(c->cg_r, n); A(c->cg_p, n); A(c->cg_Ap, n);
     // bulk-forcing partials: one per 64 x 4 row group and plane; the
     // matrix-vector product's: one per block
     const long pred_blocks = (long)div_up(c->g.nx, 64) * div_up(c->g.ny, 4) * c->g.nz;

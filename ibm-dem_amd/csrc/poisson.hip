@@ -1803,6 +1803,10 @@ int poisson_setup(ibmdem_ctx *c) {
         nx /= 2; ny /= 2; nz /= 2;
         h[0] *= 2; h[1] *= 2; h[2] *= 2;
     }
+    int rc;
+    // the mixed form reads z where its V-cycle leaves it, in FP32, but for a
+    // hierarchy of one level (precondition)
+    if ((c->cs.precision != IBMDEM_MIXED || c->nlev < 2) && (rc = dev_alloc(c, &c->cg_z, c->n))) return rc;
     // the small levels whose x, b and r fit the tail work-group's LDS
     // together run as one launch per V-cycle, when the coarsest level suits
     // the one-wavefront table sweeps (IBMDEM_NO_TAIL=1 keeps one launch per
@@ -1821,7 +1825,6 @@ int poisson_setup(ibmdem_ctx *c) {
     }
     const char *nt = std::getenv("IBMDEM_NO_TAIL");
     if (nt && *nt && *nt != '0') c->tail_first = c->nlev;
-    int rc;
     if ((rc = dev_alloc(c, &c->dlev, (size_t)c->nlev))) return rc;
     LevelDev host[IBMDEM_MAX_LEVELS];
     for (int l = 0; l < c->nlev; ++l) host[l] = c->lev64[l].d;

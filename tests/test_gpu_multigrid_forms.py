@@ -122,3 +122,17 @@ def test_small_levels_march_in_a_batch(gpu_lib, precision, pre, post):
             for x, y in zip(fields, one.download_fields()):
                 assert np.isfinite(x).all()
                 np.testing.assert_array_equal(x, y)
+
+
+# the mixed form keeps its level arrays in FP32 and no FP64 z beside them, except
+# where there is one level: 8 n more there
+def test_mixed_memory(gpu_lib):
+    def memory(n, precision):
+        with Simulation(gpu_lib, cases.build_case(*n, [W] * 6, precision=precision)) as s:
+            return s.memory_bytes()
+    n = (64, 64, 64)   # levels add up to less than 8/7 of level 0
+    cells = 64 ** 3
+    # FP64: z, r of every level, x and b of the coarser ones; mixed: x, b, r in FP32
+    assert memory(n, FP64) - memory(n, MIXED) > cells * (8 + 8 * 1.14 + 16 * 0.14 - 12 * 1.15)
+    one = (33, 35, 37)
+    assert memory(one, MIXED) - memory(one, FP64) == 4 * 33 * 35 * 37   # 12 n + 8 n against 8 n + 8 n
