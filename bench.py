@@ -115,7 +115,7 @@ def timed_run(setup, precision, steps, warmup, profile):
 KERNEL_NAMES = {
     "spread": "k_spread_tiles (IBM spread + multi-direct-forcing update)",
     "mg_smooth": "k_march, all level-0 passes (two fused red-black Gauss-Seidel half sweeps each: first, "
-                 "residual, with the prolongation, r.z)",
+                 "residual, with the prolongation, r.z; the mixed form's last two half sweeps are k_rz_half)",
     "interp": "k_interp (IBM interpolation)",
     "predictor": "k_predictor_lds (fused advection-diffusion predictor, LDS z-marching)",
 }

@@ -1639,6 +1639,7 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
     const T *uncorrected = cur;
     cur = r0;
     bytes = 0.0;
+    int launches = c->cs.mg_post;
     if (l == 0) prof_begin(c, IBMDEM_K_MG_SMOOTH);
     for (int q = 0; q < c->cs.mg_post; ++q) {
         if (q < c->cs.mg_post - 1) {
@@ -1659,6 +1660,7 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
                 bytes += 2.5 * cell;
             } else {
                 launch_rz(s, d, cur, x0, x1, c->cg_r, c->partial, stop);
+                ++launches;   // its two sweeps are a launch each
                 bytes += 2.0 * cell + 8.0 * (double)L.n;
             }
         } else {
@@ -1667,7 +1669,7 @@ int vcycle(ibmdem_ctx *c, MGLevel<T> *lev, int l, bool dot = false) {
         }
         CHECK_LAUNCH(c);
     }
-    if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, bytes, c->cs.mg_post);
+    if (l == 0) prof_end(c, IBMDEM_K_MG_SMOOTH, bytes, launches);
     return IBMDEM_OK;
 }
 

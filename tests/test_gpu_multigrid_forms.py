@@ -57,17 +57,28 @@ def test_smoothing_counts_in_tiles(gpu_lib, oracle_lib, n, bt, pre, post):
     _close(_iterate(gpu_lib, n, bt, **kw), _iterate(oracle_lib, n, bt, **kw), 1e-12)
 
 
-# a visit in tiles is a launch for every two sweeps each way (marching passes
-# would be one for each)
-@pytest.mark.parametrize("pre,post,launches", [(2, 2, 2), (1, 1, 2), (3, 3, 4), (4, 4, 4), (7, 2, 5)])
-def test_launches_of_a_visit_in_tiles(gpu_lib, pre, post, launches):
-    case = cases.build_case(48, 40, 56, [W] * 6, rtol=1e-30, max_iter=3, mg_pre=pre, mg_post=post)
-    with Simulation(gpu_lib, case) as s:
+def _visit_launches(lib, pre, post, precision):
+    """Smoothing launches of one visit of level 0."""
+    case = cases.build_case(48, 40, 56, [W] * 6, rtol=1e-30, max_iter=3, mg_pre=pre, mg_post=post, precision=precision)
+    with Simulation(lib, case) as s:
         s.upload_poisson_rhs(np.random.default_rng(2).normal(size=(56, 40, 48)))
         s.profile_kernel(K_MG_SMOOTH)
         with pytest.raises(IbmdemError):
             s.poisson()
-        assert s.profile_read()[1] == 4 * launches   # z = M^-1 r at the start and in each iteration
+        return s.profile_read()[1] / 4   # z = M^-1 r at the start and in each iteration
+
+
+# in tiles a launch for every two sweeps each way (marching passes would be one
+# for each)
+@pytest.mark.parametrize("pre,post,launches", [(2, 2, 2), (1, 1, 2), (3, 3, 4), (4, 4, 4), (7, 2, 5)])
+def test_launches_of_a_visit_in_tiles(gpu_lib, pre, post, launches):
+    assert _visit_launches(gpu_lib, pre, post, FP64) == launches
+
+
+# the mixed form marches: a pass a sweep, but the last black and red ones apart
+@pytest.mark.parametrize("pre,post,launches", [(2, 2, 5), (1, 1, 3), (3, 4, 8)])
+def test_launches_of_a_mixed_visit(gpu_lib, pre, post, launches):
+    assert _visit_launches(gpu_lib, pre, post, MIXED) == launches
 
 
 # FP32 levels: a V-cycle commits about 8 roundings of 6e-8 in each of the 95
