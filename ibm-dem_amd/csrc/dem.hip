@@ -481,10 +481,10 @@ __device__ __forceinline__ void contact_body(const Blk &kb, int M, GridDev g, co
                 const int o = s_list[e];
                 double s0 = 0.0, s1 = 0.0, s2 = 0.0;
                 const int over = __hip_atomic_load(&s_over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                const int k = __shfl(over, 0, 32) ? -1
-                                                  : contact_scan32(kb.bx * T + o, M, g, mx, mv, mmass, mrad, mbody,
-                                                                   mcell, bin_start, bin_items, cp,
-                                                                   s_cand[kb.tx >> 5], s0, s1, s2);
+                const int k = __ballot(over) ? -1
+                                             : contact_scan32(kb.bx * T + o, M, g, mx, mv, mmass, mrad, mbody, mcell,
+                                                              bin_start, bin_items, cp, s_cand[kb.tx >> 5], s0, s1,
+                                                              s2);
                 if ((kb.tx & 31) == 0) {
                     if (k < 0) __hip_atomic_store(&s_over, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     s_cnt[o] = k;
