@@ -203,8 +203,10 @@ __global__ __launch_bounds__(T) void k_body_rmax(int M, int B, GridDev g, const 
 // reach is missed.
 constexpr int NEAR_MAX = 32;
 // Short chunks fill the chip from a few hundred bodies on, long ones have less
-// to start and to store per test when there are tens of thousands of blocks:
-// 10,000 bodies take 100 us in chunks of 64 and 107 us in chunks of 16.
+// to start and to store per test when there are tens of thousands of blocks. A
+// contact call of bodies far apart, us, in chunks of 16 and of 64: 700 bodies
+// 20.5 and 24.6, 2,500 27.2 and 28.8, 4,000 36.8 and 36.2, 10,000 119 and 110,
+// 20,000 414 and 376 (chunks of 32 lie between the two everywhere).
 __host__ __device__ __forceinline__ int near_chunk(int B) { return B > 4096 ? 64 : 16; }
 __device__ __forceinline__ void body_near_clear_body(const Blk &kb, int B, int *__restrict__ near) {
     const int b = kb.bx * 64 + kb.tx;
@@ -287,7 +289,10 @@ __device__ __forceinline__ void pair_force(const ContactSelf &a, const ContactPa
 // where few markers scan (1,206 markers) and 103 us over 700 packed spheres
 // (220,000 markers); with it in one chain 10 and 23 us. Returns the
 // number of candidates, or -1 where they do not fit (more than ROWC in a row
-// or CANDC in all: the owner then scans alone).
+// or CANDC in all: the owner then scans alone). Usual shells need one or two a
+// row: 700 packed spheres take the same with room for 2, 4 or 8 and for 32 or
+// 64 in all; where shells press into each other (pitch 12.3 at D = 12) 194, 183
+// and 181 us with room for 2, 4 and 8 a row.
 constexpr int ROWC = 4, CANDC = 64;
 __device__ __forceinline__ int contact_scan32(int i, int M, const GridDev &g, const double *__restrict__ mx,
                                               const double *__restrict__ mv, const double *__restrict__ mmass,
@@ -462,7 +467,11 @@ __device__ __forceinline__ void contact_body(const Blk &kb, int M, GridDev g, co
     if constexpr (!PAIRS) {
         // The block's scanning markers are few (contact is local): up to
         // COOP_MAX of them are scanned by half-wavefronts in turn, more by
-        // their own threads, 64 side by side.
+        // their own threads, 64 side by side. A contact call, us, with own
+        // threads alone and with COOP_MAX 16, 64 and 256: 700 packed spheres of
+        // D = 8 113, 115, 45, 45; pressed together 185, 186, 183, 129; but
+        // shells within one another 220, 225, 223, 432, and with 4,000 markers
+        // a sphere 829, 842, 835, 1055.
         constexpr int COOP_MAX = 64;
         // A marker whose candidates do not fit was scanned in vain: the block's
         // markers are alike, so the first such one sends the rest to their own

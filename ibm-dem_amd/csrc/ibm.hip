@@ -759,7 +759,8 @@ __device__ __forceinline__ void stage_entry(const SpreadArgs &a, const EntryIn &
     // with a power-of-two cell volume an exact scaling (bitwise the same
     // products as fv * (w * (1/dV))), else the same two roundings in another
     // order, taken in FP64 contexts (the mixed form amplifies a last-bit
-    // change through its FP32 predictor and keeps the division of each weight)
+    // change through its FP32 predictor and keeps the division of each weight:
+    // 181 us a launch over 700 packed spheres, 124 us folded)
     if (DV == DV_POW2) {
         u.f0 = in.f0 * a.idV; u.f1 = in.f1 * a.idV; u.f2 = in.f2 * a.idV;
     } else if (DV == DV_FOLD) {
@@ -887,8 +888,8 @@ __device__ __forceinline__ void spread_tiles_body(const Blk &kb, const SpreadArg
     __shared__ double s_acc[3][ACC_N];         // the tile's force
     __shared__ unsigned s_touch[TC / 32];      // cells some entry reached
     // per staged entry: (face, centre) factor pairs for 3 dimensions x 4
-    // offsets (padded to an odd number of 16-byte pairs per entry); its
-    // support corner and fdrag*vol stay in the staging lane's registers
+    // offsets (padded to an odd number of 16-byte pairs per entry); the rest
+    // of it (EntryUni) stays in the staging lane's registers
     __shared__ double2 s_w[CAP][WST2];
     const GridDev &g = a.g;
     const int lane = kb.tx;

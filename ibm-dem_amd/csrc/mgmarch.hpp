@@ -67,7 +67,9 @@ constexpr bool RES_BLACK = std::is_same<T, float>::value;   // the black cells' 
 // each side; as many rows as the work-group holds, evenly spread; chunks so
 // that the launch has about one work-group per CU (in FP64 a work-group fills
 // a CU's registers; two in FP32), at least MARCH_MIN planes each (a chunk also
-// loads four halo planes).
+// loads four halo planes). A CG iteration with 2, 4 and 8 planes at least, us:
+// 64^3 mixed 143, 148, 161; 128^3 222, 225, 247, mixed 234, 214, 228; 256^3 740,
+// 739, 770, mixed 758, 734, 759.
 constexpr int MARCH_MIN = 4;
 template <typename T>
 __host__ __device__ inline MarchShape march_shape(const LevelDev &d, int pw) {
