@@ -1011,7 +1011,7 @@ __device__ __forceinline__ void matvec_dot_body(const Blk &kb, const LevelDev &L
     if (scal[SC_CONV] != 0.0) return;
     __shared__ double red[RB];
     // a thread takes the x-pair ip of two adjacent rows j0, j0 + 1 (blocks as
-    // the half sweep); when both rows exist, a cell's north neighbour in row
+    // sweep_shape's); when both rows exist, a cell's north neighbour in row
     // j0 is row j0 + 1's value of the same cell of its pair, and a cell's
     // south neighbour in row j0 + 1 is row j0's: those loads are shared
     const int ip = kb.bx * kb.dx + kb.tx;
@@ -1710,8 +1710,8 @@ int precondition(ibmdem_ctx *c) {
 }
 
 // z = M^{-1} r, then r.z into scal[slot] with k_final's op. In the FP64 form
-// with post-smoothing the level-0 sweeps that finalize z also leave the
-// partial sums of r.z (one per block and colour), so z is not read again.
+// with post-smoothing the last level-0 launches leave the partial sums of r.z
+// (rz_blocks), so z is not read again.
 int precondition_dot(ibmdem_ctx *c, int slot, int op) {
     if (c->cs.mg_post < 1 || c->nlev < 2) {
         int rc = precondition(c);
